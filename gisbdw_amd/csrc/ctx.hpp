@@ -38,27 +38,24 @@ struct Error {
   } while (0)
 
 // Per-graph DP descriptor, one per graph, read by the kernels with scalar
-// loads.  Vertices 0..lb-1 are the "low" vertices resolved inside a tile;
-// vertices lb..n-1 are the "high" vertices whose subset H selects the tile.
+// loads.  Vertices 0..4 are the bits of a word of 32 subsets, vertices
+// 5..lb-1 pick a word of a tile, and vertices lb..n-1 are the "high" vertices
+// whose subset H selects the tile.
 struct DPGraph {
   uint32_t n;        // vertices
   uint32_t nh;       // high vertices, max(n - lb, 0)
-  uint32_t lb;       // low bits per tile
-  uint32_t cb;       // class bits of the level layout (0, 3 or 4; see TileIndex)
-  uint32_t pk;       // packed tiles (class layout only): 4 bits per subset
-                     // plus one base byte per tile, see DPTile
+  uint32_t lb;       // 5 + log2(words per tile): 5, 6 or 7
   uint32_t pad0;
   uint64_t table;    // byte offset of this graph's tables in the arena
   uint32_t lvl[34];  // tile offset of high level h; lvl[nh+1] = 2^nh
   uint32_t adj[32];  // adjacency rows
-  uint32_t nl[32];   // N(L) for every L subset of the low vertices
   // The next three arrays are consecutive (the level kernels copy them to
-  // LDS as one block).  Masks over the low parts L of a tile use the
-  // tile-mask bit order: bit 8 (L & 3) + (L >> 2) stands for L.
-  uint32_t nbh[512];  // N(H) by 7-bit chunks of H: nbh[128 c + chunk]
-  uint32_t isoh[512]; // by 7-bit chunks of high vertices X: the L that give
-                      // every x in X a neighbour
-  uint32_t isol[32];  // by set Y of low vertices: the L in which every
+  // LDS as one block).  Vertices above 4 come in 7-bit chunks, chunk c from
+  // vertex 5 + 7 c on.
+  uint32_t nbh[512];  // neighbours of a set of them: nbh[128 c + chunk]
+  uint32_t isoh[512]; // by a set X of them: the L that give every x in X a
+                      // neighbour
+  uint32_t isol[32];  // by set Y of vertices 0..4: the L in which every
                       // y in Y n L has a neighbour in L
 };
 constexpr int kTabNbh = 0, kTabIsoH = 512, kTabIsoL = 1024, kTabWords = 1056;
@@ -67,50 +64,19 @@ static_assert(offsetof(DPGraph, isoh) == offsetof(DPGraph, nbh) + 4 * kTabIsoH,
 static_assert(offsetof(DPGraph, isol) == offsetof(DPGraph, nbh) + 4 * kTabIsoL,
               "isoh and isol must be consecutive");
 
-// Class-major level layout.  High level h (|H| = h) starts at tile lvl[h].
-// With cb class bits its tiles are grouped by class p = H & (2^cb - 1), in
-// increasing p, and class p holds the C(nh - cb, h - |p|) sets Hr = H >> cb
-// in colex order.  Removing a vertex of Hr stays in class p; removing a
-// class vertex b keeps Hr and its rank and moves to class p \ b.  cb = 0 is
-// plain colex order of H.  C(x, j) is the binomial coefficient functor.
-template <typename BinomFn>
-__host__ __device__ inline uint32_t ClassBase(int h, uint32_t p, int rest, BinomFn C) {
-  uint32_t base = 0;
-  for (uint32_t q = 0; q < p; ++q) {
-    const int k = h - __builtin_popcount(q);
-    if (k >= 0 && k <= rest) base += static_cast<uint32_t>(C(rest, k));
-  }
-  return base;
-}
-
-// Tile offset of high part H inside its level.
-template <typename BinomFn>
-__host__ __device__ inline uint32_t TileIndex(uint32_t H, int nh, int cb, BinomFn C) {
-  const uint32_t p = H & ((1u << cb) - 1u);
-  uint32_t Hr = H >> cb;
-  uint32_t r = ClassBase(__builtin_popcount(H), p, nh - cb, C);
-  int i = 0;
-  while (Hr) {
-    const int x = __builtin_ctz(Hr);
-    Hr &= Hr - 1;
-    r += static_cast<uint32_t>(C(x, ++i));
-  }
-  return r;
-}
-
 // DP launch configuration (autotuned).
 struct DPConfig {
-  int low_bits = 4;        // 2..5 (autotuned on MI355X at n = 30)
+  int low_bits = 4;        // 2..5: tiles of 1, 1, 2 or 4 words
   int tiles_per_lane = 1;  // consecutive tiles per lane (Gosper steps)
   int block = 512;         // threads per workgroup
   int batch_wg_per_cu = 4; // persistent batch kernel: workgroups per CU
   int batch_block = 1024;  // persistent batch kernel: threads per workgroup
   int use_graph = 1;       // capture the level sequence into a hipGraph
-  int xcd_remap = 0;       // contiguous tile slice per XCD (measured slower)
-  int class_bits = 0;      // single-graph level layout: 0 (plain colex), 3 or 4
-  int class_min_nh = 16;   // class layout only from this many high vertices
+  int xcd_remap = 0;       // accepted, without effect (slices are always on)
+  int class_bits = 0;      // accepted; with packed, only the bytes claimed
+  int class_min_nh = 16;
   int grid_mult = 4;       // level launch: at most grid_mult x the resident workgroups
-  int packed = 0;          // class layouts with low_bits >= 4 store packed tiles
+  int packed = 0;          // with class_bits and low_bits >= 4: claim 17/32 bytes a subset
   int streams = 2;         // batch calls: large graphs' level sequences in flight (1-3)
 };
 

@@ -7,17 +7,19 @@
 // For a disconnected S the second line equals max_{v in S} td(S \ v), so every
 // subset of size k needs only subsets of size k-1.  Connectivity is carried in
 // the table too: S (|S| >= 2) is connected iff no vertex of S is isolated in S
-// and some S \ v is connected.  Each stored byte is 2*td + connected.
+// and some S \ v is connected.
 //
-// Layout.  Vertices 0..lb-1 are "low", lb..n-1 "high".  A subset S = H u L is
-// stored in the tile of its high part H (2^lb bytes, byte L).  The tiles of
+// Layout.  A subset takes three bits, in words of 32 subsets (dpword.hpp):
+// the Gray code of td mod 4 and "connected".  Vertices 0..4 are a word's,
+// vertices 5..lb-1 pick one of the 2^(lb-5) words of a tile (1, 2 or 4), and
+// vertices lb..n-1 are "high": their subset H picks the tile.  The tiles of
 // high level h = |H| are ranked by the colex rank of H among the h-subsets of
 // the nh = n - lb high vertices (rank(H) = sum_i C(x_i, i+1),
-// set_encoder.hpp:40-46), and the levels are concatenated.  The tile of H is
-// computed from the h tiles of H \ x (x in H, all at high level h-1, each a
-// contiguous 2^lb-byte block read once) and, inside the tile, from smaller L
-// of the same tile (registers).  One lane owns a tile; a lane walks
-// consecutive ranks with Gosper's successor (colex order = numeric order).
+// set_encoder.hpp:40-46), and the levels are concatenated, once for each of
+// the three bit planes.  The tile of H is computed from the h tiles of H \ x
+// (x in H, all at high level h-1) and, inside the tile, from smaller words.
+// One lane owns a tile; a lane walks consecutive ranks with Gosper's
+// successor (colex order = numeric order).
 #include <algorithm>
 #include <atomic>
 #include <chrono>
@@ -30,11 +32,10 @@
 #include <vector>
 
 #include "ctx.hpp"
+#include "dpword.hpp"
 
 namespace tdhip {
 namespace {
-
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kCbStride = 33;  // s_cb[x * 33 + j] = C(x, j), x < 32, j <= 32
 // The Pascal buffer (global) holds: C(x, j) at word x * 33 + j; the offsets
@@ -47,42 +48,19 @@ constexpr int kCbOffs = 32 * kCbStride;
 constexpr int kTailWord = (kCbOffs + kTailBits + 1 + 31) / 32 * 32;
 constexpr int kRevWord = kTailWord + (1 << kTailBits) / 2;
 constexpr int kPascalWords = kRevWord + 32 * kCbStride;
-// The level kernels keep in LDS (s_lvl) C(31 - z, j) << LB at z * 33 + j,
-// indexed by z = leading zeros of a vertex bit, so that neighbour ranks come
-// out as byte offsets, then O_k at kLvlOffs + k.  Every entry read is at
-// most a level's byte count, below 2^32; entries never read may wrap.
+// The level kernels keep in LDS (s_lvl) C(31 - z, j) << SH at z * 33 + j
+// (a tile is 2^SH bytes in each plane), indexed by z = leading zeros of a
+// vertex bit, so that neighbour ranks come out as byte offsets, then O_k at
+// kLvlOffs + k.  Every entry read is at most a level's bytes in one plane,
+// below 2^32; entries never read may wrap.
 constexpr int kLvlOffs = 32 * kCbStride;
 constexpr int kLvlWords = kLvlOffs + kTailBits + 1;
 
-// Folding bytes with packed f16 min / max.  A table byte b (0..65) is put
-// in the HIGH byte of a 16-bit lane, over an arbitrary low byte (another
-// table byte, or 0): the pattern b:lo is a non-negative, finite f16 (b < 0x7C,
-// so the exponent is never all ones; b < 4 gives a denormal, and the kernels
-// keep f16 denormals: float_denorm_mode_16_64 = 3, the default).  Non-negative
-// f16 values order like their bit patterns, so the min / max of such lanes has
-// in its high byte the min / max of their high bytes, whatever the low bytes
-// were, and min / max return one of their inputs bit for bit.  A raw table
-// dword holds bytes 1 and 3 in those positions as loaded; bytes 0 and 2 get
-// there with one shift.  gfx950's three-input v_pk_minimum3_f16 /
-// v_pk_maximum3_f16 then fold two neighbour tiles per instruction.
-constexpr uint32_t kMinSentinel = 0x7B007B00u;  // high bytes 123 > any byte
-__device__ __forceinline__ f16x2 AsF16x2(uint32_t x) {
-  return __builtin_bit_cast(f16x2, x);
-}
-__device__ __forceinline__ f16x2 Min3(f16x2 a, f16x2 b, f16x2 c) {
-  return __builtin_elementwise_minimum(__builtin_elementwise_minimum(a, b), c);
-}
-__device__ __forceinline__ f16x2 Max3(f16x2 a, f16x2 b, f16x2 c) {
-  return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c);
-}
-// bytes 0 and 2 (E) / 1 and 3 (O) of a dword in the high bytes of the lanes
-__device__ __forceinline__ f16x2 EvenBytes(uint32_t x) { return AsF16x2(x << 8); }
-__device__ __forceinline__ f16x2 OddBytes(uint32_t x) { return AsF16x2(x); }
-// high byte of lane `hi` of a folded pair
-__device__ __forceinline__ uint32_t HighByte(f16x2 v, bool hi) {
-  const uint32_t x = __builtin_bit_cast(uint32_t, v);
-  return hi ? x >> 24 : (x >> 8) & 0xFFu;
-}
+// words per tile and log2 of its bytes in one plane
+template <int WB>
+constexpr int kTileWords = 1 << WB;
+template <int WB>
+constexpr int kTileShift = WB + 2;
 
 // Colex unrank of r among the k-subsets of {0..nh-1}; greedy from the top
 // (set_encoder.hpp:61-73) with the binomials read from LDS.  Needs
@@ -104,14 +82,14 @@ __device__ __forceinline__ uint32_t Unrank(uint32_t r, int k, int nh,
 }
 
 // Unrank for the level kernels, on the shifted table: the greedy scan down
-// to vertex 16 with r and the binomials scaled by 2^LB, then one read of the
+// to vertex 16 with r and the binomials scaled by 2^SH, then one read of the
 // 16-bit table for the rest (the remainder is then below C(16, k)).  Same
 // result as Unrank; r < C(nh, k), nh <= 32.
-template <int LB>
+template <int SH>
 __device__ __forceinline__ uint32_t UnrankTiles(uint32_t r, int k, int nh,
                                                 const uint32_t* s_lvl,
                                                 const uint16_t* __restrict__ tail) {
-  uint32_t rs = r << LB;
+  uint32_t rs = r << SH;
   uint32_t H = 0;
   for (int z = 32 - nh; z < 32 - kTailBits; ++z) {  // vertex 31 - z
     const uint32_t c = s_lvl[z * kCbStride + k];
@@ -120,13 +98,13 @@ __device__ __forceinline__ uint32_t UnrankTiles(uint32_t r, int k, int nh,
     H = 2u * H + take;
     k -= static_cast<int>(take);
   }
-  return (H << kTailBits) | tail[s_lvl[kLvlOffs + k] + (rs >> LB)];
+  return (H << kTailBits) | tail[s_lvl[kLvlOffs + k] + (rs >> SH)];
 }
 
 // C(nh, h) from the shifted table
-template <int LB>
+template <int SH>
 __device__ __forceinline__ uint32_t LevelTiles(const uint32_t* s_lvl, int nh, int h) {
-  return s_lvl[(31 - nh) * kCbStride + h] >> LB;
+  return s_lvl[(31 - nh) * kCbStride + h] >> SH;
 }
 
 // Next k-subset in colex order (Gosper's hack, shift instead of divide).
@@ -136,400 +114,164 @@ __device__ __forceinline__ uint32_t NextCombination(uint32_t x) {
   return r | (((x ^ r) >> 2) >> __builtin_ctz(x));
 }
 
-template <int LB>
-__device__ __forceinline__ void LoadTile(const uint8_t* p,
-                                         uint32_t (&w)[(1 << LB) / 4]) {
-  if constexpr (LB == 2) {
+// One plane of a tile (2^WB words).
+template <int WB>
+__device__ __forceinline__ void LoadPlane(const uint8_t* p, uint32_t (&w)[1 << WB]) {
+  if constexpr (WB == 0) {
     w[0] = *reinterpret_cast<const uint32_t*>(p);
-  } else if constexpr (LB == 3) {
+  } else if constexpr (WB == 1) {
     const uint2 v = *reinterpret_cast<const uint2*>(p);
     w[0] = v.x;
     w[1] = v.y;
   } else {
-#pragma unroll
-    for (int i = 0; i < (1 << LB) / 16; ++i) {
-      const uint4 v = reinterpret_cast<const uint4*>(p)[i];
-      w[4 * i + 0] = v.x;
-      w[4 * i + 1] = v.y;
-      w[4 * i + 2] = v.z;
-      w[4 * i + 3] = v.w;
-    }
+    const uint4 v = *reinterpret_cast<const uint4*>(p);
+    w[0] = v.x;
+    w[1] = v.y;
+    w[2] = v.z;
+    w[3] = v.w;
   }
 }
 
-template <int LB>
-__device__ __forceinline__ void StoreTile(uint8_t* p,
-                                          const uint32_t (&w)[(1 << LB) / 4]) {
-  if constexpr (LB == 2) {
+template <int WB>
+__device__ __forceinline__ void StorePlane(uint8_t* p, const uint32_t (&w)[1 << WB]) {
+  if constexpr (WB == 0)
     *reinterpret_cast<uint32_t*>(p) = w[0];
-  } else if constexpr (LB == 3) {
+  else if constexpr (WB == 1)
     *reinterpret_cast<uint2*>(p) = make_uint2(w[0], w[1]);
-  } else {
-#pragma unroll
-    for (int i = 0; i < (1 << LB) / 16; ++i)
-      reinterpret_cast<uint4*>(p)[i] =
-          make_uint4(w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]);
-  }
+  else
+    *reinterpret_cast<uint4*>(p) = make_uint4(w[0], w[1], w[2], w[3]);
 }
 
-// Packed tiles (class layout, LB >= 4).  td(H u L) - td(H) lies in
-// [0, |L|] (one more vertex raises treedepth by at most 1), so a tile stores,
-// per subset, the nibble 2 (td(H u L) - td(H)) + connected <= 2 LB + 1 < 16,
-// and td(H) once, as the byte b = 2 td(H) in a separate array (one byte per
-// tile).  Adding b to a nibble gives the subset's byte 2 td + connected.
-// Nibble dword j holds L = 8j..8j+3 in the low nibbles of its bytes and
-// L = 8j+4..8j+7 in the high nibbles, so the two unpacked dwords are byte
-// dwords 2j and 2j+1 of the byte tile.  The tables take 0.53 of the bytes of
-// byte tiles; on the MI355X at n = 30 the level kernels run 8% slower with
-// them (the unpacking adds VALU work to a kernel that memory latency and
-// VALU issue bound together), so they are the autotuner's to pick.
-// A packed tile as loaded: its nibble dwords and its base byte, unpacked
-// into byte dwords only when folded (half the registers of a byte tile per
-// load in flight).
-template <int LB>
-struct PackedRaw {
-  uint32_t nb[(1 << LB) / 8];
-  uint32_t b;
+template <int WB>
+struct TileWords {
+  uint32_t g0[1 << WB], g1[1 << WB], c[1 << WB];
+  __device__ __forceinline__ DPWord At(int w) const { return {g0[w], g1[w], c[w]}; }
 };
 
-template <int LB>
-__device__ __forceinline__ void LoadPackedRaw(const uint8_t* p, const uint8_t* pb,
-                                              PackedRaw<LB>& r) {
-  if constexpr (LB == 5) {
-    const uint4 v = *reinterpret_cast<const uint4*>(p);
-    r.nb[0] = v.x;
-    r.nb[1] = v.y;
-    r.nb[2] = v.z;
-    r.nb[3] = v.w;
-  } else {
-    const uint2 v = *reinterpret_cast<const uint2*>(p);
-    r.nb[0] = v.x;
-    r.nb[1] = v.y;
+struct AnyLane {
+  __device__ __forceinline__ bool operator()(uint32_t x) const {
+    return __builtin_amdgcn_ballot_w64(x != 0u) != 0ull;
   }
-  r.b = *pb;
-}
+};
 
-template <int LB>
-__device__ __forceinline__ void UnpackRaw(const PackedRaw<LB>& r, uint32_t (&w)[(1 << LB) / 4]) {
-  const uint32_t bb = r.b * 0x01010101u;
-#pragma unroll
-  for (int j = 0; j < (1 << LB) / 8; ++j) {
-    w[2 * j] = (r.nb[j] & 0x0F0F0F0Fu) + bb;
-    w[2 * j + 1] = ((r.nb[j] >> 4) & 0x0F0F0F0Fu) + bb;
-  }
-}
-
-template <int LB>
-__device__ __forceinline__ void StorePacked(uint8_t* p, uint8_t* pb,
-                                            const uint32_t (&w)[(1 << LB) / 4]) {
-  static_assert(LB == 4 || LB == 5, "packed tiles need 16 or 32 subsets");
-  constexpr int NN = (1 << LB) / 8;
-  // every byte is 2 td + c with td >= td(H): no byte borrows below b
-  const uint32_t b = w[0] & 0xFEu;
-  const uint32_t bb = b * 0x01010101u;
-  uint32_t nb[NN];
-#pragma unroll
-  for (int j = 0; j < NN; ++j) nb[j] = (w[2 * j] - bb) | ((w[2 * j + 1] - bb) << 4);
-  if constexpr (NN == 4)
-    *reinterpret_cast<uint4*>(p) = make_uint4(nb[0], nb[1], nb[2], nb[3]);
-  else
-    *reinterpret_cast<uint2*>(p) = make_uint2(nb[0], nb[1]);
-  *pb = static_cast<uint8_t>(b);
-}
-
-// Resolve one tile: all 2^LB subsets H u L of high part H (|H| = h).
-// Plain layout (kClass = false): t = colex rank of H in high level h, prev =
-// first tile of high level h-1, cur = first tile of high level h, Hr = H,
-// k = h.  Class layout (kClass = true): t = colex rank of Hr = H >> cb among
-// the k-subsets of its class, prev / cur = first tile of class p at levels
-// h-1 / h, and x[0..nx) = first tiles of the classes p \ b (b in p) at level
-// h-1, where the neighbour tile H \ b sits at the same rank t.
-// kTiny: h <= 1, the only levels with single-vertex subsets and the only
-// ones where a tile may have fewer than two neighbour tiles.
-// kPack (class layout only): tiles are packed (PackedRaw); prev, cur and
-// x point at the first packed tile of their class and prevb, curb, xb at its
-// base byte.
-template <int LB, bool kClass, bool kTiny, bool kPack = false>
+// Resolve one tile: all subsets of the lb = 5 + WB low vertices joined with
+// the high part H (|H| = h, t = its colex rank).  prev / cur = first tile of
+// high level h-1 / h in plane 0; plane i is i * ps bytes further.
+// kTiny: h <= 1, the only levels with the empty set and single vertices.
+template <int WB, bool kTiny>
 __device__ __forceinline__ void DPTile(const uint8_t* __restrict__ prev,
-                                       uint8_t* __restrict__ cur, uint32_t t,
-                                       uint32_t Hr, int k, uint32_t H, int h,
-                                       const uint8_t* const (&x)[4], int nx,
-                                       const uint32_t* s_lvl,
-                                       const uint32_t* s_tab,
-                                       const uint8_t* __restrict__ prevb = nullptr,
-                                       uint8_t* __restrict__ curb = nullptr,
-                                       const uint8_t* const* xb = nullptr) {
-  static_assert(!kPack || kClass, "packed tiles are a class-layout format");
-  constexpr int NB = 1 << LB;
-  constexpr int NW = NB / 4;
-  // byte-wise min / max of the neighbour tiles, kept as 16-bit lane pairs
-  // (value in the high byte of each lane): E holds bytes 0 and 2 of each
-  // dword, O bytes 1 and 3; orr ORs raw bytes (bit 0 of each byte = "some
-  // S \ x is connected").
-  f16x2 mnE[NW], mnO[NW], mxE[NW], mxO[NW];
-  uint32_t orr[NW];
-  if constexpr (kTiny) {
-#pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      mnE[w] = mnO[w] = AsF16x2(kMinSentinel);
-      mxE[w] = mxO[w] = AsF16x2(0u);
-      orr[w] = 0u;
-    }
-  }
-  // neighbour tiles Hr \ y_j, j = k-1 .. 0 (y_j = j-th smallest of Hr):
-  // rank(Hr \ y_j) = t - C(y_j, j+1) - sum_{i>j} (C(y_i, i+1) - C(y_i, i)),
-  // then (class layout) the nx tiles of the classes p \ b at rank t.
-  // k and nx are uniform across the wave, so every guard below is uniform.
-  // Up to four loads are issued before their tiles are folded, in pairs
-  // (three-input min / max, three-input or).
-  // B = (t - sum_{i>j} (C(y_i, i+1) - C(y_i, i))) << LB runs down with j.  Byte
-  // offsets within a level fit 32 bits (a level is at most C(32,16) bytes),
-  // so the loads use a uniform base plus a 32-bit lane offset.
-  uint32_t rem = Hr;
-  uint32_t B = t << LB;
-  const int total = kClass ? k + nx : k;
-  auto load = [&](int i, uint32_t (&wv)[NW]) {
-    if (!kClass || i < k) {
-      const int j = k - 1 - i;
-      const int z = __builtin_clz(rem);  // y_j = 31 - z
-      rem ^= 0x80000000u >> z;
-      const uint32_t c1 = s_lvl[z * kCbStride + j + 1];
-      const uint32_t c0 = s_lvl[z * kCbStride + j];
-      const uint32_t off = B - c1;  // rank(Hr \ y_j) << LB
-      B = off + c0;
-      LoadTile<LB>(prev + off, wv);
-    } else {
-      const int c = i - k;
-      const uint8_t* base = c == 0 ? x[0] : c == 1 ? x[1] : c == 2 ? x[2] : x[3];
-      LoadTile<LB>(base + (t << LB), wv);
-    }
-  };
-  auto fold2 = [&](const uint32_t (&wa)[NW], const uint32_t (&wb)[NW]) {
-#pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      const uint32_t a = wa[w], b = wb[w];
-      mnE[w] = Min3(mnE[w], EvenBytes(a), EvenBytes(b));
-      mnO[w] = Min3(mnO[w], OddBytes(a), OddBytes(b));
-      mxE[w] = Max3(mxE[w], EvenBytes(a), EvenBytes(b));
-      mxO[w] = Max3(mxO[w], OddBytes(a), OddBytes(b));
-      orr[w] = orr[w] | a | b;
-    }
+                                       uint8_t* __restrict__ cur, size_t ps, uint32_t t,
+                                       uint32_t H, int h, const uint32_t* s_lvl,
+                                       const uint32_t* s_tab) {
+  constexpr int W = kTileWords<WB>, SH = kTileShift<WB>;
+  DPFold f[W];
+  // neighbour tiles H \ y_j, j = h-1 .. 0 (y_j = j-th smallest of H):
+  // rank(H \ y_j) = t - C(y_j, j+1) - sum_{i>j} (C(y_i, i+1) - C(y_i, i)).
+  // h is uniform across the wave, so every guard below is uniform.
+  // Up to four tiles' loads are issued before they are folded, in pairs.
+  // B = (t - sum_{i>j} (C(y_i, i+1) - C(y_i, i))) << SH runs down with j.  Byte
+  // offsets within a level fit 32 bits, so the loads use a uniform base plus
+  // a 32-bit lane offset.
+  uint32_t rem = H;
+  uint32_t B = t << SH;
+  auto load = [&](int i, TileWords<WB>& v) {
+    const int j = h - 1 - i;
+    const int z = __builtin_clz(rem);  // y_j = 31 - z
+    rem ^= 0x80000000u >> z;
+    const uint32_t c1 = s_lvl[z * kCbStride + j + 1];
+    const uint32_t c0 = s_lvl[z * kCbStride + j];
+    const uint32_t off = B - c1;  // rank(H \ y_j) << SH
+    B = off + c0;
+    LoadPlane<WB>(prev + off, v.g0);
+    LoadPlane<WB>(prev + ps + off, v.g1);
+    LoadPlane<WB>(prev + 2 * ps + off, v.c);
   };
   int i = 0;
-  if constexpr (kPack) {
-    // packed tiles: up to eight loads in flight (raw, 5 registers each),
-    // folded in pairs from sentinels (a three-input min / max against the
-    // sentinel costs what a two-input one does)
-    if constexpr (!kTiny) {
+  for (; i + 4 <= h; i += 4) {
+    TileWords<WB> v0, v1, v2, v3;
+    load(i, v0);
+    load(i + 1, v1);
+    load(i + 2, v2);
+    load(i + 3, v3);
 #pragma unroll
-      for (int w = 0; w < NW; ++w) {
-        mnE[w] = mnO[w] = AsF16x2(kMinSentinel);
-        mxE[w] = mxO[w] = AsF16x2(0u);
-        orr[w] = 0u;
-      }
-    }
-    auto raw = [&](int q, PackedRaw<LB>& r) {
-      if (q < k) {
-        const int j = k - 1 - q;
-        const int z = __builtin_clz(rem);  // y_j = 31 - z
-        rem ^= 0x80000000u >> z;
-        const uint32_t c1 = s_lvl[z * kCbStride + j + 1];
-        const uint32_t c0 = s_lvl[z * kCbStride + j];
-        const uint32_t off = B - c1;  // rank(Hr \ y_j) << LB
-        B = off + c0;
-        LoadPackedRaw<LB>(prev + (off >> 1), prevb + (off >> LB), r);
-      } else {
-        const int c = q - k;
-        const uint8_t* base = c == 0 ? x[0] : c == 1 ? x[1] : c == 2 ? x[2] : x[3];
-        const uint8_t* bbase = c == 0 ? xb[0] : c == 1 ? xb[1] : c == 2 ? xb[2] : xb[3];
-        LoadPackedRaw<LB>(base + (t << (LB - 1)), bbase + t, r);
-      }
-    };
-    auto foldraw = [&](const PackedRaw<LB>& ra, const PackedRaw<LB>& rb) {
-      uint32_t wa[NW], wb[NW];
-      UnpackRaw<LB>(ra, wa);
-      UnpackRaw<LB>(rb, wb);
-      fold2(wa, wb);
-    };
-    for (; i + 8 <= total; i += 8) {
-      PackedRaw<LB> r[8];
+    for (int w = 0; w < W; ++w) f[w].Add2(v0.At(w), v1.At(w));
 #pragma unroll
-      for (int q = 0; q < 8; ++q) raw(i + q, r[q]);
-#pragma unroll
-      for (int q = 0; q < 8; q += 2) foldraw(r[q], r[q + 1]);
-    }
-    if (i + 4 <= total) {
-      PackedRaw<LB> r[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) raw(i + q, r[q]);
-      foldraw(r[0], r[1]);
-      foldraw(r[2], r[3]);
-      i += 4;
-    }
-    if (i + 2 <= total) {
-      PackedRaw<LB> r[2];
-      raw(i, r[0]);
-      raw(i + 1, r[1]);
-      foldraw(r[0], r[1]);
-      i += 2;
-    }
-    if (i < total) {
-      PackedRaw<LB> r0;
-      raw(i, r0);
-      uint32_t w0[NW];
-      UnpackRaw<LB>(r0, w0);
-#pragma unroll
-      for (int w = 0; w < NW; ++w) {
-        mnE[w] = __builtin_elementwise_minimum(mnE[w], EvenBytes(w0[w]));
-        mnO[w] = __builtin_elementwise_minimum(mnO[w], OddBytes(w0[w]));
-        mxE[w] = __builtin_elementwise_maximum(mxE[w], EvenBytes(w0[w]));
-        mxO[w] = __builtin_elementwise_maximum(mxO[w], OddBytes(w0[w]));
-        orr[w] |= w0[w];
-      }
-      i = total;
-    }
+    for (int w = 0; w < W; ++w) f[w].Add2(v2.At(w), v3.At(w));
   }
-  if constexpr (!kTiny && !kPack) {
-    // h >= 2, so at least two neighbour tiles: the first two start the fold
-    uint32_t wa[NW], wb[NW];
-    load(0, wa);
-    load(1, wb);
+  if (i + 2 <= h) {
+    TileWords<WB> v0, v1;
+    load(i, v0);
+    load(i + 1, v1);
 #pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      const f16x2 ae = EvenBytes(wa[w]), ao = OddBytes(wa[w]);
-      const f16x2 be = EvenBytes(wb[w]), bo = OddBytes(wb[w]);
-      mnE[w] = __builtin_elementwise_minimum(ae, be);
-      mnO[w] = __builtin_elementwise_minimum(ao, bo);
-      mxE[w] = __builtin_elementwise_maximum(ae, be);
-      mxO[w] = __builtin_elementwise_maximum(ao, bo);
-      orr[w] = wa[w] | wb[w];
-    }
-    i = 2;
-  }
-  for (; !kPack && i + 4 <= total; i += 4) {
-    uint32_t w0[NW], w1[NW], w2[NW], w3[NW];
-    load(i, w0);
-    load(i + 1, w1);
-    load(i + 2, w2);
-    load(i + 3, w3);
-    fold2(w0, w1);
-    fold2(w2, w3);
-  }
-  if (!kPack && i + 2 <= total) {
-    uint32_t w0[NW], w1[NW];
-    load(i, w0);
-    load(i + 1, w1);
-    fold2(w0, w1);
+    for (int w = 0; w < W; ++w) f[w].Add2(v0.At(w), v1.At(w));
     i += 2;
   }
-  if (!kPack && i < total) {
-    uint32_t w0[NW];
-    load(i, w0);
+  if (i < h) {
+    TileWords<WB> v0;
+    load(i, v0);
 #pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      mnE[w] = __builtin_elementwise_minimum(mnE[w], EvenBytes(w0[w]));
-      mnO[w] = __builtin_elementwise_minimum(mnO[w], OddBytes(w0[w]));
-      mxE[w] = __builtin_elementwise_maximum(mxE[w], EvenBytes(w0[w]));
-      mxO[w] = __builtin_elementwise_maximum(mxO[w], OddBytes(w0[w]));
-      orr[w] |= w0[w];
-    }
+    for (int w = 0; w < W; ++w) f[w].Add(v0.g0[w], v0.g1[w], v0.c[w]);
   }
-  // Connectivity.  S = H u L is connected iff no vertex of S is isolated in S
-  // and some S \ v is connected (or S is a single vertex).  The first part
-  // is one mask per tile, F, over the 2^LB low parts, in the tile-mask bit
-  // order (bit 8 (L & 3) + (L >> 2) for low part L, so that F >> w holds the
-  // four low parts of dword w in bit 0 of its bytes):
-  //   high x in H with no neighbour in H needs a neighbour in L;
-  //   low y in L with no neighbour in H needs a neighbour in L;
-  // both from per-graph tables (7-bit chunks of the isolated high vertices,
-  // and the set of low vertices H does not reach).
-  const uint32_t NH = s_tab[kTabNbh + (H & 127u)] |
-                      s_tab[kTabNbh + 128 + ((H >> 7) & 127u)] |
-                      s_tab[kTabNbh + 256 + ((H >> 14) & 127u)] |
-                      s_tab[kTabNbh + 384 + ((H >> 21) & 127u)];
-  const uint32_t IH = H & ~(NH >> LB);
-  const uint32_t W = ~NH & ((1u << LB) - 1u);
-  const uint32_t F = s_tab[kTabIsoL + W] & s_tab[kTabIsoH + (IH & 127u)] &
-                     s_tab[kTabIsoH + 128 + ((IH >> 7) & 127u)] &
-                     s_tab[kTabIsoH + 256 + ((IH >> 14) & 127u)] &
-                     s_tab[kTabIsoH + 384 + ((IH >> 21) & 127u)];
-  // The second part, bytewise: C[w] has bit 0 of byte b set iff low part
-  // 4w + b gives a connected S.  Predecessors of 4w + b: the same byte of
-  // the neighbour tiles (orr), the same byte of dwords w \ j (done before w),
-  // and inside the dword byte 0 -> bytes 1, 2 -> byte 3.
-  uint32_t C[NW];
+  // No vertex of S isolated in S, for the 32 subsets of each word, from
+  // per-graph tables over 7-bit chunks of the vertices above 4:
+  //   a vertex of H or of w with no neighbour there needs one in L;
+  //   a vertex of L with no neighbour in H or w needs one in L.
+  const uint32_t Hw = H << WB;
+  const uint32_t NH = s_tab[kTabNbh + (Hw & 127u)] |
+                      s_tab[kTabNbh + 128 + ((Hw >> 7) & 127u)] |
+                      s_tab[kTabNbh + 256 + ((Hw >> 14) & 127u)] |
+                      s_tab[kTabNbh + 384 + ((Hw >> 21) & 127u)];
+  TileWords<WB> out;
 #pragma unroll
-  for (int w = 0; w < NW; ++w) {
-    uint32_t a = orr[w];
+  for (int w = 0; w < W; ++w) {
+    const uint32_t N = w ? NH | s_tab[kTabNbh + w] : NH;
+    const uint32_t I = (Hw | static_cast<uint32_t>(w)) & ~(N >> 5);
+    const uint32_t fine = s_tab[kTabIsoL + (~N & 31u)] & s_tab[kTabIsoH + (I & 127u)] &
+                          s_tab[kTabIsoH + 128 + ((I >> 7) & 127u)] &
+                          s_tab[kTabIsoH + 256 + ((I >> 14) & 127u)] &
+                          s_tab[kTabIsoH + 384 + ((I >> 21) & 127u)];
+    // the words of w \ b are neighbours too
 #pragma unroll
-    for (int j = 0; j < LB - 2; ++j)
-      if (w >> j & 1) a |= C[w ^ (1 << j)];
-    uint32_t Fw = (F >> w) & 0x01010101u;
+    for (int b = 0; b < WB; ++b)
+      if (w >> b & 1) f[w].Add(out.g0[w ^ (1 << b)], out.g1[w ^ (1 << b)], out.c[w ^ (1 << b)]);
+    uint32_t single = 0u;
+    bool empty = false;
     if constexpr (kTiny) {
-      // single vertices: L = {l} at h = 0 (bytes 1, 2 of dword 0 and byte 0
-      // of dwords 1, 2, 4), L = 0 at h = 1
-      uint32_t single = 0u;
-      if (h == 0) single = w == 0 ? 0x00010100u : (w & (w - 1)) == 0 ? 1u : 0u;
-      else if (w == 0) single = 1u;
-      Fw |= single;
-      a |= single;
+      const int size = h + __builtin_popcount(static_cast<unsigned>(w));
+      single = size == 0 ? 0x00010116u : size == 1 ? 1u : 0u;
+      empty = size == 0;
     }
-    a &= Fw;
-    a = (a | __builtin_amdgcn_perm(a, a, 0x0c00000cu)) & Fw;
-    a = (a | ((a << 8 | a << 16) & 0xFF000000u)) & Fw;
-    C[w] = a;
+    const DPWord r = SolveWord(f[w], fine, single, empty, AnyLane());
+    out.g0[w] = r.g0;
+    out.g1[w] = r.g1;
+    out.c[w] = r.c;
   }
-  // Values, kept as 2 td + junk (bit 0 is left as min / max found it; only
-  // the td part orders): connected -> 1 + min, else max; bit 0 := C at the end.
-  uint32_t V[NB];
-#pragma unroll
-  for (int L = 0; L < NB; ++L) {
-    const int w = L >> 2;
-    uint32_t m = HighByte((L & 1) ? mnO[w] : mnE[w], L & 2);
-    uint32_t M = HighByte((L & 1) ? mxO[w] : mxE[w], L & 2);
-#pragma unroll
-    for (int l = 0; l < LB; ++l) {
-      if (L >> l & 1) {
-        const uint32_t v = V[L ^ (1 << l)];
-        m = min(m, v);
-        M = max(M, v);
-      }
-    }
-    const bool conn = ((C[w] >> (8 * (L & 3))) & 0xFFu) != 0u;
-    V[L] = conn ? m + 2u : M;
-  }
-  uint32_t ow[NW];
-#pragma unroll
-  for (int w = 0; w < NW; ++w)
-    ow[w] = ((V[4 * w] | (V[4 * w + 1] << 8) | (V[4 * w + 2] << 16) |
-              (V[4 * w + 3] << 24)) & 0xFEFEFEFEu) | C[w];
-  if constexpr (kPack)
-    StorePacked<LB>(cur + (t << (LB - 1)), curb + t, ow);
-  else
-    StoreTile<LB>(cur + (t << LB), ow);
+  StorePlane<WB>(cur + (t << SH), out.g0);
+  StorePlane<WB>(cur + ps + (t << SH), out.g1);
+  StorePlane<WB>(cur + 2 * ps + (t << SH), out.c);
 }
 
-template <int LB>
+template <int WB>
 __device__ __forceinline__ void LoadPascal(const uint32_t* __restrict__ g_cb,
                                            uint32_t* s_lvl) {
   for (int i = threadIdx.x; i < 32 * kCbStride; i += blockDim.x)
-    s_lvl[i] = g_cb[kRevWord + i] << LB;
+    s_lvl[i] = g_cb[kRevWord + i] << kTileShift<WB>;
   if (threadIdx.x <= kTailBits) s_lvl[kLvlOffs + threadIdx.x] = g_cb[kCbOffs + threadIdx.x];
 }
 
-template <int LB>
+template <int WB>
 __device__ __forceinline__ void LoadShared(const DPGraph* __restrict__ g,
                                            const uint32_t* __restrict__ g_cb,
                                            uint32_t* s_lvl, uint32_t* s_tab,
                                            bool load_cb) {
-  if (load_cb) LoadPascal<LB>(g_cb, s_lvl);
+  if (load_cb) LoadPascal<WB>(g_cb, s_lvl);
   // nbh, isoh and isol are consecutive in DPGraph
   for (int i = threadIdx.x; i < kTabWords; i += blockDim.x) s_tab[i] = g->nbh[i];
 }
 
 // Tiles [first, end) of high level h of graph g, R consecutive per lane,
 // lanes of the launch striding by `stride` tiles.
-template <int LB>
+template <int WB>
 __device__ __forceinline__ void DPLevelRange(const DPGraph* __restrict__ g,
                                              const uint32_t* __restrict__ g_cb,
                                              uint8_t* __restrict__ arena,
@@ -539,20 +281,21 @@ __device__ __forceinline__ void DPLevelRange(const DPGraph* __restrict__ g,
                                              const uint32_t* s_lvl,
                                              const uint32_t* s_tab) {
   const int nh = static_cast<int>(g->nh);
+  constexpr int SH = kTileShift<WB>;
   uint8_t* base = arena + g->table;
   const uint8_t* prev =
-      h > 0 ? base + (static_cast<size_t>(g->lvl[h - 1]) << LB) : base;
-  uint8_t* cur = base + (static_cast<size_t>(g->lvl[h]) << LB);
-  const uint8_t* const none[4] = {nullptr, nullptr, nullptr, nullptr};
+      h > 0 ? base + (static_cast<size_t>(g->lvl[h - 1]) << SH) : base;
+  uint8_t* cur = base + (static_cast<size_t>(g->lvl[h]) << SH);
+  const size_t ps = static_cast<size_t>(g->lvl[nh + 1]) << SH;
   const uint16_t* tail = reinterpret_cast<const uint16_t*>(g_cb + kTailWord);
   for (uint32_t t0 = first + lane_id * R; t0 < end; t0 += stride) {
-    uint32_t H = UnrankTiles<LB>(t0, h, nh, s_lvl, tail);
+    uint32_t H = UnrankTiles<kTileShift<WB>>(t0, h, nh, s_lvl, tail);
     const uint32_t tend = min(t0 + static_cast<uint32_t>(R), end);
     for (uint32_t t = t0;;) {
       if (h <= 1)
-        DPTile<LB, false, true>(prev, cur, t, H, h, H, h, none, 0, s_lvl, s_tab);
+        DPTile<WB, true>(prev, cur, ps, t, H, h, s_lvl, s_tab);
       else
-        DPTile<LB, false, false>(prev, cur, t, H, h, H, h, none, 0, s_lvl, s_tab);
+        DPTile<WB, false>(prev, cur, ps, t, H, h, s_lvl, s_tab);
       if (++t >= tend) break;
       H = NextCombination(H);
     }
@@ -561,98 +304,28 @@ __device__ __forceinline__ void DPLevelRange(const DPGraph* __restrict__ g,
 
 // One high level of one graph.
 // Workgroups are dealt to the 8 XCDs round-robin (workgroup i -> XCD i % 8).
-// With xcd_remap the tile range is cut into 8 contiguous slices and XCD x
-// works through slice x, so the neighbour tiles that consecutive tiles share
-// stay in one XCD's L2.  Needs gridDim.x % 8 == 0 (the host ensures it).
+// The tile range is cut into 8 contiguous slices and XCD x works through
+// slice x (where the grid is a multiple of 8, which the host sees to for
+// grids of 64 and more), so the neighbour tiles that consecutive tiles share
+// are fetched by one XCD's L2 instead of by all eight.  At n = 30 (two graphs
+// in flight, 128-subset tiles, 256 threads) a graph takes 430 us with slices
+// and 500 us without; at n <= 26 both take the same.
 constexpr uint32_t kXcds = 8;
 
-template <int LB>
+template <int WB>
 __global__ __launch_bounds__(1024) void DPLevelKernel(
     const DPGraph* __restrict__ g, const uint32_t* __restrict__ g_cb,
-    uint8_t* __restrict__ arena, int h, uint32_t ntiles, int R, int xcd_remap) {
+    uint8_t* __restrict__ arena, int h, uint32_t ntiles, int R) {
   __shared__ uint32_t s_lvl[kLvlWords];
   __shared__ uint32_t s_tab[kTabWords];
-  LoadShared<LB>(g, g_cb, s_lvl, s_tab, true);
+  LoadShared<WB>(g, g_cb, s_lvl, s_tab, true);
   __syncthreads();
   uint32_t bid = blockIdx.x;
-  if (xcd_remap && gridDim.x % kXcds == 0)
+  if (gridDim.x % kXcds == 0)
     bid = (bid % kXcds) * (gridDim.x / kXcds) + bid / kXcds;
   const uint32_t lane_id = bid * blockDim.x + threadIdx.x;
   const uint32_t stride = gridDim.x * blockDim.x * R;
-  DPLevelRange<LB>(g, g_cb, arena, h, 0, ntiles, lane_id, stride, R, s_lvl, s_tab);
-}
-
-// Static schedule of one class-layout level launch: for each XCD, up to
-// kMaxSeg segments (class p, tiles [first, end) of that class), with the tile
-// offsets of class p at levels h-1 and h and of the classes p \ b at h-1.
-constexpr int kMaxSeg = 12;
-struct ClassSeg {
-  uint32_t p, first, end, prev, cur, x[4];
-};
-struct ClassSched {
-  uint32_t nseg[kXcds];
-  ClassSeg seg[kXcds][kMaxSeg];
-};
-
-// One high level of one graph in the class layout (cb = 3 or 4).  The host
-// gives each XCD its own classes (class p belongs to XCD p mod 8 for cb = 3;
-// for cb = 4 to XCD p and 15 - p, one class of each complementary pair) and
-// moves the tail of over-full XCDs' classes to the others, so every XCD gets
-// the same number of tiles.  Workgroups are dealt to XCDs round-robin, so
-// workgroup w works for XCD w mod 8: the XCD's workgroups walk its segments
-// in order, chunk c of a segment going to its workgroup c mod (grid / 8).
-// An XCD's neighbour reads stay in its classes' part of level h-1 and in its
-// own L2.  No atomics and no barriers.
-template <int LB, bool kPack>
-__global__ __launch_bounds__(1024) void DPClassLevelKernel(
-    const DPGraph* __restrict__ g, const uint32_t* __restrict__ g_cb,
-    uint8_t* __restrict__ arena, int h, int R, const ClassSched sched) {
-  __shared__ uint32_t s_lvl[kLvlWords];
-  __shared__ uint32_t s_tab[kTabWords];
-  LoadShared<LB>(g, g_cb, s_lvl, s_tab, true);
-  __syncthreads();
-  const int cb = static_cast<int>(g->cb);
-  const int rest = static_cast<int>(g->nh) - cb;
-  const uint16_t* tail = reinterpret_cast<const uint16_t*>(g_cb + kTailWord);
-  const uint32_t CH = blockDim.x * static_cast<uint32_t>(R);
-  const uint32_t xcd = blockIdx.x % kXcds;
-  const uint32_t wx = blockIdx.x / kXcds, gx = gridDim.x / kXcds;
-  uint8_t* base = arena + g->table;
-  // packed: tiles of 2^(LB-1) bytes, then the base bytes, one per tile
-  constexpr int TS = kPack ? LB - 1 : LB;
-  uint8_t* bytes = base + (static_cast<size_t>(g->lvl[g->nh + 1]) << TS);
-  const uint32_t nseg = sched.nseg[xcd];
-  for (uint32_t s = 0; s < nseg; ++s) {
-    const ClassSeg& sg = sched.seg[xcd][s];
-    const uint32_t p = sg.p;
-    const int np = __builtin_popcount(p);
-    const int k = h - np;
-    const uint8_t* prev = base + (static_cast<size_t>(sg.prev) << TS);
-    uint8_t* cur = base + (static_cast<size_t>(sg.cur) << TS);
-    const uint8_t* const x[4] = {base + (static_cast<size_t>(sg.x[0]) << TS),
-                                 base + (static_cast<size_t>(sg.x[1]) << TS),
-                                 base + (static_cast<size_t>(sg.x[2]) << TS),
-                                 base + (static_cast<size_t>(sg.x[3]) << TS)};
-    const uint8_t* const xb[4] = {bytes + sg.x[0], bytes + sg.x[1], bytes + sg.x[2],
-                                  bytes + sg.x[3]};
-    for (uint32_t c0 = sg.first + wx * CH; c0 < sg.end; c0 += gx * CH) {
-      const uint32_t t0 = c0 + threadIdx.x * static_cast<uint32_t>(R);
-      if (t0 >= sg.end) continue;
-      uint32_t Hr = UnrankTiles<LB>(t0, k, rest, s_lvl, tail);
-      const uint32_t tend = min(t0 + static_cast<uint32_t>(R), sg.end);
-      for (uint32_t t = t0;;) {
-        const uint32_t H = p | (Hr << cb);
-        if (h <= 1)
-          DPTile<LB, true, true, kPack>(prev, cur, t, Hr, k, H, h, x, np, s_lvl, s_tab,
-                                        bytes + sg.prev, bytes + sg.cur, xb);
-        else
-          DPTile<LB, true, false, kPack>(prev, cur, t, Hr, k, H, h, x, np, s_lvl, s_tab,
-                                         bytes + sg.prev, bytes + sg.cur, xb);
-        if (++t >= tend) break;
-        Hr = NextCombination(Hr);
-      }
-    }
-  }
+  DPLevelRange<WB>(g, g_cb, arena, h, 0, ntiles, lane_id, stride, R, s_lvl, s_tab);
 }
 
 // Level-synchronous batch: one launch per high level h over all graphs;
@@ -661,7 +334,7 @@ struct Chunk {
   uint32_t gi, first, end, pad;
 };
 
-template <int LB>
+template <int WB>
 __global__ __launch_bounds__(1024) void DPChunkKernel(
     const DPGraph* __restrict__ gs, const uint32_t* __restrict__ g_cb,
     uint8_t* __restrict__ arena, const Chunk* __restrict__ chunks, int h,
@@ -670,9 +343,9 @@ __global__ __launch_bounds__(1024) void DPChunkKernel(
   __shared__ uint32_t s_tab[kTabWords];
   const Chunk c = chunks[blockIdx.x];
   const DPGraph* g = gs + c.gi;
-  LoadShared<LB>(g, g_cb, s_lvl, s_tab, true);
+  LoadShared<WB>(g, g_cb, s_lvl, s_tab, true);
   __syncthreads();
-  DPLevelRange<LB>(g, g_cb, arena, h, c.first, c.end, threadIdx.x,
+  DPLevelRange<WB>(g, g_cb, arena, h, c.first, c.end, threadIdx.x,
                    blockDim.x * R, R, s_lvl, s_tab);
 }
 
@@ -680,20 +353,15 @@ __global__ __launch_bounds__(1024) void DPChunkKernel(
 // pre-sorted largest first) and resolve every level of a graph with a
 // workgroup barrier between levels, so no level of a graph ever waits on
 // another workgroup and the graph's tables stay in one XCD's L2.
-// Masks over the low parts L of a tile (tile-mask bit order: bit
-// 8 (L & 3) + (L >> 2) stands for L): s_m[0] = every L, s_m[1 + T] = the L
-// meeting T (none for T = 0), s_m[33 + y] = the L without low vertex y.
-constexpr int kLowMaskWords = 38;
-template <int LB>
+// Masks over the 32 low parts L of a word: s_m[T] = the L meeting the low set
+// T (none for T = 0), s_m[32 + y] = the L without low vertex y.
+constexpr int kLowMaskWords = 37;
 __device__ __forceinline__ void LowMasksShared(uint32_t* s_m) {
-  const int t = threadIdx.x;
-  if (t < 38) {
+  const uint32_t t = threadIdx.x;
+  if (t < kLowMaskWords) {
     uint32_t m = 0;
-    for (int L = 0; L < (1 << LB); ++L) {
-      const bool take = t == 0 ? true : t < 33 ? (L & (t - 1)) != 0
-                                               : (t - 33 < LB && !((L >> (t - 33)) & 1));
-      if (take) m |= 1u << (8 * (L & 3) + (L >> 2));
-    }
+    for (uint32_t L = 0; L < 32; ++L)
+      if (t < 32 ? (L & t) != 0u : !(L >> (t - 32) & 1u)) m |= 1u << L;
     s_m[t] = m;
   }
 }
@@ -702,46 +370,37 @@ __device__ __forceinline__ void LowMasksShared(uint32_t* s_m) {
 // nbh / isoh / isol arrays MakeGraph builds on the host), built in LDS from
 // g's adjacency rows: entry by entry the same unions and intersections over
 // the bits of each chunk.  s_m from LowMasksShared.
-template <int LB>
 __device__ __forceinline__ void BuildTables(const DPGraph* __restrict__ g, const uint32_t* s_m,
                                             uint32_t* s_tab) {
-  const int nh = static_cast<int>(g->nh);
-  constexpr uint32_t kLow = (1u << LB) - 1u;
+  const int n = static_cast<int>(g->n);
   for (int i = threadIdx.x; i < kTabWords; i += blockDim.x) {
     uint32_t m;
     if (i < kTabIsoH) {  // N(chunk) = union of its vertices' rows
       const int c = i >> 7;
       m = 0;
       for (uint32_t ch = i & 127; ch; ch &= ch - 1) {
-        const int x = 7 * c + __builtin_ctz(ch);
-        if (x < nh) m |= g->adj[LB + x];
+        const int x = 5 + 7 * c + __builtin_ctz(ch);
+        if (x < n) m |= g->adj[x];
       }
     } else if (i < kTabIsoL) {  // the L that give every x of the chunk a neighbour
       const int j = i - kTabIsoH, c = j >> 7;
-      m = s_m[0];
+      m = ~0u;
       for (uint32_t ch = j & 127; ch; ch &= ch - 1) {
-        const int x = 7 * c + __builtin_ctz(ch);
-        const uint32_t low = x < nh ? g->adj[LB + x] & kLow : 0u;
-        m &= low ? s_m[1 + low] : 0u;
+        const int x = 5 + 7 * c + __builtin_ctz(ch);
+        m &= x < n ? s_m[g->adj[x] & 31u] : 0u;
       }
     } else {  // the L in which every y of Y n L has a neighbour in L
-      const uint32_t Y = static_cast<uint32_t>(i - kTabIsoL);
-      if (Y > kLow) {
-        m = 0;
-      } else {
-        m = s_m[0];
-        for (uint32_t yy = Y; yy; yy &= yy - 1) {
-          const int y = __builtin_ctz(yy);
-          const uint32_t low = g->adj[y] & kLow;
-          m &= s_m[33 + y] | (low ? s_m[1 + low] : 0u);
-        }
+      m = ~0u;
+      for (uint32_t yy = static_cast<uint32_t>(i - kTabIsoL); yy; yy &= yy - 1) {
+        const int y = __builtin_ctz(yy);
+        m &= s_m[32 + y] | s_m[g->adj[y] & 31u];
       }
     }
     s_tab[i] = m;
   }
 }
 
-template <int LB>
+template <int WB>
 __global__ __launch_bounds__(1024) void DPPersistentKernel(
     const DPGraph* __restrict__ gs, const uint32_t* __restrict__ g_cb,
     uint8_t* __restrict__ arena, int ngraphs, uint32_t* __restrict__ queue,
@@ -750,8 +409,8 @@ __global__ __launch_bounds__(1024) void DPPersistentKernel(
   __shared__ uint32_t s_tab[kTabWords];
   __shared__ uint32_t s_masks[kLowMaskWords];
   __shared__ int s_gi;
-  LoadPascal<LB>(g_cb, s_lvl);
-  LowMasksShared<LB>(s_masks);
+  LoadPascal<WB>(g_cb, s_lvl);
+  LowMasksShared(s_masks);
   for (;;) {
     if (threadIdx.x == 0) s_gi = static_cast<int>(atomicAdd(queue, 1u));
     __syncthreads();
@@ -759,12 +418,12 @@ __global__ __launch_bounds__(1024) void DPPersistentKernel(
     if (gi >= ngraphs) break;  // uniform: every thread read the same s_gi
     const DPGraph* g = gs + gi;
     // only the record's head (up to nbh) comes from the host
-    BuildTables<LB>(g, s_masks, s_tab);
+    BuildTables(g, s_masks, s_tab);
     __syncthreads();
     const int nh = static_cast<int>(g->nh);
     for (int h = 0; h <= nh; ++h) {
-      const uint32_t ntiles = LevelTiles<LB>(s_lvl, nh, h);  // no padding
-      DPLevelRange<LB>(g, g_cb, arena, h, 0, ntiles, threadIdx.x, blockDim.x * R, R,
+      const uint32_t ntiles = LevelTiles<kTileShift<WB>>(s_lvl, nh, h);  // no padding
+      DPLevelRange<WB>(g, g_cb, arena, h, 0, ntiles, threadIdx.x, blockDim.x * R, R,
                        s_lvl, s_tab);
       __syncthreads();
     }
@@ -774,18 +433,18 @@ __global__ __launch_bounds__(1024) void DPPersistentKernel(
 // A run of small high levels [h0, h1] of one graph in one workgroup, with a
 // workgroup barrier between levels (the first and last levels of a large
 // graph have few tiles; one launch replaces h1 - h0 + 1 of them).
-template <int LB>
+template <int WB>
 __global__ __launch_bounds__(1024) void DPSmallLevelsKernel(
     const DPGraph* __restrict__ g, const uint32_t* __restrict__ g_cb,
     uint8_t* __restrict__ arena, int h0, int h1) {
   __shared__ uint32_t s_lvl[kLvlWords];
   __shared__ uint32_t s_tab[kTabWords];
-  LoadShared<LB>(g, g_cb, s_lvl, s_tab, true);
+  LoadShared<WB>(g, g_cb, s_lvl, s_tab, true);
   __syncthreads();
   const int nh = static_cast<int>(g->nh);
   for (int h = h0; h <= h1; ++h) {
-    const uint32_t ntiles = LevelTiles<LB>(s_lvl, nh, h);
-    DPLevelRange<LB>(g, g_cb, arena, h, 0, ntiles, threadIdx.x, blockDim.x, 1, s_lvl, s_tab);
+    const uint32_t ntiles = LevelTiles<kTileShift<WB>>(s_lvl, nh, h);
+    DPLevelRange<WB>(g, g_cb, arena, h, 0, ntiles, threadIdx.x, blockDim.x, 1, s_lvl, s_tab);
     __syncthreads();
   }
 }
@@ -794,53 +453,72 @@ __global__ void ResetCounter(uint32_t* c) {
   if (threadIdx.x == 0 && blockIdx.x == 0) *c = 0u;
 }
 
-// td of subset S (raw byte >> 1) of graph g.
-// Binomials, the level offsets (read per lane, so LDS spares a memory round
-// trip before each table read) and, for a class layout, the first tile of
-// each class per high level: s_cbase[16 h + p] = ClassBase(h, p, nh - cb),
-// all in LDS.  s_cbase[kCbaseWords..] holds lvl[].  Ends with a barrier.
-constexpr int kCbaseWords = 33 * 16;
-constexpr int kLookupWords = kCbaseWords + 34;
+// Binomials and the level offsets (read per lane, so LDS spares a memory
+// round trip before each table read).  Ends with a barrier.
+constexpr int kLookupWords = 34;
 __device__ __forceinline__ void LoadLookupTables(const DPGraph* __restrict__ g,
                                                  const uint32_t* __restrict__ g_cb,
-                                                 uint32_t* s_cb, uint32_t* s_cbase) {
+                                                 uint32_t* s_cb, uint32_t* s_base) {
   for (int i = threadIdx.x; i < 32 * kCbStride; i += blockDim.x) s_cb[i] = g_cb[i];
-  for (int i = threadIdx.x; i < 34; i += blockDim.x) s_cbase[kCbaseWords + i] = g->lvl[i];
-  __syncthreads();
-  const int cb = static_cast<int>(g->cb), nh = static_cast<int>(g->nh);
-  if (cb > 0)
-    for (int i = threadIdx.x; i < (nh + 1) * 16; i += blockDim.x)
-      s_cbase[i] = ClassBase(i >> 4, static_cast<uint32_t>(i & 15), nh - cb,
-                             [&](int x, int j) { return s_cb[x * kCbStride + j]; });
+  for (int i = threadIdx.x; i < kLookupWords; i += blockDim.x) s_base[i] = g->lvl[i];
   __syncthreads();
 }
 
-// td of subset S (bit v = vertex v) from the finished tables.
-__device__ __forceinline__ uint32_t Lookup(const DPGraph* __restrict__ g,
-                                           const uint8_t* __restrict__ arena,
-                                           const uint32_t* s_cb, const uint32_t* s_cbase,
-                                           uint32_t S) {
+// Gray code of td(S) mod 4 (bit v of S = vertex v) from the finished tables.
+__device__ __forceinline__ uint32_t LookupCode(const DPGraph* __restrict__ g,
+                                               const uint8_t* __restrict__ arena,
+                                               const uint32_t* s_cb, const uint32_t* s_base,
+                                               uint32_t S) {
   const uint32_t lb = g->lb;
-  const int cb = static_cast<int>(g->cb);
-  const uint32_t L = S & ((1u << lb) - 1u);
-  const uint32_t H = S >> lb;
-  const int h = __builtin_popcount(H);
-  uint32_t r = cb > 0 ? s_cbase[16 * h + (H & ((1u << cb) - 1u))] : 0u;
-  uint32_t Hr = H >> cb;
-  for (int i = 1; Hr; ++i) {
-    r += s_cb[__builtin_ctz(Hr) * kCbStride + i];
-    Hr &= Hr - 1;
+  uint32_t H = S >> lb;
+  uint32_t tile = s_base[__builtin_popcount(H)];
+  for (int i = 1; H; ++i) {
+    tile += s_cb[__builtin_ctz(H) * kCbStride + i];
+    H &= H - 1;
   }
-  const size_t tile = static_cast<size_t>(s_cbase[kCbaseWords + h]) + r;
-  if (g->pk) {
-    // nibble of L: byte 4 (L >> 3) + (L & 3) of the tile, high nibble when
-    // L & 4; plus the tile's base byte
-    const size_t tiles = g->lvl[g->nh + 1];
-    const uint32_t nb = arena[g->table + (tile << (lb - 1)) + 4 * (L >> 3) + (L & 3)];
-    const uint32_t b = arena[g->table + (tiles << (lb - 1)) + tile];
-    return (((nb >> (L & 4)) & 15u) + b) >> 1;
+  const size_t ps = static_cast<size_t>(s_base[g->nh + 1]) << (lb - 3);
+  const uint8_t* p = arena + g->table + (static_cast<size_t>(tile) << (lb - 3)) +
+                     4 * ((S >> 5) & ((1u << (lb - 5)) - 1u));
+  const uint32_t g0 = *reinterpret_cast<const uint32_t*>(p);
+  const uint32_t g1 = *reinterpret_cast<const uint32_t*>(p + ps);
+  return ((g0 >> (S & 31u)) & 1u) | (((g1 >> (S & 31u)) & 1u) << 1);
+}
+
+// td mod 4 of a Gray code
+__device__ __forceinline__ uint32_t GrayValue(uint32_t code) { return code ^ (code >> 1); }
+
+// td(S): three more vertices raise td by 0..3, which the codes mod 4 tell, so
+// S is put together three vertices at a time, lowest first: one pass over its
+// vertices keeps the rank, the reads do not wait for each other, and the sets
+// of the lowest vertices are few and stay in the caches.
+__device__ __forceinline__ uint32_t LookupTd(const DPGraph* __restrict__ g,
+                                             const uint8_t* __restrict__ arena,
+                                             const uint32_t* s_cb, const uint32_t* s_base,
+                                             uint32_t S) {
+  const int lb = static_cast<int>(g->lb);
+  const size_t ps = static_cast<size_t>(s_base[g->nh + 1]) << (lb - 3);
+  const uint8_t* base = arena + g->table;
+  const uint32_t words = (1u << (lb - 5)) - 1u;
+  uint32_t td = 0, last = 0, T = 0, r = 0;
+  int h = 0, since = 0;
+  while (S) {
+    const int v = __builtin_ctz(S);
+    S &= S - 1;
+    T |= 1u << v;
+    if (v >= lb) r += s_cb[(v - lb) * kCbStride + ++h];
+    if (++since == 3 || !S) {
+      since = 0;
+      const uint32_t tile = s_base[h] + r;
+      const uint8_t* p = base + (static_cast<size_t>(tile) << (lb - 3)) + 4 * ((T >> 5) & words);
+      const uint32_t g0 = *reinterpret_cast<const uint32_t*>(p);
+      const uint32_t g1 = *reinterpret_cast<const uint32_t*>(p + ps);
+      const uint32_t now =
+          GrayValue(((g0 >> (T & 31u)) & 1u) | (((g1 >> (T & 31u)) & 1u) << 1));
+      td += (now - last) & 3u;
+      last = now;
+    }
   }
-  return static_cast<uint32_t>(arena[g->table + (tile << lb) + L]) >> 1;
+  return td;
 }
 
 __device__ __forceinline__ uint32_t WaveMax(uint32_t v) {
@@ -860,18 +538,19 @@ __global__ __launch_bounds__(64) void DPWalkKernel(
     const int32_t* __restrict__ nsteps, int32_t* __restrict__ orders,
     int order_stride) {
   __shared__ uint32_t s_cb[32 * kCbStride];
-  __shared__ uint32_t s_cbase[kLookupWords];
+  __shared__ uint32_t s_base[kLookupWords];
   const DPGraph* g = gs + blockIdx.x;
-  LoadLookupTables(g, g_cb, s_cb, s_cbase);
+  LoadLookupTables(g, g_cb, s_cb, s_base);
   const int lane = threadIdx.x;
   const uint32_t myadj = lane < 32 ? g->adj[lane] : 0u;
   uint32_t S = start[blockIdx.x];
   const int steps = nsteps[blockIdx.x];
   int32_t* out = orders + static_cast<size_t>(blockIdx.x) * order_stride;
   for (int step = 0; step < steps && S != 0u; ++step) {
-    // component of every vertex of S, by ballot BFS from each lowest vertex
-    const bool in = lane < 32 && ((S >> lane) & 1u);
-    uint32_t rest = S, mine = 0u;
+    // component of every vertex of S, by ballot BFS from each lowest vertex,
+    // and its td: lane i reads the code of the component's vertices 0..i, and
+    // td is the number of places where that code changes
+    uint32_t rest = S, C = 0u, T = 0u;
     while (rest) {
       uint32_t comp = rest & (0u - rest), front = comp;
       for (;;) {
@@ -881,18 +560,24 @@ __global__ __launch_bounds__(64) void DPWalkKernel(
         comp |= nb;
         front = nb;
       }
-      if ((comp >> lane) & 1u) mine = comp;
+      const uint32_t upto = lane < 31 ? (2u << lane) - 1u : ~0u;
+      const uint32_t code =
+          lane < 32 ? LookupCode(g, arena, s_cb, s_base, comp & upto) : 0u;
+      const uint32_t below = __shfl_up(code, 1);
+      const uint32_t td = static_cast<uint32_t>(
+          __popcll(__ballot(lane < 32 && code != (lane ? below : 0u))));
+      if (td > T) {
+        T = td;
+        C = comp;
+      }
       rest &= ~comp;
     }
-    // one round of lookups: td of v's component and of that component minus v
-    const uint32_t tdc = in ? Lookup(g, arena, s_cb, s_cbase, mine) : 0u;
-    const uint32_t tv = in ? Lookup(g, arena, s_cb, s_cbase, mine & ~(1u << lane)) : 0xFFu;
-    const uint32_t T = WaveMax(tdc);
-    // the first component (lowest vertex order) of largest td holds the
-    // lowest vertex whose component has td T
-    const unsigned long long cb = __ballot(in && tdc == T);
-    const uint32_t C = __shfl(mine, __ffsll(static_cast<long long>(cb)) - 1);
-    const unsigned long long rb = __ballot(in && ((C >> lane) & 1u) && tv + 1u == T);
+    // the root: the lowest v of the first component C of largest td whose
+    // removal lowers td, that is, changes the code
+    const bool inC = lane < 32 && ((C >> lane) & 1u);
+    const uint32_t cc = inC ? LookupCode(g, arena, s_cb, s_base, C) : 0u;
+    const uint32_t cv = inC ? LookupCode(g, arena, s_cb, s_base, C & ~(1u << lane)) : 0u;
+    const unsigned long long rb = __ballot(inC && cv != cc);
     const int root = __ffsll(static_cast<long long>(rb)) - 1;
     if (lane == 0) out[step] = root;
     S &= ~(1u << root);
@@ -911,9 +596,9 @@ __global__ __launch_bounds__(64) void DPTreeKernel(
     const uint8_t* __restrict__ arena, const uint32_t* __restrict__ start,
     int8_t* __restrict__ parent_out, int32_t* __restrict__ td_out) {
   __shared__ uint32_t s_cb[32 * kCbStride];
-  __shared__ uint32_t s_cbase[kLookupWords];
+  __shared__ uint32_t s_base[kLookupWords];
   const DPGraph* g = gs + blockIdx.x;
-  LoadLookupTables(g, g_cb, s_cb, s_cbase);
+  LoadLookupTables(g, g_cb, s_cb, s_base);
   const int lane = threadIdx.x;
   const uint32_t myadj = lane < 32 ? g->adj[lane] : 0u;
   uint32_t S = start[blockIdx.x];
@@ -934,9 +619,10 @@ __global__ __launch_bounds__(64) void DPTreeKernel(
       if ((comp >> lane) & 1u) mine = comp;
       rest &= ~comp;
     }
-    const uint32_t tdc = in ? Lookup(g, arena, s_cb, s_cbase, mine) : 0u;
-    const uint32_t tv = in ? Lookup(g, arena, s_cb, s_cbase, mine & ~(1u << lane)) : 0xFFu;
-    const uint32_t cand = static_cast<uint32_t>(__ballot(in && tv + 1u == tdc));
+    // td(C \ v) is td(C) or td(C) - 1: the codes mod 4 tell which
+    const uint32_t cc = in ? LookupCode(g, arena, s_cb, s_base, mine) : 0u;
+    const uint32_t cv = in ? LookupCode(g, arena, s_cb, s_base, mine & ~(1u << lane)) : 0u;
+    const uint32_t cand = static_cast<uint32_t>(__ballot(in && cv != cc));
     // a connected set always has a vertex with td(C \ v) = td(C) - 1; the
     // lowest vertex stands in only so that a damaged table cannot stall
     const uint32_t rc = cand & mine;
@@ -956,19 +642,20 @@ __global__ __launch_bounds__(64) void DPTreeKernel(
   if (lane == 0) td_out[blockIdx.x] = static_cast<int32_t>(d);
 }
 
-// Level-k table in colex order over n vertices (td values).
+// Level-k table in colex order over n vertices (td values): the `count`
+// subsets from code `first` on.
 __global__ __launch_bounds__(256) void DPExportLevelKernel(
     const DPGraph* __restrict__ g, const uint32_t* __restrict__ g_cb,
-    const uint8_t* __restrict__ arena, int k, uint32_t count,
+    const uint8_t* __restrict__ arena, int k, uint32_t first, uint32_t count,
     uint8_t* __restrict__ out) {
   __shared__ uint32_t s_cb[32 * kCbStride];
-  __shared__ uint32_t s_cbase[kLookupWords];
-  LoadLookupTables(g, g_cb, s_cb, s_cbase);
+  __shared__ uint32_t s_base[kLookupWords];
+  LoadLookupTables(g, g_cb, s_cb, s_base);
   const int n = static_cast<int>(g->n);
   for (uint32_t r = blockIdx.x * blockDim.x + threadIdx.x; r < count;
        r += gridDim.x * blockDim.x) {
-    const uint32_t S = Unrank(r, k, n, s_cb);
-    out[r] = static_cast<uint8_t>(Lookup(g, arena, s_cb, s_cbase, S));
+    const uint32_t S = Unrank(first + r, k, n, s_cb);
+    out[r] = static_cast<uint8_t>(LookupTd(g, arena, s_cb, s_base, S));
   }
 }
 
@@ -978,46 +665,35 @@ __global__ __launch_bounds__(256) void DPExportLevelKernel(
 constexpr int kMaxDPN = 32;
 constexpr int kMaxBatchN = 26;
 
-// Masks over the low parts L of a tile (tile-mask bit order: bit
-// 8 (L & 3) + (L >> 2)) that depend only on lb: all L, the L meeting a low
-// set T, and the L without low vertex y.
+// Masks over the 32 low parts L of a word: the L meeting a low set T, and
+// the L without low vertex y.
 struct LowMasks {
-  uint32_t all = 0, meet[32] = {}, without[5] = {};
-};
-const LowMasks& LowMasksFor(int lb) {
-  static const auto tables = [] {
-    std::vector<LowMasks> t(6);
-    for (int b = 0; b <= 5; ++b) {
-      LowMasks& M = t[b];
-      const int NB = 1 << b;
-      auto bit = [](int L) { return 1u << (8 * (L & 3) + (L >> 2)); };
-      for (int L = 0; L < NB; ++L) M.all |= bit(L);
-      for (int T = 1; T < NB; ++T)
-        for (int L = 0; L < NB; ++L)
-          if (L & T) M.meet[T] |= bit(L);
-      for (int y = 0; y < b; ++y)
-        for (int L = 0; L < NB; ++L)
-          if (!(L >> y & 1)) M.without[y] |= bit(L);
+  uint32_t meet[32] = {}, without[5] = {};
+  LowMasks() {
+    for (uint32_t L = 0; L < 32; ++L) {
+      for (uint32_t T = 0; T < 32; ++T)
+        if (L & T) meet[T] |= 1u << L;
+      for (int y = 0; y < 5; ++y)
+        if (!(L >> y & 1u)) without[y] |= 1u << L;
     }
-    return t;
-  }();
-  return tables[lb];
-}
+  }
+};
 
-// Tile offsets of each high level, each level padded to a 256-byte boundary
-// so no cache line holds tiles of two levels.
-DPGraph MakeGraph(int n, const uint64_t* adj, int lb, uint64_t table_off, int cb = 0,
-                  bool tables = true, bool packed = false) {
+// Words per tile (as a power of two) of the parameter dp.low_bits.
+int WordBits(int low_bits) { return low_bits >= 5 ? 2 : low_bits == 4 ? 1 : 0; }
+
+// Tile offsets of each high level, each level padded to a 128-byte boundary
+// of its plane so no cache line holds tiles of two levels.  Vertices n and
+// up, where a tile has more than n, count as isolated.
+DPGraph MakeGraph(int n, const uint64_t* adj, int wb, uint64_t table_off, bool tables = true) {
   DPGraph G;
   std::memset(&G, 0, sizeof(G));
+  const int lb = 5 + wb;
   G.n = n;
   G.lb = lb;
   G.nh = n > lb ? n - lb : 0;
-  G.cb = static_cast<uint32_t>(cb);
-  G.pk = packed ? 1u : 0u;
   G.table = table_off;
-  // packed tiles are 2^(lb-1) bytes; their base bytes follow all levels
-  const uint32_t pad_tiles = std::max(1u, 256u >> (packed ? lb - 1 : lb));
+  const uint32_t pad_tiles = 128u >> (lb - 3);
   uint64_t off = 0;
   for (uint32_t h = 0; h <= G.nh; ++h) {
     G.lvl[h] = static_cast<uint32_t>(off);
@@ -1026,47 +702,40 @@ DPGraph MakeGraph(int n, const uint64_t* adj, int lb, uint64_t table_off, int cb
   }
   G.lvl[G.nh + 1] = static_cast<uint32_t>(off);
   for (int v = 0; v < n; ++v) G.adj[v] = static_cast<uint32_t>(adj[v]);
-  for (int L = 0; L < (1 << lb); ++L) {
-    uint32_t m = 0;
-    for (int l = 0; l < lb && l < n; ++l)
-      if (L >> l & 1) m |= G.adj[l];
-    G.nl[L] = m;
-  }
   if (!tables) return G;  // the persistent kernel builds them in LDS
-  // N(chunk) = N(chunk without its lowest bit) | N(lowest bit)
+  // N(chunk) = N(chunk without its lowest bit) | N(lowest bit), and the low
+  // parts that give every vertex of the chunk a neighbour
+  static const LowMasks M;
   for (int c = 0; c < 4; ++c) {
     G.nbh[128 * c] = 0;
+    G.isoh[128 * c] = ~0u;
     for (int chunk = 1; chunk < 128; ++chunk) {
-      const int b = __builtin_ctz(static_cast<unsigned>(chunk));
-      const int x = 7 * c + b;
-      const uint32_t row = x < static_cast<int>(G.nh) ? G.adj[lb + x] : 0u;
+      const int x = 5 + 7 * c + __builtin_ctz(static_cast<unsigned>(chunk));
+      const uint32_t row = x < n ? G.adj[x] : 0u;
       G.nbh[128 * c + chunk] = G.nbh[128 * c + (chunk & (chunk - 1))] | row;
-    }
-  }
-  // isolation masks over the low parts L (tile-mask bit order), each built
-  // from the one with its lowest element removed
-  const LowMasks& M = LowMasksFor(lb);
-  const uint32_t lowmask = (1u << lb) - 1u;
-  for (int c = 0; c < 4; ++c) {
-    G.isoh[128 * c] = M.all;
-    for (int chunk = 1; chunk < 128; ++chunk) {
-      const int x = 7 * c + __builtin_ctz(static_cast<unsigned>(chunk));
-      const uint32_t low = x < static_cast<int>(G.nh) ? G.adj[lb + x] & lowmask : 0u;
-      G.isoh[128 * c + chunk] = G.isoh[128 * c + (chunk & (chunk - 1))] & M.meet[low];
+      G.isoh[128 * c + chunk] = G.isoh[128 * c + (chunk & (chunk - 1))] & M.meet[row & 31u];
     }
   }
   // L is fine for low vertex y iff y is not in L or L meets N(y)
-  G.isol[0] = M.all;
-  for (int Y = 1; Y < (1 << lb); ++Y) {
+  G.isol[0] = ~0u;
+  for (int Y = 1; Y < 32; ++Y) {
     const int y = __builtin_ctz(static_cast<unsigned>(Y));
-    G.isol[Y] = G.isol[Y & (Y - 1)] & (M.without[y] | M.meet[G.adj[y] & lowmask]);
+    G.isol[Y] = G.isol[Y & (Y - 1)] & (M.without[y] | M.meet[G.adj[y] & 31u]);
   }
   return G;
 }
 
+// Bytes of a graph's three planes.
 uint64_t TableBytes(const DPGraph& G) {
-  const uint64_t tiles = G.lvl[G.nh + 1];
-  return G.pk ? (tiles << (G.lb - 1)) + (tiles + 255) / 256 * 256 : tiles << G.lb;
+  return 3 * (static_cast<uint64_t>(G.lvl[G.nh + 1]) << (G.lb - 3));
+}
+
+// Bytes that a graph's table takes from the context's budget: one per subset,
+// though only 3/8 are used, or (dp.packed with dp.class_bits) 17/32, so that a
+// byte budget admits and refuses the same calls as with byte tables.
+uint64_t ClaimedBytes(const DPGraph& G, bool packed = false) {
+  const uint64_t subsets = 1ull << G.n;
+  return std::max(TableBytes(G), packed ? subsets / 2 + subsets / 32 : subsets);
 }
 
 // binomials, O_k, the 16-bit unrank table (2 entries per word), then the
@@ -1103,68 +772,9 @@ int GridFor(td_ctx* ctx, uint64_t lanes_needed, int block) {
   const uint64_t blocks = (lanes_needed + block - 1) / block;
   const uint64_t cap = static_cast<uint64_t>(ctx->prop.multiProcessorCount) *
                        (2048 / block) * static_cast<uint64_t>(ctx->dp.grid_mult);
-  return static_cast<int>(std::max<uint64_t>(1, std::min(blocks, cap)));
-}
-
-// Balanced static schedule of level h (see DPClassLevelKernel).
-ClassSched MakeClassSched(const DPGraph& G, int h) {
-  const int cb = static_cast<int>(G.cb);
-  const int P = 1 << cb;
-  const int rest = static_cast<int>(G.nh) - cb;
-  auto C = [](int x, int j) { return Binom(x, j); };
-  std::vector<uint64_t> size(P), taken(P, 0);
-  uint64_t total = 0;
-  for (int q = 0; q < P; ++q) {
-    const int k = h - __builtin_popcount(static_cast<unsigned>(q));
-    size[q] = (k < 0 || k > rest) ? 0 : Binom(rest, k);
-    total += size[q];
-  }
-  const uint64_t target = (total + kXcds - 1) / kXcds;
-  ClassSched S;
-  std::memset(&S, 0, sizeof(S));
-  std::vector<uint64_t> load(kXcds, 0);
-  auto add = [&](int x, int q, uint64_t first, uint64_t end) {
-    TD_REQUIRE(S.nseg[x] < static_cast<uint32_t>(kMaxSeg), TD_E_INVALID,
-               "class schedule needs too many segments");
-    ClassSeg& s = S.seg[x][S.nseg[x]++];
-    s.p = static_cast<uint32_t>(q);
-    s.first = static_cast<uint32_t>(first);
-    s.end = static_cast<uint32_t>(end);
-    s.prev = h > 0 ? G.lvl[h - 1] + ClassBase(h - 1, s.p, rest, C) : 0u;
-    s.cur = G.lvl[h] + ClassBase(h, s.p, rest, C);
-    uint32_t m = s.p;
-    for (int c = 0; c < 4; ++c) {
-      s.x[c] = 0;
-      if (m) {
-        const uint32_t b = m & (0u - m);
-        m ^= b;
-        s.x[c] = G.lvl[h - 1] + ClassBase(h - 1, s.p ^ b, rest, C);
-      }
-    }
-    load[x] += end - first;
-  };
-  // own classes first, from the start of each class, up to the target
-  for (int q = 0; q < P; ++q) {
-    const int x = (P == 16 && q >= 8) ? 15 - q : q % static_cast<int>(kXcds);
-    const uint64_t take = std::min(size[q] - taken[q], target - std::min(target, load[x]));
-    if (take > 0) {
-      add(x, q, taken[q], taken[q] + take);
-      taken[q] += take;
-    }
-  }
-  // the rest of every class to the XCDs below the target
-  for (int q = 0; q < P; ++q) {
-    while (taken[q] < size[q]) {
-      int x = 0;
-      for (int y = 1; y < static_cast<int>(kXcds); ++y)
-        if (load[y] < load[x]) x = y;
-      const uint64_t room = load[x] < target ? target - load[x] : size[q] - taken[q];
-      const uint64_t take = std::min(size[q] - taken[q], room);
-      add(x, q, taken[q], taken[q] + take);
-      taken[q] += take;
-    }
-  }
-  return S;
+  // the same number of passes for every workgroup
+  const uint64_t passes = std::max<uint64_t>(1, (blocks + cap - 1) / cap);
+  return static_cast<int>(std::max<uint64_t>(1, (blocks + passes - 1) / passes));
 }
 
 // Runs of small levels at either end of a graph's level sequence go to one
@@ -1197,10 +807,6 @@ uint64_t PartLaunches(const DPGraph& G, int part, int K) {
   const int nh = static_cast<int>(G.nh);
   auto want = [&](int h0) { return part < 0 || PartOf(G, h0, K) == part; };
   uint64_t c = 0;
-  if (G.cb > 0) {
-    for (int h = 0; h <= nh; ++h) c += want(h) ? 1 : 0;
-    return c;
-  }
   int lo, hi;
   SmallLevelRuns(nh, &lo, &hi);
   if (lo >= 0 && want(0)) ++c;
@@ -1214,40 +820,17 @@ uint64_t LevelKernelCount(const DPGraph& G) { return PartLaunches(G, -1, 1); }
 
 // The level launches of one graph on stream `st`: all of them (part = -1),
 // or the launches whose first level lies in part `part` of K (PartOf).
-template <int LB>
+template <int WB>
 void LaunchLevels(td_ctx* ctx, const DPGraph& G, const DPGraph* dG,
                   const uint32_t* cb, uint8_t* arena, uint64_t* launches,
                   hipStream_t st, int part, int K) {
   const int R = ctx->dp.tiles_per_lane, block = ctx->dp.block;
   auto want = [&](int h0) { return part < 0 || PartOf(G, h0, K) == part; };
-  if (G.cb > 0) {
-    for (int h = 0; h <= static_cast<int>(G.nh); ++h) {
-      if (!want(h)) continue;
-      const ClassSched sched = MakeClassSched(G, h);
-      const uint64_t ntiles = Binom(G.nh, h);
-      int grid = GridFor(ctx, (ntiles + R - 1) / R, block);
-      grid = std::max(static_cast<int>(kXcds), (grid + 7) / 8 * 8);
-      if constexpr (LB >= 4) {
-        if (G.pk)
-          hipLaunchKernelGGL((DPClassLevelKernel<LB, true>), dim3(grid), dim3(block), 0,
-                             st, dG, cb, arena, h, R, sched);
-        else
-          hipLaunchKernelGGL((DPClassLevelKernel<LB, false>), dim3(grid), dim3(block), 0,
-                             st, dG, cb, arena, h, R, sched);
-      } else {
-        hipLaunchKernelGGL((DPClassLevelKernel<LB, false>), dim3(grid), dim3(block), 0,
-                           st, dG, cb, arena, h, R, sched);
-      }
-      ++*launches;
-    }
-    TD_HIP(hipGetLastError());
-    return;
-  }
   const int nh = static_cast<int>(G.nh);
   int lo, hi;
   SmallLevelRuns(nh, &lo, &hi);
   if (lo >= 0 && want(0)) {
-    hipLaunchKernelGGL(DPSmallLevelsKernel<LB>, dim3(1), dim3(1024), 0, st, dG, cb,
+    hipLaunchKernelGGL(DPSmallLevelsKernel<WB>, dim3(1), dim3(1024), 0, st, dG, cb,
                        arena, 0, lo);
     ++*launches;
   }
@@ -1255,13 +838,13 @@ void LaunchLevels(td_ctx* ctx, const DPGraph& G, const DPGraph* dG,
     if (!want(h)) continue;
     const uint32_t ntiles = static_cast<uint32_t>(Binom(G.nh, h));
     int grid = GridFor(ctx, (ntiles + R - 1) / R, block);
-    if (ctx->dp.xcd_remap && grid >= 64) grid = (grid + 7) / 8 * 8;
-    hipLaunchKernelGGL(DPLevelKernel<LB>, dim3(grid), dim3(block), 0,
-                       st, dG, cb, arena, h, ntiles, R, ctx->dp.xcd_remap);
+    if (grid >= 64) grid = (grid + 7) / 8 * 8;  // slices, see DPLevelKernel
+    hipLaunchKernelGGL(DPLevelKernel<WB>, dim3(grid), dim3(block), 0,
+                       st, dG, cb, arena, h, ntiles, R);
     ++*launches;
   }
   if (hi <= nh && want(hi)) {
-    hipLaunchKernelGGL(DPSmallLevelsKernel<LB>, dim3(1), dim3(1024), 0, st, dG, cb,
+    hipLaunchKernelGGL(DPSmallLevelsKernel<WB>, dim3(1), dim3(1024), 0, st, dG, cb,
                        arena, hi, nh);
     ++*launches;
   }
@@ -1279,11 +862,9 @@ void LaunchLevelsLB(td_ctx* ctx, const DPGraph& G, const DPGraph* dG,
                     const uint32_t* cb, uint8_t* arena, uint64_t* launches,
                     hipStream_t st, int part, int K) {
   switch (G.lb) {
-    case 2: LaunchLevels<2>(ctx, G, dG, cb, arena, launches, st, part, K); break;
-    case 3: LaunchLevels<3>(ctx, G, dG, cb, arena, launches, st, part, K); break;
-    case 4: LaunchLevels<4>(ctx, G, dG, cb, arena, launches, st, part, K); break;
-    case 5: LaunchLevels<5>(ctx, G, dG, cb, arena, launches, st, part, K); break;
-    default: throw Error{TD_E_INVALID, "low_bits must be in [2, 5]"};
+    case 5: LaunchLevels<0>(ctx, G, dG, cb, arena, launches, st, part, K); break;
+    case 6: LaunchLevels<1>(ctx, G, dG, cb, arena, launches, st, part, K); break;
+    default: LaunchLevels<2>(ctx, G, dG, cb, arena, launches, st, part, K); break;
   }
 }
 
@@ -1301,8 +882,7 @@ void RunLevels(td_ctx* ctx, const DPGraph& G, const DPGraph* dG,
     return;
   }
   // key includes the buffer addresses baked into the captured launches
-  td_ctx::GraphKey key{static_cast<int>(G.n) | static_cast<int>(G.cb << 8) | (slot << 16) |
-                           static_cast<int>(G.pk << 20) | ((part + 1) << 24) | (K << 28),
+  td_ctx::GraphKey key{static_cast<int>(G.n) | (slot << 16) | ((part + 1) << 24) | (K << 28),
                        static_cast<int>(G.lb), ctx->dp.tiles_per_lane, ctx->dp.block};
   auto& p = ctx->dp_graph_ptrs[key];
   auto it = ctx->dp_graphs.find(key);
@@ -1357,17 +937,20 @@ float Elapsed(hipEvent_t a, hipEvent_t b) {
   return ms;
 }
 
-// Record of one graph for the single-graph level kernels: the context's low
-// bits (more where the N(H) chunk tables, which cover 28 high vertices, need
-// it) and its class layout where the graph is large enough.
+// Record of one graph for the single-graph level kernels.  Larger tiles cost
+// fewer instructions and bytes per subset, but leave fewer lanes: tiles take
+// the context's words only as far as 22 high vertices remain (705,432 tiles in
+// the middle level).  Level kernels of one graph with 1 / 2 / 4 words, us:
+// n = 23: 92 / 97 / 108; n = 27: 168 / 170 / 180; n = 28: 236 / 227 / 233;
+// n = 29: 366 / 341 / 331; n = 30: 635 / 560 / 527.
 DPGraph SingleGraph(td_ctx* ctx, int n, const uint64_t* adj, bool tables = true) {
-  const int lb = std::max(ctx->dp.low_bits, n - 28);
-  const int nh = n > lb ? n - lb : 0;
-  const int cbits = (ctx->dp.class_bits > 0 && nh >= ctx->dp.class_min_nh &&
-                     nh > ctx->dp.class_bits)
-                        ? ctx->dp.class_bits
-                        : 0;
-  return MakeGraph(n, adj, lb, 0, cbits, tables, ctx->dp.packed && cbits > 0 && lb >= 4);
+  return MakeGraph(n, adj, std::min(WordBits(ctx->dp.low_bits), std::max(0, n - 27)), 0, tables);
+}
+
+// Whether the context claims a packed table's bytes for this graph.
+bool ClaimsPacked(const td_ctx* ctx, int n) {
+  return ctx->dp.packed && ctx->dp.class_bits > 0 && ctx->dp.low_bits >= 4 &&
+         n - ctx->dp.low_bits >= ctx->dp.class_min_nh;
 }
 
 // descriptor, walk start set and step count in one device block, uploaded
@@ -1385,7 +968,7 @@ void SolveOne(td_ctx* ctx, int n, const uint64_t* adj, uint8_t* td_out,
   // queries have no tables to read
   ctx->have_dp = false;
   DPGraph G = SingleGraph(ctx, n, adj);
-  const uint64_t tbytes = TableBytes(G);
+  const uint64_t tbytes = ClaimedBytes(G, ClaimsPacked(ctx, n));
   uint8_t* arena = static_cast<uint8_t*>(ctx->Buffer("dp.arena", tbytes));
   uint8_t* din = static_cast<uint8_t*>(ctx->Buffer("dp.graph", kInBytes));
   DPGraph* dG = reinterpret_cast<DPGraph*>(din);
@@ -1443,7 +1026,7 @@ constexpr int kNoAllocMaxN = 24;
 constexpr size_t kNoAllocTreeOff = 8192;
 constexpr size_t kNoAllocPascalOff = 16384;
 constexpr size_t kNoAllocArenaOff = 256 * 1024;
-// 2^n table bytes plus at most 255 bytes of padding per high level
+// at most 2^n table bytes (3/8 of them used) plus padding
 constexpr size_t kNoAllocArenaBytes = (size_t{1} << kNoAllocMaxN) + 64 * 1024;
 constexpr size_t kNoAllocScratchBytes = kNoAllocArenaOff + kNoAllocArenaBytes;
 static_assert(kInBytes <= kNoAllocTreeOff, "descriptor block overlaps the tree output");
@@ -1559,7 +1142,8 @@ void SolveLarge(td_ctx* ctx, const std::vector<int>& idx, const int32_t* ns,
   // every buffer at its final size before the first launch
   uint64_t tmax = 0;
   for (int i : idx)
-    tmax = std::max(tmax, TableBytes(SingleGraph(ctx, ns[i], adj_concat + row_off[i], false)));
+    tmax = std::max(tmax, ClaimedBytes(SingleGraph(ctx, ns[i], adj_concat + row_off[i], false),
+                                       ClaimsPacked(ctx, ns[i])));
   uint8_t *arena[kSlots], *din[kSlots], *dtree[kSlots];
   for (int s = 0; s < S; ++s) {
     const std::string sfx = s ? std::to_string(s) : std::string();
@@ -1657,7 +1241,7 @@ void SolveLarge(td_ctx* ctx, const std::vector<int>& idx, const int32_t* ns,
   *level_ms += total;
 }
 
-template <int LB>
+template <int WB>
 void LaunchBatch(td_ctx* ctx, int mode, int ngraphs,
                  const DPGraph* Gs, const DPGraph* dGs,
                  const uint32_t* cb, uint8_t* arena, uint32_t* dqueue,
@@ -1670,14 +1254,14 @@ void LaunchBatch(td_ctx* ctx, int mode, int ngraphs,
     const int bblock = ctx->dp.batch_block;
     auto launch = [&] {
       hipLaunchKernelGGL(ResetCounter, dim3(1), dim3(64), 0, ctx->stream, dqueue);
-      hipLaunchKernelGGL(DPPersistentKernel<LB>, dim3(grid), dim3(bblock), 0,
+      hipLaunchKernelGGL(DPPersistentKernel<WB>, dim3(grid), dim3(bblock), 0,
                          ctx->stream, dGs, cb, arena, ngraphs, dqueue, R);
     };
     if (!ctx->dp.use_graph) {
       launch();
       *launches += 2;
     } else {
-      const td_ctx::GraphKey key{-ngraphs, LB, R, bblock * 64 + ctx->dp.batch_wg_per_cu};
+      const td_ctx::GraphKey key{-ngraphs, WB, R, bblock * 64 + ctx->dp.batch_wg_per_cu};
       const void* sig[3] = {arena, dGs, dqueue};
       auto it = ctx->dp_graphs.find(key);
       auto& p = ctx->dp_graph_ptrs[key];
@@ -1727,7 +1311,7 @@ void LaunchBatch(td_ctx* ctx, int mode, int ngraphs,
     for (int h = 0; h <= maxnh; ++h) {
       const size_t cnt = per_level[h].size();
       if (cnt) {
-        hipLaunchKernelGGL(DPChunkKernel<LB>, dim3(cnt), dim3(block), 0,
+        hipLaunchKernelGGL(DPChunkKernel<WB>, dim3(cnt), dim3(block), 0,
                            ctx->stream, dGs, cb, arena, dch + off, h, R);
         ++*launches;
       }
@@ -1738,8 +1322,8 @@ void LaunchBatch(td_ctx* ctx, int mode, int ngraphs,
       for (int h = 0; h <= static_cast<int>(Gs[i].nh); ++h) {
         const uint32_t ntiles = static_cast<uint32_t>(Binom(Gs[i].nh, h));
         const int grid = GridFor(ctx, (ntiles + R - 1) / R, block);
-        hipLaunchKernelGGL(DPLevelKernel<LB>, dim3(grid), dim3(block), 0,
-                           ctx->stream, dGs + i, cb, arena, h, ntiles, R, 0);
+        hipLaunchKernelGGL(DPLevelKernel<WB>, dim3(grid), dim3(block), 0,
+                           ctx->stream, dGs + i, cb, arena, h, ntiles, R);
         ++*launches;
       }
   }
@@ -1796,7 +1380,7 @@ void SolveBatch(td_ctx* ctx, int ngraphs, const int32_t* ns,
       }
       for (int j = t; j < nsmall; j += T) {
         const int i = perm[j];
-        Gs[j] = MakeGraph(ns[i], adj_concat + row_off[i], lb, 0, 0, mode != 0);
+        Gs[j] = MakeGraph(ns[i], adj_concat + row_off[i], WordBits(lb), 0, mode != 0);
       }
     };
     if (ngraphs < 256) {
@@ -1839,12 +1423,13 @@ void SolveBatch(td_ctx* ctx, int ngraphs, const int32_t* ns,
     return;
   }
   ngraphs = nsmall;
-  uint64_t off = 0;
+  uint64_t off = 0, claimed = 0;
   for (int j = 0; j < ngraphs; ++j) {
     Gs[j].table = off;
     off += (TableBytes(Gs[j]) + 255) / 256 * 256;
+    claimed += (ClaimedBytes(Gs[j]) + 255) / 256 * 256;
   }
-  uint8_t* arena = static_cast<uint8_t*>(ctx->Buffer("dp.batch_arena", off));
+  uint8_t* arena = static_cast<uint8_t*>(ctx->Buffer("dp.batch_arena", claimed));
   DPGraph* dGs = static_cast<DPGraph*>(
       ctx->Buffer("dp.batch_graphs", sizeof(DPGraph) * ngraphs));
   const uint32_t* cb = PascalDevice(ctx);
@@ -1868,12 +1453,10 @@ void SolveBatch(td_ctx* ctx, int ngraphs, const int32_t* ns,
   TD_HIP(hipMemcpyAsync(dstart, start, 4 * ngraphs, hipMemcpyHostToDevice, ctx->stream));
   uint64_t small_launches = 0;
   TD_HIP(hipEventRecord(ctx->ev[0], ctx->stream));
-  switch (lb) {
-    case 2: LaunchBatch<2>(ctx, mode, ngraphs, Gs, dGs, cb, arena, dq, &small_launches); break;
-    case 3: LaunchBatch<3>(ctx, mode, ngraphs, Gs, dGs, cb, arena, dq, &small_launches); break;
-    case 4: LaunchBatch<4>(ctx, mode, ngraphs, Gs, dGs, cb, arena, dq, &small_launches); break;
-    case 5: LaunchBatch<5>(ctx, mode, ngraphs, Gs, dGs, cb, arena, dq, &small_launches); break;
-    default: throw Error{TD_E_INVALID, "low_bits must be in [2, 5]"};
+  switch (WordBits(lb)) {
+    case 0: LaunchBatch<0>(ctx, mode, ngraphs, Gs, dGs, cb, arena, dq, &small_launches); break;
+    case 1: LaunchBatch<1>(ctx, mode, ngraphs, Gs, dGs, cb, arena, dq, &small_launches); break;
+    default: LaunchBatch<2>(ctx, mode, ngraphs, Gs, dGs, cb, arena, dq, &small_launches); break;
   }
   TD_HIP(hipEventRecord(ctx->ev[1], ctx->stream));
   // mode 0: the persistent kernel (its queue reset aside); else the launches
@@ -2059,29 +1642,17 @@ int td_dp_get_treedepth(td_ctx* ctx, int32_t k, uint64_t code,
     const int n = ctx->last_n;
     TD_REQUIRE(k >= 0 && k <= n && code < Binom(n, k), TD_E_STATE,
                "subset code out of range");
-    const uint64_t S = UnrankColex(n, k, code);
-    const DPGraph& G = ctx->last_graph;
-    const uint64_t L = S & ((1ull << G.lb) - 1);
-    const uint64_t H = S >> G.lb;
-    const int h = __builtin_popcountll(H);
-    const uint64_t r = TileIndex(static_cast<uint32_t>(H), static_cast<int>(G.nh),
-                                 static_cast<int>(G.cb),
-                                 [](int x, int j) { return Binom(x, j); });
-    const uint64_t tile = static_cast<uint64_t>(G.lvl[h]) + r;
-    const uint8_t* arena = static_cast<const uint8_t*>(ctx->bufs["dp.arena"].p);
-    uint8_t raw = 0;
-    if (G.pk) {
-      // nibble of L plus the tile's base byte (DPTile's packed format)
-      uint8_t nb = 0, b = 0;
-      const uint64_t tiles = G.lvl[G.nh + 1];
-      TD_HIP(hipMemcpy(&nb, arena + (tile << (G.lb - 1)) + 4 * (L >> 3) + (L & 3), 1,
-                       hipMemcpyDeviceToHost));
-      TD_HIP(hipMemcpy(&b, arena + (tiles << (G.lb - 1)) + tile, 1, hipMemcpyDeviceToHost));
-      raw = static_cast<uint8_t>(((nb >> (L & 4)) & 15u) + b);
-    } else {
-      TD_HIP(hipMemcpy(&raw, arena + (tile << G.lb) + L, 1, hipMemcpyDeviceToHost));
-    }
-    *td_out = raw >> 1;
+    // one subset of level k, as td_dp_get_level reads them
+    uint8_t* d = static_cast<uint8_t*>(ctx->Buffer("dp.walk_order", 64 * 4));
+    hipLaunchKernelGGL(DPExportLevelKernel, dim3(1), dim3(64), 0, ctx->stream,
+                       static_cast<const DPGraph*>(ctx->bufs["dp.graph"].p), PascalDevice(ctx),
+                       static_cast<const uint8_t*>(ctx->bufs["dp.arena"].p), k,
+                       static_cast<uint32_t>(code), 1u, d);
+    TD_HIP(hipGetLastError());
+    uint8_t td = 0;
+    TD_HIP(hipMemcpyAsync(&td, d, 1, hipMemcpyDeviceToHost, ctx->stream));
+    TD_HIP(hipStreamSynchronize(ctx->stream));
+    *td_out = td;
   });
 }
 
@@ -2097,7 +1668,7 @@ int td_dp_get_level(td_ctx* ctx, int32_t k, uint8_t* out, uint64_t out_len) {
     const uint8_t* arena = static_cast<const uint8_t*>(ctx->bufs["dp.arena"].p);
     const int grid = GridFor(ctx, count, 256);
     hipLaunchKernelGGL(DPExportLevelKernel, dim3(grid), dim3(256), 0,
-                       ctx->stream, dG, PascalDevice(ctx), arena, k,
+                       ctx->stream, dG, PascalDevice(ctx), arena, k, 0u,
                        static_cast<uint32_t>(count), d);
     TD_HIP(hipGetLastError());
     TD_HIP(hipMemcpyAsync(out, d, count, hipMemcpyDeviceToHost, ctx->stream));

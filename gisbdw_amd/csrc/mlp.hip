@@ -565,28 +565,24 @@ __global__ void MLPToBf16Kernel(const float* __restrict__ w, uint16_t* __restric
 // Optimal-root labels from the last single-graph DP: for a connected vertex
 // set S (one per wave), positives = {v in S : td(S \ v) = td(S) - 1}.
 struct DPLookup {
-  const uint8_t* arena;
-  uint32_t lb, nh, cb, pk;
+  const uint8_t* table;
+  uint32_t lb, nh;
   uint32_t lvl[34];
 };
 
-// td of S from the tables: a byte 2 td + connected per subset, or (packed
-// tiles) the nibble of the low part plus the tile's base byte, which follows
-// all levels' tiles
-__device__ __forceinline__ uint32_t LookupTd(const DPLookup& L, const uint32_t* cb, uint32_t S) {
-  const uint32_t low = S & ((1u << L.lb) - 1u);
-  const uint32_t H = S >> L.lb;
-  const int h = __builtin_popcount(H);
-  const uint32_t r = TileIndex(H, static_cast<int>(L.nh), static_cast<int>(L.cb),
-                               [&](int x, int j) { return cb[x * 33 + j]; });
-  const size_t tile = static_cast<size_t>(L.lvl[h]) + r;
-  if (L.pk) {
-    const size_t tiles = L.lvl[L.nh + 1];
-    const uint32_t nb = L.arena[(tile << (L.lb - 1)) + 4 * (low >> 3) + (low & 3)];
-    const uint32_t b = L.arena[(tiles << (L.lb - 1)) + tile];
-    return (((nb >> (low & 4)) & 15u) + b) >> 1;
+// Gray code of td(S) mod 4 from the tables (two bit planes; dpword.hpp)
+__device__ __forceinline__ uint32_t LookupCode(const DPLookup& L, const uint32_t* cb, uint32_t S) {
+  uint32_t H = S >> L.lb;
+  size_t tile = L.lvl[__builtin_popcount(H)];
+  for (int i = 1; H; ++i) {
+    tile += cb[__builtin_ctz(H) * 33 + i];
+    H &= H - 1;
   }
-  return static_cast<uint32_t>(L.arena[(tile << L.lb) + low]) >> 1;
+  const size_t plane = static_cast<size_t>(L.lvl[L.nh + 1]) << (L.lb - 3);
+  const uint8_t* p = L.table + (tile << (L.lb - 3)) + 4 * ((S >> 5) & ((1u << (L.lb - 5)) - 1u));
+  const uint32_t g0 = *reinterpret_cast<const uint32_t*>(p);
+  const uint32_t g1 = *reinterpret_cast<const uint32_t*>(p + plane);
+  return ((g0 >> (S & 31u)) & 1u) | (((g1 >> (S & 31u)) & 1u) << 1);
 }
 
 __global__ __launch_bounds__(64) void LabelKernel(DPLookup L, const uint32_t* __restrict__ g_cb,
@@ -598,13 +594,19 @@ __global__ __launch_bounds__(64) void LabelKernel(DPLookup L, const uint32_t* __
   Sync();
   const uint32_t S = sets[blockIdx.x];
   const int v = threadIdx.x;
-  const uint32_t T = LookupTd(L, s_cb, S);
   const bool in = v < 32 && ((S >> v) & 1u);
-  const uint32_t tv = in ? LookupTd(L, s_cb, S & ~(1u << v)) : 0xFFu;
-  const uint64_t b = static_cast<uint64_t>(__ballot(in && tv + 1u == T));
+  // td(S \ v) is td(S) or td(S) - 1: the codes mod 4 tell which
+  const uint32_t all = LookupCode(L, s_cb, S);
+  const uint32_t one = in ? LookupCode(L, s_cb, S & ~(1u << v)) : all;
+  const uint64_t b = static_cast<uint64_t>(__ballot(in && one != all));
+  // td(S): lane i reads the code of S's vertices 0..i; td is the number of
+  // places where that code changes
+  const uint32_t code = v < 32 ? LookupCode(L, s_cb, S & (v < 31 ? (2u << v) - 1u : ~0u)) : 0u;
+  const uint32_t below = __shfl_up(code, 1);
+  const uint64_t steps = static_cast<uint64_t>(__ballot(v < 32 && code != (v ? below : 0u)));
   if (v == 0) {
     pos[blockIdx.x] = static_cast<uint32_t>(b);
-    tdout[blockIdx.x] = static_cast<uint8_t>(T);
+    tdout[blockIdx.x] = static_cast<uint8_t>(__builtin_popcountll(steps));
   }
 }
 
@@ -912,11 +914,9 @@ int td_mlp_make_samples(td_ctx* ctx, int32_t count, uint64_t seed, int32_t* n_ou
     auto* dtd = static_cast<uint8_t*>(ctx->Buffer("mlp.lab.td", static_cast<size_t>(count)));
     TD_HIP(hipMemcpyAsync(dsets, sets.data(), 4ull * count, hipMemcpyHostToDevice, ctx->stream));
     DPLookup L;
-    L.arena = static_cast<const uint8_t*>(ctx->bufs["dp.arena"].p);
+    L.table = static_cast<const uint8_t*>(ctx->bufs["dp.arena"].p) + G.table;
     L.lb = G.lb;
     L.nh = G.nh;
-    L.cb = G.cb;
-    L.pk = G.pk;
     std::memcpy(L.lvl, G.lvl, sizeof(L.lvl));
     const uint32_t* cb = static_cast<const uint32_t*>(ctx->bufs["dp.pascal"].p);
     hipLaunchKernelGGL(LabelKernel, dim3(count), dim3(64), 0, ctx->stream, L, cb, dsets, dpos,

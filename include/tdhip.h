@@ -40,19 +40,22 @@ int td_ctx_create(td_ctx** out, int device, uint64_t mem_budget_bytes);
 void td_ctx_destroy(td_ctx* ctx);
 /* Last error message of this context ("" if none). */
 const char* td_last_error(const td_ctx* ctx);
-/* Tuning knobs (see td_dp_autotune): "dp.low_bits" (2..5, default 4),
+/* Tuning knobs (see td_dp_autotune): "dp.low_bits" (2..5, default 4: level
+ * tables in tiles of 1, 1, 2 or 4 words of 32 subsets; a single graph takes
+ * fewer words where larger tiles would leave lanes idle),
  * "dp.tiles_per_lane" (1..64, default 1), "dp.block" (64..1024, default 512),
  * "dp.grid_mult" (1..64, default 4: level launches use at most this many
  * times the workgroups the device holds at once),
- * "dp.batch_wg_per_cu", "dp.use_graph" (0/1), "dp.class_bits" (0, 3 or 4,
- * default 0: level tables grouped into 2^bits vertex classes, one class per
- * XCD, for single graphs with at least "dp.class_min_nh" (default 16)
- * vertices above the low bits), "dp.packed" (0/1, default 0: class layouts
- * with low_bits >= 4 store 4 bits per subset plus one byte per tile, 0.53 of
- * the table bytes), "dp.streams" (1..3, default 2: graphs above 26
- * vertices in a td_dp_solve_batch call run their level sequences that many
- * at a time on that many streams, each graph starting when the previous one
- * has done the first 1/streams of its subsets; 1: one graph at a time),
+ * "dp.batch_wg_per_cu", "dp.use_graph" (0/1), "dp.streams" (1..3, default 2:
+ * graphs above 26 vertices in a td_dp_solve_batch call run their level
+ * sequences that many at a time on that many streams, each graph starting
+ * when the previous one has done the first 1/streams of its subsets; 1: one
+ * graph at a time).  "dp.class_bits" (0, 3 or 4, default 0),
+ * "dp.class_min_nh" (5..32, default 16), "dp.packed" (0/1, default 0) and
+ * "dp.xcd_remap" (0/1) are accepted and kept for callers and tuning caches
+ * that set them: one table layout, three bits per subset and contiguous
+ * slices per XCD, serves all of them.  A table claims one byte per subset of
+ * the byte budget, or 17/32 with class_bits and packed both set.
  * "bnb.node_budget"
  * (per graph, default 2e6), "bnb.waves_per_graph" (1..16; 0, the
  * default: 16 for batches of at most one graph per CU, 12 for up to two,
@@ -104,8 +107,7 @@ int td_dp_solve(td_ctx* ctx, int32_t n, const uint64_t* adj,
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
  * No counterpart in the reference.  Same inputs, outputs and results as
  * td_dp_solve, for n <= 24: the descriptor, Pascal tables, level tables and
- * tree output live in one fixed device array of 17,104,896 bytes (16 MiB of
- * level tables plus 256 KiB) that the library's code object holds on each
+ * tree output live in one fixed device array of 17,104,896 bytes that the library's code object holds on each
  * device it runs on until the process ends.  The call allocates no device or
  * page-locked memory and captures no graph (its level kernels launch
  * directly).  n > 24 is TD_E_INVALID.  Every call on one device shares that

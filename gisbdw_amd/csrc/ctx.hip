@@ -95,6 +95,8 @@ void* td_ctx::Buffer(const std::string& name, size_t bytes) {
     b.p = nullptr;
     b.bytes = 0;
   }
+  // DPFlowKernel's buffer is a help, not a need: it makes room
+  if (budget && allocated + bytes > budget && name != "dp.flow") Release("dp.flow");
   if (budget && allocated + bytes > budget)
     throw tdhip::Error{TD_E_NOMEM, "buffer '" + name + "' of " +
                                        std::to_string(bytes) +
@@ -192,6 +194,9 @@ int td_ctx_create(td_ctx** out, int device, uint64_t mem_budget_bytes) {
       td_ctx_destroy(c);
       return TD_E_HIP;
     }
+  int khz = 0;
+  if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device) == hipSuccess && khz > 0)
+    c->clock_khz = khz;
   try {
     tdhip::NoAllocSetup(c);
   } catch (const tdhip::Error&) {
@@ -268,6 +273,9 @@ int td_ctx_set_param(td_ctx* c, const char* key, int64_t v) {
     c->dp.grid_mult = (int)v;
   } else if (k == "dp.packed") {
     c->dp.packed = v ? 1 : 0;
+  } else if (k == "dp.flow_spin") {
+    if (v < 0 || v > (1 << 30)) return bad("must be in [0, 2^30]");
+    c->dp.flow_spin = (int)v;
   } else if (k == "dp.streams") {
     if (v < 1 || v > 3) return bad("must be 1, 2 or 3");
     c->dp.streams = (int)v;
@@ -296,6 +304,7 @@ int td_ctx_get_param(const td_ctx* c, const char* key, int64_t* v) {
   else if (k == "dp.class_min_nh") *v = c->dp.class_min_nh;
   else if (k == "dp.grid_mult") *v = c->dp.grid_mult;
   else if (k == "dp.packed") *v = c->dp.packed;
+  else if (k == "dp.flow_spin") *v = c->dp.flow_spin;
   else if (k == "dp.streams") *v = c->dp.streams;
   else {
     auto it = c->params.find(k);

@@ -45,7 +45,7 @@ struct DPGraph {
   uint32_t n;        // vertices
   uint32_t nh;       // high vertices, max(n - lb, 0)
   uint32_t lb;       // 5 + log2(words per tile): 5, 6 or 7
-  uint32_t pad0;
+  uint32_t direct;   // planes indexed by S >> 5 itself, 2^max(n-5, 0) words each
   uint64_t table;    // byte offset of this graph's tables in the arena
   uint32_t lvl[34];  // tile offset of high level h; lvl[nh+1] = 2^nh
   uint32_t adj[32];  // adjacency rows
@@ -77,6 +77,7 @@ struct DPConfig {
   int class_min_nh = 16;
   int grid_mult = 4;       // level launch: at most grid_mult x the resident workgroups
   int packed = 0;          // with class_bits and low_bits >= 4: claim 17/32 bytes a subset
+  int flow_spin = 1 << 17; // reads of one published word before DPFlowKernel gives up
   int streams = 2;         // batch calls: large graphs' level sequences in flight (1-3)
 };
 
@@ -173,6 +174,7 @@ struct td_ctx {
   uint64_t allocated = 0;
   std::string err;
   hipDeviceProp_t prop{};
+  double clock_khz = 1e5;  // rate of the device's wall clock
   tdhip::DPConfig dp;
   std::map<std::string, int64_t> params;
 
@@ -219,6 +221,10 @@ struct td_ctx {
   // state of the last td_dp_solve (for the queries)
   int last_n = 0;
   bool have_dp = false;
+  // DPFlowKernel's buffer: the words published in it carry the call's tag, and
+  // its ticket counter has seen flow_tickets workgroups (see FlowBuffer)
+  uint32_t flow_tag = 0, flow_tickets = 0;
+  bool record_up = false;  // its record is in "dp.graph" (see LastRecord)
   tdhip::DPGraph last_graph{};
 
   // state of the last td_bottom_up (for its queries): vertex count, levels

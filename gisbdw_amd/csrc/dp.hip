@@ -469,6 +469,11 @@ __device__ __forceinline__ uint32_t LookupCode(const DPGraph* __restrict__ g,
                                                const uint8_t* __restrict__ arena,
                                                const uint32_t* s_cb, const uint32_t* s_base,
                                                uint32_t S) {
+  if (g->direct) {
+    const size_t plane = static_cast<size_t>(1) << (g->n > 5 ? g->n - 5 : 0);
+    const uint32_t* p = reinterpret_cast<const uint32_t*>(arena + g->table) + (S >> 5);
+    return (p[0] >> (S & 31u) & 1u) | (p[plane] >> (S & 31u) & 1u) << 1;
+  }
   const uint32_t lb = g->lb;
   uint32_t H = S >> lb;
   uint32_t tile = s_base[__builtin_popcount(H)];
@@ -496,7 +501,9 @@ __device__ __forceinline__ uint32_t LookupTd(const DPGraph* __restrict__ g,
                                              const uint32_t* s_cb, const uint32_t* s_base,
                                              uint32_t S) {
   const int lb = static_cast<int>(g->lb);
-  const size_t ps = static_cast<size_t>(s_base[g->nh + 1]) << (lb - 3);
+  // direct planes have tiles of one word, lb = 5
+  const size_t ps = g->direct ? static_cast<size_t>(4) << (g->n > 5 ? g->n - 5 : 0)
+                              : static_cast<size_t>(s_base[g->nh + 1]) << (lb - 3);
   const uint8_t* base = arena + g->table;
   const uint32_t words = (1u << (lb - 5)) - 1u;
   uint32_t td = 0, last = 0, T = 0, r = 0;
@@ -505,10 +512,10 @@ __device__ __forceinline__ uint32_t LookupTd(const DPGraph* __restrict__ g,
     const int v = __builtin_ctz(S);
     S &= S - 1;
     T |= 1u << v;
-    if (v >= lb) r += s_cb[(v - lb) * kCbStride + ++h];
+    if (v >= lb && !g->direct) r += s_cb[(v - lb) * kCbStride + ++h];
     if (++since == 3 || !S) {
       since = 0;
-      const uint32_t tile = s_base[h] + r;
+      const uint32_t tile = g->direct ? T >> 5 : s_base[h] + r;
       const uint8_t* p = base + (static_cast<size_t>(tile) << (lb - 3)) + 4 * ((T >> 5) & words);
       const uint32_t g0 = *reinterpret_cast<const uint32_t*>(p);
       const uint32_t g1 = *reinterpret_cast<const uint32_t*>(p + ps);
@@ -584,24 +591,20 @@ __global__ __launch_bounds__(64) void DPWalkKernel(
   }
 }
 
-// The canonical decomposition of one start set per wave, level by level of
-// the tree: every component of the vertices left takes its root (the
-// smallest v with td(C \ v) = td(C) - 1) in the same round, the parent of a
-// root is the root whose removal created its component, and all roots leave
-// together.  The tree is the one GetElimination's order produces (each
-// component's root depends only on the component), in about td rounds
-// instead of n.  parent_out: 64 int8 per graph; td_out: the tree's depth.
-__global__ __launch_bounds__(64) void DPTreeKernel(
-    const DPGraph* __restrict__ gs, const uint32_t* __restrict__ g_cb,
-    const uint8_t* __restrict__ arena, const uint32_t* __restrict__ start,
-    int8_t* __restrict__ parent_out, int32_t* __restrict__ td_out) {
-  __shared__ uint32_t s_cb[32 * kCbStride];
-  __shared__ uint32_t s_base[kLookupWords];
-  const DPGraph* g = gs + blockIdx.x;
-  LoadLookupTables(g, g_cb, s_cb, s_base);
-  const int lane = threadIdx.x;
-  const uint32_t myadj = lane < 32 ? g->adj[lane] : 0u;
-  uint32_t S = start[blockIdx.x];
+// The canonical decomposition of vertex set S by one wave (lane u holds
+// adj[u] in myadj), level by level of the tree: every component of the
+// vertices left takes its root (the smallest v with td(C \ v) = td(C) - 1) in
+// the same round, the parent of a root is the root whose removal created its
+// component, and all roots leave together.  The tree is the one
+// GetElimination's order produces (each component's root depends only on the
+// component), in about td rounds instead of n.  code(S): the Gray code of
+// td(S) mod 4.  Returns lane u's parent (-1: a root); *depth_out = the tree's
+// depth in every lane.
+template <typename Code>
+__device__ __forceinline__ int DecomposeWave(uint32_t myadj, uint32_t S, int* depth_out,
+                                             Code code) {
+  const int lane = threadIdx.x & 63;
+  if (lane >= 32) myadj = 0u;
   int creator = -1, depth = 0, parent = -1;
   // every round removes at least one vertex per component, so at most 32
   for (int round = 0; round < 32 && S; ++round) {
@@ -620,8 +623,8 @@ __global__ __launch_bounds__(64) void DPTreeKernel(
       rest &= ~comp;
     }
     // td(C \ v) is td(C) or td(C) - 1: the codes mod 4 tell which
-    const uint32_t cc = in ? LookupCode(g, arena, s_cb, s_base, mine) : 0u;
-    const uint32_t cv = in ? LookupCode(g, arena, s_cb, s_base, mine & ~(1u << lane)) : 0u;
+    const uint32_t cc = in ? code(mine) : 0u;
+    const uint32_t cv = in ? code(mine & ~(1u << lane)) : 0u;
     const uint32_t cand = static_cast<uint32_t>(__ballot(in && cv != cc));
     // a connected set always has a vertex with td(C \ v) = td(C) - 1; the
     // lowest vertex stands in only so that a damaged table cannot stall
@@ -636,10 +639,29 @@ __global__ __launch_bounds__(64) void DPTreeKernel(
     }
     S &= ~static_cast<uint32_t>(__ballot(in && root == lane));
   }
+  *depth_out = static_cast<int>(WaveMax(static_cast<uint32_t>(depth)));
+  return parent;
+}
+
+// DecomposeWave for one whole graph per workgroup, from tables in memory.
+// parent_out: 64 int8 per graph; td_out: the tree's depth.
+__global__ __launch_bounds__(64) void DPTreeKernel(
+    const DPGraph* __restrict__ gs, const uint32_t* __restrict__ g_cb,
+    const uint8_t* __restrict__ arena, int8_t* __restrict__ parent_out,
+    int32_t* __restrict__ td_out) {
+  __shared__ uint32_t s_cb[32 * kCbStride];
+  __shared__ uint32_t s_base[kLookupWords];
+  const DPGraph* g = gs + blockIdx.x;
+  LoadLookupTables(g, g_cb, s_cb, s_base);
+  const int lane = threadIdx.x;
+  const uint32_t S = g->n >= 32 ? ~0u : (1u << g->n) - 1u;
+  int depth = 0;
+  const int parent =
+      DecomposeWave(lane < 32 ? g->adj[lane] : 0u, S, &depth,
+                    [&](uint32_t C) { return LookupCode(g, arena, s_cb, s_base, C); });
   int8_t* out = parent_out + static_cast<size_t>(blockIdx.x) * 64;
-  if (lane < 32 && ((start[blockIdx.x] >> lane) & 1u)) out[lane] = static_cast<int8_t>(parent);
-  const uint32_t d = WaveMax(static_cast<uint32_t>(depth));
-  if (lane == 0) td_out[blockIdx.x] = static_cast<int32_t>(d);
+  if (lane < 32 && ((S >> lane) & 1u)) out[lane] = static_cast<int8_t>(parent);
+  if (lane == 0) td_out[blockIdx.x] = depth;
 }
 
 // Level-k table in colex order over n vertices (td values): the `count`
@@ -658,6 +680,14 @@ __global__ __launch_bounds__(256) void DPExportLevelKernel(
     out[r] = static_cast<uint8_t>(LookupTd(g, arena, s_cb, s_base, S));
   }
 }
+
+}  // namespace
+}  // namespace tdhip
+
+#include "dplds.hpp"
+
+namespace tdhip {
+namespace {
 
 // ---------------------------------------------------------------------------
 // host side
@@ -953,12 +983,127 @@ bool ClaimsPacked(const td_ctx* ctx, int n) {
          n - ctx->dp.low_bits >= ctx->dp.class_min_nh;
 }
 
-// descriptor, walk start set and step count in one device block, uploaded
-// from page-locked staging in one copy; the tree (64 parents, then the depth)
-// comes back the same way
-constexpr size_t kStartOff = (sizeof(DPGraph) + 15) / 16 * 16;
-constexpr size_t kInBytes = kStartOff + 16;
+// The descriptor goes up from page-locked staging in one copy; the tree (64
+// parents, then the depth) comes back the same way.
+constexpr size_t kInBytes = (sizeof(DPGraph) + 15) / 16 * 16 + 16;
 constexpr size_t kTreeBytes = 64 + 16;
+
+// What a single solve reports besides its answer.
+void FillStats(td_dp_stats* stats, int n, uint64_t launches, uint64_t level_kernels,
+               double level_ms, double tree_ms, std::chrono::steady_clock::time_point t0) {
+  stats->graphs = 1;
+  stats->level_kernels = level_kernels;
+  stats->subsets = 1ull << n;
+  stats->alg_bytes = (1ull << (n - 1)) * static_cast<uint64_t>(n + 2);
+  stats->launches = launches;
+  stats->level_ms = level_ms;
+  stats->tree_ms = tree_ms;
+  stats->total_ms =
+      std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+}
+
+// Results of DPLdsKernel in host-visible memory: 64 parents, the depth, and
+// three readings of the device's clock.
+struct LdsOut {
+  int8_t parent[64];
+  int32_t td;
+  int32_t status;
+  unsigned long long clock[3];
+};
+
+// One launch for a graph of at most kLdsMaxN vertices: the graph goes up in
+// the kernel's arguments and the kernel writes its results to `out` itself, so
+// no copy and no event stands beside it.
+void LaunchLds(td_ctx* ctx, const DPGraph& G, const uint32_t* cb, uint8_t* arena, LdsOut* out) {
+  LdsGraph one;
+  one.n = G.n;
+  for (int v = 0; v < kLdsMaxN; ++v) one.adj[v] = G.adj[v];
+  const int n = static_cast<int>(G.n);
+  hipLaunchKernelGGL(DPLdsKernel, dim3(1), dim3(LdsThreads(n)), LdsBytes(n), ctx->stream,
+                     static_cast<const LdsGraph*>(nullptr), one, cb,
+                     reinterpret_cast<uint32_t*>(arena), out->parent, &out->td, out->clock);
+  TD_HIP(hipGetLastError());
+}
+
+// DPFlowKernel's buffer with room for `words` bytes of published words behind
+// the ticket counter: null where the byte budget or the device has no room for
+// it (the other kernels do without).  It is cleared when it is new and
+// (LaunchFlow) when the 16-bit tags have come round, so no word in it carries
+// a tag that is still to come.
+constexpr size_t kFlowHead = 256;
+void ClearFlow(td_ctx* ctx) {
+  const auto& b = ctx->bufs["dp.flow"];
+  TD_HIP(hipMemsetAsync(b.p, 0, b.bytes, ctx->stream));
+  ctx->flow_tag = 0;
+  ctx->flow_tickets = 0;
+}
+uint8_t* FlowBuffer(td_ctx* ctx, size_t words) {
+  const size_t bytes = kFlowHead + words;
+  auto it = ctx->bufs.find("dp.flow");
+  const bool fits = it != ctx->bufs.end() && it->second.p && it->second.bytes >= bytes;
+  uint8_t* p = nullptr;
+  try {
+    p = static_cast<uint8_t*>(ctx->Buffer("dp.flow", bytes));
+  } catch (const Error& e) {
+    if (e.code != TD_E_NOMEM) throw;
+    return nullptr;
+  }
+  if (!fits) ClearFlow(ctx);
+  return p;
+}
+
+// The first of `count` graphs of kFlowMinN..kFlowMaxN vertices, largest first
+// (sizes at ns[i * stride]), as many as fit one launch of a workgroup per CU
+// (or one graph): the launch's classes.  *words and *planes receive the bytes
+// of published words and planes, *groups the workgroups; returns the graphs.
+int PlanFlow(const td_ctx* ctx, int count, const uint32_t* ns, size_t stride, FlowCall* f,
+             size_t* words, size_t* planes, uint32_t* groups) {
+  *words = *planes = 0;
+  *groups = 0;
+  f->classes = 0;
+  int i = 0;
+  for (; i < count; ++i) {
+    const uint32_t n = ns[i * stride];
+    const uint32_t more = 1u << FlowTop(static_cast<int>(n));
+    if (i && *groups + more > static_cast<uint32_t>(ctx->prop.multiProcessorCount)) break;
+    if (!f->classes || f->c[f->classes - 1].n != n)
+      f->c[f->classes++] = {n, *groups, static_cast<uint32_t>(i), *words / 8, *planes / 4};
+    *groups += more;
+    *words += FlowBytes(static_cast<int>(n));
+    *planes += DirectBytes(static_cast<int>(n));
+  }
+  return i;
+}
+
+// The levels and decompositions of the planned graphs.
+void LaunchFlow(td_ctx* ctx, FlowCall& f, int count, uint32_t groups, const FlowGraph* gs,
+                const uint32_t* cb, uint8_t* planes, uint8_t* buf, int8_t* parents, int32_t* tds,
+                int32_t* status, unsigned long long* clock) {
+  if (ctx->flow_tag >= 0xFFFFu) ClearFlow(ctx);
+  f.ticket0 = ctx->flow_tickets;
+  f.tag = ++ctx->flow_tag;
+  f.spin = static_cast<uint32_t>(ctx->dp.flow_spin);
+  uint32_t* ticket = reinterpret_cast<uint32_t*>(buf);
+  auto* ex = reinterpret_cast<unsigned long long*>(buf + kFlowHead);
+  uint32_t* table = reinterpret_cast<uint32_t*>(planes);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(groups), dim3(512), 0, ctx->stream, f, gs, cb, ex, ticket,
+                       table, status, clock);
+  };
+  switch (f.c[0].n) {  // the largest
+    case 19: launch(DPFlowKernel<3>); break;
+    case 20: launch(DPFlowKernel<4>); break;
+    case 21: launch(DPFlowKernel<5>); break;
+    case 22: launch(DPFlowKernel<6>); break;
+    case 23: launch(DPFlowKernel<7>); break;
+    default: launch(DPFlowKernel<8>); break;
+  }
+  TD_HIP(hipGetLastError());
+  ctx->flow_tickets += groups;
+  hipLaunchKernelGGL(DPDirectTreeKernel, dim3(count), dim3(64), 0, ctx->stream, f, gs, table,
+                     parents, tds, clock);
+  TD_HIP(hipGetLastError());
+}
 
 void SolveOne(td_ctx* ctx, int n, const uint64_t* adj, uint8_t* td_out,
               int8_t* parent_out, td_dp_stats* stats) {
@@ -967,24 +1112,58 @@ void SolveOne(td_ctx* ctx, int n, const uint64_t* adj, uint8_t* td_out,
   // the buffers below may be reallocated: until this solve completes, the
   // queries have no tables to read
   ctx->have_dp = false;
-  DPGraph G = SingleGraph(ctx, n, adj);
+  const bool lds = n <= kLdsMaxN, flow = !lds && n <= kFlowMaxN;
+  DPGraph G = SingleGraph(ctx, n, adj, !lds && !flow);
   const uint64_t tbytes = ClaimedBytes(G, ClaimsPacked(ctx, n));
   uint8_t* arena = static_cast<uint8_t*>(ctx->Buffer("dp.arena", tbytes));
   uint8_t* din = static_cast<uint8_t*>(ctx->Buffer("dp.graph", kInBytes));
   DPGraph* dG = reinterpret_cast<DPGraph*>(din);
-  uint32_t* dstart = reinterpret_cast<uint32_t*>(din + kStartOff);
   const uint32_t* cb = PascalDevice(ctx);
   uint8_t* dtree = static_cast<uint8_t*>(ctx->Buffer("dp.tree_out", kTreeBytes));
-  uint8_t* stage = static_cast<uint8_t*>(ctx->Pinned(kInBytes + kTreeBytes));
-  const uint32_t full = n >= 32 ? 0xFFFFFFFFu : ((1u << n) - 1u);
+  uint8_t* stage = static_cast<uint8_t*>(ctx->Pinned(kInBytes + sizeof(LdsOut)));
+  uint8_t* fbuf = flow ? FlowBuffer(ctx, FlowBytes(n)) : nullptr;
+  ctx->last_n = n;
+  ctx->record_up = !lds && !fbuf;
+  if (lds || fbuf) {
+    LdsOut* out = reinterpret_cast<LdsOut*>(stage + kInBytes);
+    if (lds) {
+      LaunchLds(ctx, G, cb, arena, out);
+    } else {
+      FlowCall f;
+      size_t words, planes;
+      uint32_t groups;
+      PlanFlow(ctx, 1, &G.n, 1, &f, &words, &planes, &groups);
+      std::memcpy(f.one.adj, G.adj, sizeof(f.one.adj));
+      out->status = 0;
+      LaunchFlow(ctx, f, 1, groups, nullptr, cb, arena, fbuf, out->parent, &out->td, &out->status,
+                 out->clock);
+    }
+    TD_HIP(hipStreamSynchronize(ctx->stream));
+    if (lds || !out->status) {
+      if (td_out) *td_out = static_cast<uint8_t>(out->td);
+      if (parent_out) std::memcpy(parent_out, out->parent, n);
+      G.direct = 1;
+      ctx->last_graph = G;
+      ctx->have_dp = true;
+      if (stats) {
+        const double ms = 1.0 / ctx->clock_khz;
+        FillStats(stats, n, lds ? 1 : 2, 1,
+                  static_cast<double>(out->clock[1] - out->clock[0]) * ms,
+                  static_cast<double>(out->clock[2] - out->clock[1]) * ms, t0);
+      }
+      return;
+    }
+    ctx->record_up = true;  // a wait was given up: the level kernels solve it
+  }
+  if (flow) G = SingleGraph(ctx, n, adj);
+  ctx->last_graph = G;
   std::memcpy(stage, &G, sizeof(G));
-  std::memcpy(stage + kStartOff, &full, 4);
   TD_HIP(hipMemcpyAsync(din, stage, kInBytes, hipMemcpyHostToDevice, ctx->stream));
   uint64_t launches = 0;
   TD_HIP(hipEventRecord(ctx->ev[0], ctx->stream));
   RunLevels(ctx, G, dG, cb, arena, &launches);
   TD_HIP(hipEventRecord(ctx->ev[1], ctx->stream));
-  hipLaunchKernelGGL(DPTreeKernel, dim3(1), dim3(64), 0, ctx->stream, dG, cb, arena, dstart,
+  hipLaunchKernelGGL(DPTreeKernel, dim3(1), dim3(64), 0, ctx->stream, dG, cb, arena,
                      reinterpret_cast<int8_t*>(dtree), reinterpret_cast<int32_t*>(dtree + 64));
   TD_HIP(hipGetLastError());
   ++launches;
@@ -996,21 +1175,22 @@ void SolveOne(td_ctx* ctx, int n, const uint64_t* adj, uint8_t* td_out,
   std::memcpy(&td, staged + 64, 4);
   if (td_out) *td_out = static_cast<uint8_t>(td);
   if (parent_out) std::memcpy(parent_out, staged, n);
-  ctx->last_n = n;
-  ctx->last_graph = G;
   ctx->have_dp = true;
-  if (stats) {
-    stats->graphs = 1;
-    stats->level_kernels = LevelKernelCount(G);
-    stats->subsets = 1ull << n;
-    stats->alg_bytes = (1ull << (n - 1)) * static_cast<uint64_t>(n + 2);
-    stats->launches = launches;
-    stats->level_ms = Elapsed(ctx->ev[0], ctx->ev[1]);
-    stats->tree_ms = Elapsed(ctx->ev[1], ctx->ev[2]);
-    stats->total_ms = std::chrono::duration<double, std::milli>(
-                          std::chrono::steady_clock::now() - t0)
-                          .count();
+  if (stats)
+    FillStats(stats, n, launches, LevelKernelCount(G), Elapsed(ctx->ev[0], ctx->ev[1]),
+              Elapsed(ctx->ev[1], ctx->ev[2]), t0);
+}
+
+// The device record of the last single solve, which the queries read; a graph
+// solved by DPLdsKernel has none until the first query.
+const DPGraph* LastRecord(td_ctx* ctx) {
+  void* d = ctx->bufs["dp.graph"].p;
+  if (!ctx->record_up) {
+    TD_HIP(hipMemcpyAsync(d, &ctx->last_graph, sizeof(DPGraph), hipMemcpyHostToDevice,
+                          ctx->stream));
+    ctx->record_up = true;
   }
+  return static_cast<const DPGraph*>(d);
 }
 
 // ---------------------------------------------------------------------------
@@ -1060,7 +1240,6 @@ void SolveOneNoAlloc(td_ctx* ctx, int n, const uint64_t* adj, uint8_t* td_out,
              "level tables exceed the fixed device array");
   uint8_t* din = base;
   const DPGraph* dG = reinterpret_cast<const DPGraph*>(din);
-  const uint32_t* dstart = reinterpret_cast<const uint32_t*>(din + kStartOff);
   uint8_t* dtree = base + kNoAllocTreeOff;
   const uint32_t* cb = reinterpret_cast<const uint32_t*>(base + kNoAllocPascalOff);
   uint8_t* arena = base + kNoAllocArenaOff;
@@ -1068,16 +1247,14 @@ void SolveOneNoAlloc(td_ctx* ctx, int n, const uint64_t* adj, uint8_t* td_out,
   // before the frame ends), results back into it
   alignas(16) uint8_t in[kInBytes];
   alignas(16) uint8_t tree[kTreeBytes];
-  const uint32_t full = (1u << n) - 1u;
   std::memcpy(in, &G, sizeof(G));
-  std::memcpy(in + kStartOff, &full, 4);
   TD_HIP(hipMemcpyAsync(din, in, kInBytes, hipMemcpyHostToDevice, ctx->stream));
   uint64_t launches = 0;
   TD_HIP(hipEventRecord(ctx->ev[0], ctx->stream));
   // direct launches: a captured graph would be instantiated (allocated) here
   LaunchLevelsLB(ctx, G, dG, cb, arena, &launches, ctx->stream, -1, 1);
   TD_HIP(hipEventRecord(ctx->ev[1], ctx->stream));
-  hipLaunchKernelGGL(DPTreeKernel, dim3(1), dim3(64), 0, ctx->stream, dG, cb, arena, dstart,
+  hipLaunchKernelGGL(DPTreeKernel, dim3(1), dim3(64), 0, ctx->stream, dG, cb, arena,
                      reinterpret_cast<int8_t*>(dtree), reinterpret_cast<int32_t*>(dtree + 64));
   TD_HIP(hipGetLastError());
   ++launches;
@@ -1088,18 +1265,9 @@ void SolveOneNoAlloc(td_ctx* ctx, int n, const uint64_t* adj, uint8_t* td_out,
   std::memcpy(&td, tree + 64, 4);
   if (td_out) *td_out = static_cast<uint8_t>(td);
   if (parent_out) std::memcpy(parent_out, tree, n);
-  if (stats) {
-    stats->graphs = 1;
-    stats->level_kernels = LevelKernelCount(G);
-    stats->subsets = 1ull << n;
-    stats->alg_bytes = (1ull << (n - 1)) * static_cast<uint64_t>(n + 2);
-    stats->launches = launches;
-    stats->level_ms = Elapsed(ctx->ev[0], ctx->ev[1]);
-    stats->tree_ms = Elapsed(ctx->ev[1], ctx->ev[2]);
-    stats->total_ms = std::chrono::duration<double, std::milli>(
-                          std::chrono::steady_clock::now() - t0)
-                          .count();
-  }
+  if (stats)
+    FillStats(stats, n, launches, LevelKernelCount(G), Elapsed(ctx->ev[0], ctx->ev[1]),
+              Elapsed(ctx->ev[1], ctx->ev[2]), t0);
 }
 
 // ---------------------------------------------------------------------------
@@ -1186,9 +1354,7 @@ void SolveLarge(td_ctx* ctx, const std::vector<int>& idx, const int32_t* ns,
       if (j >= S) consume(j - S);  // frees slot s: its tree, copies and levels are done
       const DPGraph G = SingleGraph(ctx, ns[i], adj_concat + row_off[i]);
       uint8_t* in = stage + s * kSlot;
-      const uint32_t full = G.n >= 32 ? 0xFFFFFFFFu : ((1u << G.n) - 1u);
       std::memcpy(in, &G, sizeof(G));
-      std::memcpy(in + kStartOff, &full, 4);
       TD_HIP(hipMemcpyAsync(din[s], in, kInBytes, hipMemcpyHostToDevice, st));
       const DPGraph* dG = reinterpret_cast<const DPGraph*>(din[s]);
       const bool split = K > 1 && SplitsInto(G, K);
@@ -1207,7 +1373,6 @@ void SolveLarge(td_ctx* ctx, const std::vector<int>& idx, const int32_t* ns,
       *level_kernels += LevelKernelCount(G);
       TD_HIP(hipStreamWaitEvent(ctx->side, lv_end[s], 0));
       hipLaunchKernelGGL(DPTreeKernel, dim3(1), dim3(64), 0, ctx->side, dG, cb, arena[s],
-                         reinterpret_cast<const uint32_t*>(din[s] + kStartOff),
                          reinterpret_cast<int8_t*>(dtree[s]),
                          reinterpret_cast<int32_t*>(dtree[s] + 64));
       TD_HIP(hipGetLastError());
@@ -1330,6 +1495,45 @@ void LaunchBatch(td_ctx* ctx, int mode, int ngraphs,
   TD_HIP(hipGetLastError());
 }
 
+// Whether DPFlowKernel takes a batch's graphs of 19..24 vertices (the first
+// `count` of perm, largest first) rather than the persistent kernel.  A launch
+// of DPFlowKernel (one workgroup per CU) and its trees takes 70 us or less; the
+// persistent kernel takes a workgroup's time for the largest graph, measured as 75 us +
+// 1150 us 2^(n - 24) (n = 19: 103 us, 20: 135, 22: 345, 24: 1220), and then
+// the others cost it little.  16 graphs of n = 19 / 20 / 22: 76 / 82 / 240 us
+// a call against 134 / 173 / 398, four of n = 24 345 against 1283.
+bool FlowPays(const td_ctx* ctx, int count, const int32_t* ns, const std::vector<int>& perm) {
+  if (count == 0 || ns[perm[0]] > kFlowMaxN) return false;
+  uint64_t groups = 0;
+  for (int j = 0; j < count; ++j) groups += 1ull << FlowTop(ns[perm[j]]);
+  const uint64_t cus = static_cast<uint64_t>(ctx->prop.multiProcessorCount);
+  return (groups + cus - 1) / cus * 70 <= 75 + (1150u >> (24 - ns[perm[0]]));
+}
+
+// Graphs of at most kLdsMaxN vertices, largest first, one workgroup each.
+// More graphs than CUs go in one launch per workgroup size, so that small
+// graphs do not hold the LDS and threads of large ones; fewer fit in one
+// launch, a CU each.
+uint64_t LaunchLdsBatch(td_ctx* ctx, int count, const LdsGraph* Ls, const uint32_t* cb,
+                        int8_t* parents, int32_t* tds) {
+  uint64_t launches = 0;
+  for (int at = 0; at < count;) {
+    const int n = static_cast<int>(Ls[at].n), threads = LdsThreads(n);
+    int end = at + 1;
+    while (end < count && (count <= ctx->prop.multiProcessorCount ||
+                           LdsThreads(static_cast<int>(Ls[end].n)) == threads))
+      ++end;
+    hipLaunchKernelGGL(DPLdsKernel, dim3(end - at), dim3(threads), LdsBytes(n), ctx->stream,
+                       Ls + at, LdsGraph{}, cb, static_cast<uint32_t*>(nullptr),
+                       parents + 64ull * at, tds + at,
+                       static_cast<unsigned long long*>(nullptr));
+    TD_HIP(hipGetLastError());
+    ++launches;
+    at = end;
+  }
+  return launches;
+}
+
 void SolveBatch(td_ctx* ctx, int ngraphs, const int32_t* ns,
                 const uint64_t* adj_concat, uint8_t* td_out,
                 int8_t* parent_concat, int mode, td_dp_stats* stats) {
@@ -1356,12 +1560,24 @@ void SolveBatch(td_ctx* ctx, int ngraphs, const int32_t* ns,
   std::stable_sort(perm.begin(), perm.end(),
                    [&](int a, int b) { return ns[a] > ns[b]; });
   const int nsmall = static_cast<int>(perm.size());
-  // page-locked block of the small graphs' records, start sets and results
-  const size_t o_start = sizeof(DPGraph) * nsmall;
-  const size_t o_par = (o_start + 4ull * nsmall + 15) / 16 * 16;
+  // of these, mode 0 gives the last ones, of at most kLdsMaxN vertices, to
+  // DPLdsKernel
+  int nmid = nsmall;
+  while (mode == 0 && nmid > 0 && ns[perm[nmid - 1]] <= kLdsMaxN) --nmid;
+  // and, where that is faster, the others to DPFlowKernel
+  int nbig = mode == 0 && FlowPays(ctx, nmid, ns, perm) ? 0 : nmid;
+  // page-locked block of the small graphs' records and results; the kernels
+  // write the results (and DPLdsKernel reads its graphs) there themselves
+  const size_t o_lds = sizeof(DPGraph) * nsmall;
+  const size_t o_flow = o_lds + sizeof(LdsGraph) * (nsmall - nmid);
+  const size_t o_par = (o_flow + sizeof(FlowGraph) * (nmid - nbig) + 63) / 64 * 64;
   const size_t o_td = o_par + 64ull * nsmall;
   uint8_t* block = static_cast<uint8_t*>(ctx->Pinned(o_td + 4ull * nsmall + 16, 1));
+  int32_t* flow_status = reinterpret_cast<int32_t*>(block + o_td + 4ull * nsmall);
+  *flow_status = 0;
   DPGraph* Gs = reinterpret_cast<DPGraph*>(block);
+  LdsGraph* Ls = reinterpret_cast<LdsGraph*>(block + o_lds);
+  FlowGraph* Fs = reinterpret_cast<FlowGraph*>(block + o_flow);
   // every graph is checked, and the small graphs' records are built, on the
   // context's worker threads (about 0.3 us and 1 us a graph) before any GPU work;
   // a failure is reported for the lowest failing graph, as a serial check
@@ -1381,6 +1597,12 @@ void SolveBatch(td_ctx* ctx, int ngraphs, const int32_t* ns,
       for (int j = t; j < nsmall; j += T) {
         const int i = perm[j];
         Gs[j] = MakeGraph(ns[i], adj_concat + row_off[i], WordBits(lb), 0, mode != 0);
+        if (j >= nmid) {
+          Ls[j - nmid].n = Gs[j].n;
+          std::memcpy(Ls[j - nmid].adj, Gs[j].adj, sizeof(Ls[0].adj));
+        } else if (j >= nbig) {
+          std::memcpy(Fs[j - nbig].adj, Gs[j].adj, sizeof(Fs[0].adj));
+        }
       }
     };
     if (ngraphs < 256) {
@@ -1426,7 +1648,7 @@ void SolveBatch(td_ctx* ctx, int ngraphs, const int32_t* ns,
   uint64_t off = 0, claimed = 0;
   for (int j = 0; j < ngraphs; ++j) {
     Gs[j].table = off;
-    off += (TableBytes(Gs[j]) + 255) / 256 * 256;
+    if (j < nbig) off += (TableBytes(Gs[j]) + 255) / 256 * 256;
     claimed += (ClaimedBytes(Gs[j]) + 255) / 256 * 256;
   }
   uint8_t* arena = static_cast<uint8_t*>(ctx->Buffer("dp.batch_arena", claimed));
@@ -1434,43 +1656,82 @@ void SolveBatch(td_ctx* ctx, int ngraphs, const int32_t* ns,
       ctx->Buffer("dp.batch_graphs", sizeof(DPGraph) * ngraphs));
   const uint32_t* cb = PascalDevice(ctx);
   uint32_t* dq = static_cast<uint32_t*>(ctx->Buffer("dp.batch_queue", 256));
-  uint32_t* dstart = static_cast<uint32_t*>(ctx->Buffer("dp.batch_start", 4 * ngraphs));
-  int8_t* dpar = static_cast<int8_t*>(ctx->Buffer("dp.batch_parent", 64ull * ngraphs));
-  int32_t* dtd = static_cast<int32_t*>(ctx->Buffer("dp.batch_td", 4ull * ngraphs));
-  uint32_t* start = reinterpret_cast<uint32_t*>(block + o_start);
-  for (int j = 0; j < ngraphs; ++j)
-    start[j] = Gs[j].n >= 32 ? 0xFFFFFFFFu : ((1u << Gs[j].n) - 1u);
+  int8_t* par = reinterpret_cast<int8_t*>(block + o_par);
+  int32_t* tds = reinterpret_cast<int32_t*>(block + o_td);
+  // without room for DPFlowKernel's words its graphs take the persistent launch
+  FlowCall flow;
+  size_t flow_words = 0, flow_planes = 0;
+  uint32_t flow_groups = 0;
+  uint8_t* fbuf = nullptr;
+  if (nbig < nmid) {
+    // the first launch holds the largest graphs, but later ones more of them
+    size_t most = 0;
+    for (int j = nbig; j < nmid;) {
+      j += PlanFlow(ctx, nmid - j, &Gs[j].n, sizeof(DPGraph) / 4, &flow, &flow_words,
+                    &flow_planes, &flow_groups);
+      most = std::max(most, flow_words);
+    }
+    fbuf = FlowBuffer(ctx, most);
+  }
+  if (!fbuf) {
+    for (int j = nbig; j < nmid; ++j) {
+      Gs[j].table = off;
+      off += (TableBytes(Gs[j]) + 255) / 256 * 256;
+    }
+    nbig = nmid;
+  }
   if (mode == 0) {
     // the persistent kernel reads only each record's head and builds the
-    // tables itself: 416 of the 4640 bytes per graph go up
+    // tables itself: 288 of the 4512 bytes per graph go up
     constexpr size_t kHead = offsetof(DPGraph, nbh);
-    TD_HIP(hipMemcpy2DAsync(dGs, sizeof(DPGraph), Gs, sizeof(DPGraph), kHead, ngraphs,
-                            hipMemcpyHostToDevice, ctx->stream));
+    if (nbig > 0)
+      TD_HIP(hipMemcpy2DAsync(dGs, sizeof(DPGraph), Gs, sizeof(DPGraph), kHead, nbig,
+                              hipMemcpyHostToDevice, ctx->stream));
   } else {
     TD_HIP(hipMemcpyAsync(dGs, Gs, sizeof(DPGraph) * ngraphs, hipMemcpyHostToDevice,
                           ctx->stream));
   }
-  TD_HIP(hipMemcpyAsync(dstart, start, 4 * ngraphs, hipMemcpyHostToDevice, ctx->stream));
   uint64_t small_launches = 0;
   TD_HIP(hipEventRecord(ctx->ev[0], ctx->stream));
-  switch (WordBits(lb)) {
-    case 0: LaunchBatch<0>(ctx, mode, ngraphs, Gs, dGs, cb, arena, dq, &small_launches); break;
-    case 1: LaunchBatch<1>(ctx, mode, ngraphs, Gs, dGs, cb, arena, dq, &small_launches); break;
-    default: LaunchBatch<2>(ctx, mode, ngraphs, Gs, dGs, cb, arena, dq, &small_launches); break;
+  if (nbig > 0) {
+    switch (WordBits(lb)) {
+      case 0: LaunchBatch<0>(ctx, mode, nbig, Gs, dGs, cb, arena, dq, &small_launches); break;
+      case 1: LaunchBatch<1>(ctx, mode, nbig, Gs, dGs, cb, arena, dq, &small_launches); break;
+      default: LaunchBatch<2>(ctx, mode, nbig, Gs, dGs, cb, arena, dq, &small_launches); break;
+    }
   }
+  for (int j = nbig; j < nmid;) {
+    const int k = PlanFlow(ctx, nmid - j, &Gs[j].n, sizeof(DPGraph) / 4, &flow, &flow_words,
+                           &flow_planes, &flow_groups);
+    LaunchFlow(ctx, flow, k, flow_groups, Fs + (j - nbig), cb, arena + off, fbuf, par + 64ull * j,
+               tds + j, flow_status, nullptr);
+    off += (flow_planes + 255) / 256 * 256;
+    small_launches += 2;
+    j += k;
+  }
+  if (nmid < nsmall)
+    small_launches += LaunchLdsBatch(ctx, nsmall - nmid, Ls, cb, par + 64ull * nmid, tds + nmid);
   TD_HIP(hipEventRecord(ctx->ev[1], ctx->stream));
-  // mode 0: the persistent kernel (its queue reset aside); else the launches
+  // mode 0 counts as one level kernel however its graphs were shared out;
+  // else the launches
   level_kernels += mode == 0 ? 1 : small_launches;
-  hipLaunchKernelGGL(DPTreeKernel, dim3(ngraphs), dim3(64), 0, ctx->stream,
-                     dGs, cb, arena, dstart, dpar, dtd);
-  TD_HIP(hipGetLastError());
-  launches += small_launches + 1;
+  if (nbig > 0) {
+    hipLaunchKernelGGL(DPTreeKernel, dim3(nbig), dim3(64), 0, ctx->stream, dGs, cb, arena, par,
+                       tds);
+    TD_HIP(hipGetLastError());
+    ++launches;
+  }
+  launches += small_launches;
   TD_HIP(hipEventRecord(ctx->ev[2], ctx->stream));
-  int8_t* par = reinterpret_cast<int8_t*>(block + o_par);
-  int32_t* tds = reinterpret_cast<int32_t*>(block + o_td);
-  TD_HIP(hipMemcpyAsync(par, dpar, 64ull * ngraphs, hipMemcpyDeviceToHost, ctx->stream));
-  TD_HIP(hipMemcpyAsync(tds, dtd, 4ull * ngraphs, hipMemcpyDeviceToHost, ctx->stream));
   TD_HIP(hipStreamSynchronize(ctx->stream));
+  // a wait was given up: those graphs one by one (SolveOne falls back itself)
+  if (*flow_status)
+    for (int j = nbig; j < nmid; ++j) {
+      uint8_t td = 0;
+      SolveOne(ctx, ns[perm[j]], adj_concat + row_off[perm[j]], &td, par + 64ull * j, nullptr);
+      tds[j] = td;
+    }
+  if (*flow_status) ctx->have_dp = false;
   for (int j = 0; j < ngraphs; ++j) {
     const int i = perm[j];
     if (td_out) td_out[i] = static_cast<uint8_t>(tds[j]);
@@ -1603,6 +1864,10 @@ void NoAllocSetup(td_ctx* ctx) {
   TD_REQUIRE(ctx->device >= 0 && ctx->device < kNoAllocMaxDevices, TD_E_INVALID,
              "device index beyond the scratch table");
   if (g_noalloc_ptr[ctx->device]) return;
+  // DPLdsKernel takes up to 96 KiB of words
+  TD_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&DPLdsKernel),
+                             hipFuncAttributeMaxDynamicSharedMemorySize,
+                             static_cast<int>(LdsBytes(kLdsMaxN))));
   void* p = nullptr;
   TD_HIP(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)));
   TD_REQUIRE(p != nullptr, TD_E_HIP, "hipGetSymbolAddress returned no address");
@@ -1645,7 +1910,7 @@ int td_dp_get_treedepth(td_ctx* ctx, int32_t k, uint64_t code,
     // one subset of level k, as td_dp_get_level reads them
     uint8_t* d = static_cast<uint8_t*>(ctx->Buffer("dp.walk_order", 64 * 4));
     hipLaunchKernelGGL(DPExportLevelKernel, dim3(1), dim3(64), 0, ctx->stream,
-                       static_cast<const DPGraph*>(ctx->bufs["dp.graph"].p), PascalDevice(ctx),
+                       LastRecord(ctx), PascalDevice(ctx),
                        static_cast<const uint8_t*>(ctx->bufs["dp.arena"].p), k,
                        static_cast<uint32_t>(code), 1u, d);
     TD_HIP(hipGetLastError());
@@ -1664,7 +1929,7 @@ int td_dp_get_level(td_ctx* ctx, int32_t k, uint8_t* out, uint64_t out_len) {
     const uint64_t count = Binom(n, k);
     TD_REQUIRE(out && out_len >= count, TD_E_INVALID, "output too small");
     uint8_t* d = static_cast<uint8_t*>(ctx->Buffer("dp.export", count));
-    const DPGraph* dG = static_cast<const DPGraph*>(ctx->bufs["dp.graph"].p);
+    const DPGraph* dG = LastRecord(ctx);
     const uint8_t* arena = static_cast<const uint8_t*>(ctx->bufs["dp.arena"].p);
     const int grid = GridFor(ctx, count, 256);
     hipLaunchKernelGGL(DPExportLevelKernel, dim3(grid), dim3(256), 0,
@@ -1695,7 +1960,7 @@ int td_dp_get_elimination(td_ctx* ctx, int32_t nverts, int32_t subset_size,
     int32_t* dorder = static_cast<int32_t*>(ctx->Buffer("dp.walk_order", 64 * 4));
     TD_HIP(hipMemcpyAsync(dstart, &S, 4, hipMemcpyHostToDevice, ctx->stream));
     TD_HIP(hipMemcpyAsync(dsteps, &steps, 4, hipMemcpyHostToDevice, ctx->stream));
-    const DPGraph* dG = static_cast<const DPGraph*>(ctx->bufs["dp.graph"].p);
+    const DPGraph* dG = LastRecord(ctx);
     const uint8_t* arena = static_cast<const uint8_t*>(ctx->bufs["dp.arena"].p);
     hipLaunchKernelGGL(DPWalkKernel, dim3(1), dim3(64), 0, ctx->stream, dG,
                        PascalDevice(ctx), arena, dstart, dsteps, dorder, 64);

@@ -566,12 +566,17 @@ __global__ void MLPToBf16Kernel(const float* __restrict__ w, uint16_t* __restric
 // set S (one per wave), positives = {v in S : td(S \ v) = td(S) - 1}.
 struct DPLookup {
   const uint8_t* table;
-  uint32_t lb, nh;
+  uint32_t n, lb, nh, direct;  // as in DPGraph
   uint32_t lvl[34];
 };
 
 // Gray code of td(S) mod 4 from the tables (two bit planes; dpword.hpp)
 __device__ __forceinline__ uint32_t LookupCode(const DPLookup& L, const uint32_t* cb, uint32_t S) {
+  if (L.direct) {
+    const size_t plane = static_cast<size_t>(1) << (L.n > 5 ? L.n - 5 : 0);
+    const uint32_t* p = reinterpret_cast<const uint32_t*>(L.table) + (S >> 5);
+    return (p[0] >> (S & 31u) & 1u) | (p[plane] >> (S & 31u) & 1u) << 1;
+  }
   uint32_t H = S >> L.lb;
   size_t tile = L.lvl[__builtin_popcount(H)];
   for (int i = 1; H; ++i) {
@@ -915,7 +920,9 @@ int td_mlp_make_samples(td_ctx* ctx, int32_t count, uint64_t seed, int32_t* n_ou
     TD_HIP(hipMemcpyAsync(dsets, sets.data(), 4ull * count, hipMemcpyHostToDevice, ctx->stream));
     DPLookup L;
     L.table = static_cast<const uint8_t*>(ctx->bufs["dp.arena"].p) + G.table;
+    L.n = G.n;
     L.lb = G.lb;
+    L.direct = G.direct;
     L.nh = G.nh;
     std::memcpy(L.lvl, G.lvl, sizeof(L.lvl));
     const uint32_t* cb = static_cast<const uint32_t*>(ctx->bufs["dp.pascal"].p);

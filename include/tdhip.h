@@ -50,7 +50,9 @@ const char* td_last_error(const td_ctx* ctx);
  * graphs above 26 vertices in a td_dp_solve_batch call run their level
  * sequences that many at a time on that many streams, each graph starting
  * when the previous one has done the first 1/streams of its subsets; 1: one
- * graph at a time).  "dp.class_bits" (0, 3 or 4, default 0),
+ * graph at a time), "dp.flow_spin" (0..2^30, default 2^17: how often a
+ * workgroup of a graph of 19..24 vertices reads a word that another one has
+ * to publish, before the call is solved without such waits).  "dp.class_bits" (0, 3 or 4, default 0),
  * "dp.class_min_nh" (5..32, default 16), "dp.packed" (0/1, default 0) and
  * "dp.xcd_remap" (0/1) are accepted and kept for callers and tuning caches
  * that set them: one table layout, three bits per subset and contiguous
@@ -84,12 +86,16 @@ typedef struct td_dp_stats {
   uint64_t subsets;      /* sum over graphs of 2^n                        */
   uint64_t alg_bytes;    /* sum over graphs of 2^(n-1) (n+2)              */
   uint64_t launches;     /* kernel launches (or graph replays)            */
-  double level_ms;       /* GPU time of the level kernels (HIP events;
+  double level_ms;       /* GPU time of the level kernels (HIP events, or the
+                            device's clock for single graphs of at most 24
+                            vertices, which one launch resolves;
                             with two graphs' levels in flight, the union of
                             the graphs' level intervals)                  */
   double tree_ms;        /* GPU time of the decomposition (tree) kernel   */
   double total_ms;       /* host wall time of the whole call              */
-  uint64_t level_kernels; /* level-kernel executions behind level_ms       */
+  uint64_t level_kernels; /* level-kernel executions behind level_ms (a batch
+                            call's graphs of at most 26 vertices count as
+                            one in mode 0)                                */
 } td_dp_stats;
 
 /* DynamicGPU::operator()(g) + GetElimination(n, n, 0) + EliminationTree +
@@ -142,7 +148,8 @@ int td_dp_get_elimination(td_ctx* ctx, int32_t nverts, int32_t subset_size,
  * adj_concat holds the rows of graph 0, then graph 1, ...; parent_concat
  * likewise (sum n[i] entries).  For the graphs of at most 26 vertices, mode:
  * 0 = one persistent launch (graphs pulled from a device queue, all levels
- * inside), 1 = level-synchronous launches over the whole batch, 2 = one
+ * inside; graphs of at most 18 vertices in LDS, a workgroup each, and few
+ * graphs of 19..24 vertices in several workgroups each), 1 = level-synchronous launches over the whole batch, 2 = one
  * launch per graph and level (the baseline the persistent launch is
  * measured against).  Larger graphs go one after another through
  * td_dp_solve's level kernels, each graph's decomposition on a second stream

@@ -40,8 +40,9 @@ struct Error {
 // Per-graph DP descriptor, one per graph, read by the kernels with scalar
 // loads.  Vertices 0..4 are the bits of a word of 32 subsets, vertices
 // 5..lb-1 pick a word of a tile, and vertices lb..n-1 are the "high" vertices
-// whose subset H selects the tile.
-struct DPGraph {
+// whose subset H selects the tile.  The head is all that the batch's
+// persistent kernel and the tree kernel read.
+struct DPHead {
   uint32_t n;        // vertices
   uint32_t nh;       // high vertices, max(n - lb, 0)
   uint32_t lb;       // 5 + log2(words per tile): 5, 6 or 7
@@ -49,9 +50,11 @@ struct DPGraph {
   uint64_t table;    // byte offset of this graph's tables in the arena
   uint32_t lvl[34];  // tile offset of high level h; lvl[nh+1] = 2^nh
   uint32_t adj[32];  // adjacency rows
-  // The next three arrays are consecutive (the level kernels copy them to
-  // LDS as one block).  Vertices above 4 come in 7-bit chunks, chunk c from
-  // vertex 5 + 7 c on.
+};
+// The head and the level kernels' tables: three consecutive arrays, which the
+// kernels copy to LDS as one block.  Vertices above 4 come in 7-bit chunks,
+// chunk c from vertex 5 + 7 c on.
+struct DPGraph : DPHead {
   uint32_t nbh[512];  // neighbours of a set of them: nbh[128 c + chunk]
   uint32_t isoh[512]; // by a set X of them: the L that give every x in X a
                       // neighbour
@@ -59,10 +62,8 @@ struct DPGraph {
                       // y in Y n L has a neighbour in L
 };
 constexpr int kTabNbh = 0, kTabIsoH = 512, kTabIsoL = 1024, kTabWords = 1056;
-static_assert(offsetof(DPGraph, isoh) == offsetof(DPGraph, nbh) + 4 * kTabIsoH,
-              "nbh and isoh must be consecutive");
-static_assert(offsetof(DPGraph, isol) == offsetof(DPGraph, nbh) + 4 * kTabIsoL,
-              "isoh and isol must be consecutive");
+static_assert(sizeof(DPGraph) == sizeof(DPHead) + 4 * kTabWords,
+              "nbh, isoh and isol must follow each other and the head");
 
 // DP launch configuration (autotuned).
 struct DPConfig {

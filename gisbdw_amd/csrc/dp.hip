@@ -29,6 +29,7 @@
 #include <mutex>
 #include <string>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 #include "ctx.hpp"
@@ -272,7 +273,7 @@ __device__ __forceinline__ void LoadShared(const DPGraph* __restrict__ g,
 // Tiles [first, end) of high level h of graph g, R consecutive per lane,
 // lanes of the launch striding by `stride` tiles.
 template <int WB>
-__device__ __forceinline__ void DPLevelRange(const DPGraph* __restrict__ g,
+__device__ __forceinline__ void DPLevelRange(const DPHead* __restrict__ g,
                                              const uint32_t* __restrict__ g_cb,
                                              uint8_t* __restrict__ arena,
                                              int h, uint32_t first,
@@ -370,7 +371,7 @@ __device__ __forceinline__ void LowMasksShared(uint32_t* s_m) {
 // nbh / isoh / isol arrays MakeGraph builds on the host), built in LDS from
 // g's adjacency rows: entry by entry the same unions and intersections over
 // the bits of each chunk.  s_m from LowMasksShared.
-__device__ __forceinline__ void BuildTables(const DPGraph* __restrict__ g, const uint32_t* s_m,
+__device__ __forceinline__ void BuildTables(const DPHead* __restrict__ g, const uint32_t* s_m,
                                             uint32_t* s_tab) {
   const int n = static_cast<int>(g->n);
   for (int i = threadIdx.x; i < kTabWords; i += blockDim.x) {
@@ -402,7 +403,7 @@ __device__ __forceinline__ void BuildTables(const DPGraph* __restrict__ g, const
 
 template <int WB>
 __global__ __launch_bounds__(1024) void DPPersistentKernel(
-    const DPGraph* __restrict__ gs, const uint32_t* __restrict__ g_cb,
+    const DPHead* __restrict__ gs, const uint32_t* __restrict__ g_cb,
     uint8_t* __restrict__ arena, int ngraphs, uint32_t* __restrict__ queue,
     int R) {
   __shared__ uint32_t s_lvl[kLvlWords];
@@ -416,8 +417,7 @@ __global__ __launch_bounds__(1024) void DPPersistentKernel(
     __syncthreads();
     const int gi = s_gi;
     if (gi >= ngraphs) break;  // uniform: every thread read the same s_gi
-    const DPGraph* g = gs + gi;
-    // only the record's head (up to nbh) comes from the host
+    const DPHead* g = gs + gi;
     BuildTables(g, s_masks, s_tab);
     __syncthreads();
     const int nh = static_cast<int>(g->nh);
@@ -456,7 +456,7 @@ __global__ void ResetCounter(uint32_t* c) {
 // Binomials and the level offsets (read per lane, so LDS spares a memory
 // round trip before each table read).  Ends with a barrier.
 constexpr int kLookupWords = 34;
-__device__ __forceinline__ void LoadLookupTables(const DPGraph* __restrict__ g,
+__device__ __forceinline__ void LoadLookupTables(const DPHead* __restrict__ g,
                                                  const uint32_t* __restrict__ g_cb,
                                                  uint32_t* s_cb, uint32_t* s_base) {
   for (int i = threadIdx.x; i < 32 * kCbStride; i += blockDim.x) s_cb[i] = g_cb[i];
@@ -465,7 +465,7 @@ __device__ __forceinline__ void LoadLookupTables(const DPGraph* __restrict__ g,
 }
 
 // Gray code of td(S) mod 4 (bit v of S = vertex v) from the finished tables.
-__device__ __forceinline__ uint32_t LookupCode(const DPGraph* __restrict__ g,
+__device__ __forceinline__ uint32_t LookupCode(const DPHead* __restrict__ g,
                                                const uint8_t* __restrict__ arena,
                                                const uint32_t* s_cb, const uint32_t* s_base,
                                                uint32_t S) {
@@ -496,7 +496,7 @@ __device__ __forceinline__ uint32_t GrayValue(uint32_t code) { return code ^ (co
 // S is put together three vertices at a time, lowest first: one pass over its
 // vertices keeps the rank, the reads do not wait for each other, and the sets
 // of the lowest vertices are few and stay in the caches.
-__device__ __forceinline__ uint32_t LookupTd(const DPGraph* __restrict__ g,
+__device__ __forceinline__ uint32_t LookupTd(const DPHead* __restrict__ g,
                                              const uint8_t* __restrict__ arena,
                                              const uint32_t* s_cb, const uint32_t* s_base,
                                              uint32_t S) {
@@ -645,13 +645,14 @@ __device__ __forceinline__ int DecomposeWave(uint32_t myadj, uint32_t S, int* de
 
 // DecomposeWave for one whole graph per workgroup, from tables in memory.
 // parent_out: 64 int8 per graph; td_out: the tree's depth.
+template <typename Record>
 __global__ __launch_bounds__(64) void DPTreeKernel(
-    const DPGraph* __restrict__ gs, const uint32_t* __restrict__ g_cb,
+    const Record* __restrict__ gs, const uint32_t* __restrict__ g_cb,
     const uint8_t* __restrict__ arena, int8_t* __restrict__ parent_out,
     int32_t* __restrict__ td_out) {
   __shared__ uint32_t s_cb[32 * kCbStride];
   __shared__ uint32_t s_base[kLookupWords];
-  const DPGraph* g = gs + blockIdx.x;
+  const Record* g = gs + blockIdx.x;
   LoadLookupTables(g, g_cb, s_cb, s_base);
   const int lane = threadIdx.x;
   const uint32_t S = g->n >= 32 ? ~0u : (1u << g->n) - 1u;
@@ -715,14 +716,13 @@ int WordBits(int low_bits) { return low_bits >= 5 ? 2 : low_bits == 4 ? 1 : 0; }
 // Tile offsets of each high level, each level padded to a 128-byte boundary
 // of its plane so no cache line holds tiles of two levels.  Vertices n and
 // up, where a tile has more than n, count as isolated.
-DPGraph MakeGraph(int n, const uint64_t* adj, int wb, uint64_t table_off, bool tables = true) {
-  DPGraph G;
+DPHead MakeHead(int n, const uint64_t* adj, int wb) {
+  DPHead G;
   std::memset(&G, 0, sizeof(G));
   const int lb = 5 + wb;
   G.n = n;
   G.lb = lb;
   G.nh = n > lb ? n - lb : 0;
-  G.table = table_off;
   const uint32_t pad_tiles = 128u >> (lb - 3);
   uint64_t off = 0;
   for (uint32_t h = 0; h <= G.nh; ++h) {
@@ -732,7 +732,14 @@ DPGraph MakeGraph(int n, const uint64_t* adj, int wb, uint64_t table_off, bool t
   }
   G.lvl[G.nh + 1] = static_cast<uint32_t>(off);
   for (int v = 0; v < n; ++v) G.adj[v] = static_cast<uint32_t>(adj[v]);
-  if (!tables) return G;  // the persistent kernel builds them in LDS
+  return G;
+}
+
+// The head and the tables; without `tables`, the head only.
+DPGraph MakeGraph(int n, const uint64_t* adj, int wb, bool tables = true) {
+  DPGraph G;
+  static_cast<DPHead&>(G) = MakeHead(n, adj, wb);
+  if (!tables) return G;
   // N(chunk) = N(chunk without its lowest bit) | N(lowest bit), and the low
   // parts that give every vertex of the chunk a neighbour
   static const LowMasks M;
@@ -756,14 +763,14 @@ DPGraph MakeGraph(int n, const uint64_t* adj, int wb, uint64_t table_off, bool t
 }
 
 // Bytes of a graph's three planes.
-uint64_t TableBytes(const DPGraph& G) {
+uint64_t TableBytes(const DPHead& G) {
   return 3 * (static_cast<uint64_t>(G.lvl[G.nh + 1]) << (G.lb - 3));
 }
 
 // Bytes that a graph's table takes from the context's budget: one per subset,
 // though only 3/8 are used, or (dp.packed with dp.class_bits) 17/32, so that a
 // byte budget admits and refuses the same calls as with byte tables.
-uint64_t ClaimedBytes(const DPGraph& G, bool packed = false) {
+uint64_t ClaimedBytes(const DPHead& G, bool packed = false) {
   const uint64_t subsets = 1ull << G.n;
   return std::max(TableBytes(G), packed ? subsets / 2 + subsets / 32 : subsets);
 }
@@ -974,7 +981,7 @@ float Elapsed(hipEvent_t a, hipEvent_t b) {
 // n = 23: 92 / 97 / 108; n = 27: 168 / 170 / 180; n = 28: 236 / 227 / 233;
 // n = 29: 366 / 341 / 331; n = 30: 635 / 560 / 527.
 DPGraph SingleGraph(td_ctx* ctx, int n, const uint64_t* adj, bool tables = true) {
-  return MakeGraph(n, adj, std::min(WordBits(ctx->dp.low_bits), std::max(0, n - 27)), 0, tables);
+  return MakeGraph(n, adj, std::min(WordBits(ctx->dp.low_bits), std::max(0, n - 27)), tables);
 }
 
 // Whether the context claims a packed table's bytes for this graph.
@@ -1053,17 +1060,17 @@ uint8_t* FlowBuffer(td_ctx* ctx, size_t words) {
 }
 
 // The first of `count` graphs of kFlowMinN..kFlowMaxN vertices, largest first
-// (sizes at ns[i * stride]), as many as fit one launch of a workgroup per CU
+// (sizes in ns), as many as fit one launch of a workgroup per CU
 // (or one graph): the launch's classes.  *words and *planes receive the bytes
 // of published words and planes, *groups the workgroups; returns the graphs.
-int PlanFlow(const td_ctx* ctx, int count, const uint32_t* ns, size_t stride, FlowCall* f,
-             size_t* words, size_t* planes, uint32_t* groups) {
+int PlanFlow(const td_ctx* ctx, int count, const uint32_t* ns, FlowCall* f, size_t* words,
+             size_t* planes, uint32_t* groups) {
   *words = *planes = 0;
   *groups = 0;
   f->classes = 0;
   int i = 0;
   for (; i < count; ++i) {
-    const uint32_t n = ns[i * stride];
+    const uint32_t n = ns[i];
     const uint32_t more = 1u << FlowTop(static_cast<int>(n));
     if (i && *groups + more > static_cast<uint32_t>(ctx->prop.multiProcessorCount)) break;
     if (!f->classes || f->c[f->classes - 1].n != n)
@@ -1132,7 +1139,7 @@ void SolveOne(td_ctx* ctx, int n, const uint64_t* adj, uint8_t* td_out,
       FlowCall f;
       size_t words, planes;
       uint32_t groups;
-      PlanFlow(ctx, 1, &G.n, 1, &f, &words, &planes, &groups);
+      PlanFlow(ctx, 1, &G.n, &f, &words, &planes, &groups);
       std::memcpy(f.one.adj, G.adj, sizeof(f.one.adj));
       out->status = 0;
       LaunchFlow(ctx, f, 1, groups, nullptr, cb, arena, fbuf, out->parent, &out->td, &out->status,
@@ -1163,7 +1170,7 @@ void SolveOne(td_ctx* ctx, int n, const uint64_t* adj, uint8_t* td_out,
   TD_HIP(hipEventRecord(ctx->ev[0], ctx->stream));
   RunLevels(ctx, G, dG, cb, arena, &launches);
   TD_HIP(hipEventRecord(ctx->ev[1], ctx->stream));
-  hipLaunchKernelGGL(DPTreeKernel, dim3(1), dim3(64), 0, ctx->stream, dG, cb, arena,
+  hipLaunchKernelGGL(DPTreeKernel<DPGraph>, dim3(1), dim3(64), 0, ctx->stream, dG, cb, arena,
                      reinterpret_cast<int8_t*>(dtree), reinterpret_cast<int32_t*>(dtree + 64));
   TD_HIP(hipGetLastError());
   ++launches;
@@ -1186,7 +1193,7 @@ void SolveOne(td_ctx* ctx, int n, const uint64_t* adj, uint8_t* td_out,
 const DPGraph* LastRecord(td_ctx* ctx) {
   void* d = ctx->bufs["dp.graph"].p;
   if (!ctx->record_up) {
-    TD_HIP(hipMemcpyAsync(d, &ctx->last_graph, sizeof(DPGraph), hipMemcpyHostToDevice,
+    TD_HIP(hipMemcpyAsync(d, &ctx->last_graph, sizeof(DPHead), hipMemcpyHostToDevice,
                           ctx->stream));
     ctx->record_up = true;
   }
@@ -1254,7 +1261,7 @@ void SolveOneNoAlloc(td_ctx* ctx, int n, const uint64_t* adj, uint8_t* td_out,
   // direct launches: a captured graph would be instantiated (allocated) here
   LaunchLevelsLB(ctx, G, dG, cb, arena, &launches, ctx->stream, -1, 1);
   TD_HIP(hipEventRecord(ctx->ev[1], ctx->stream));
-  hipLaunchKernelGGL(DPTreeKernel, dim3(1), dim3(64), 0, ctx->stream, dG, cb, arena,
+  hipLaunchKernelGGL(DPTreeKernel<DPGraph>, dim3(1), dim3(64), 0, ctx->stream, dG, cb, arena,
                      reinterpret_cast<int8_t*>(dtree), reinterpret_cast<int32_t*>(dtree + 64));
   TD_HIP(hipGetLastError());
   ++launches;
@@ -1372,7 +1379,7 @@ void SolveLarge(td_ctx* ctx, const std::vector<int>& idx, const int32_t* ns,
       prev_split = split;
       *level_kernels += LevelKernelCount(G);
       TD_HIP(hipStreamWaitEvent(ctx->side, lv_end[s], 0));
-      hipLaunchKernelGGL(DPTreeKernel, dim3(1), dim3(64), 0, ctx->side, dG, cb, arena[s],
+      hipLaunchKernelGGL(DPTreeKernel<DPGraph>, dim3(1), dim3(64), 0, ctx->side, dG, cb, arena[s],
                          reinterpret_cast<int8_t*>(dtree[s]),
                          reinterpret_cast<int32_t*>(dtree[s] + 64));
       TD_HIP(hipGetLastError());
@@ -1407,49 +1414,56 @@ void SolveLarge(td_ctx* ctx, const std::vector<int>& idx, const int32_t* ns,
 }
 
 template <int WB>
+void LaunchPersistent(td_ctx* ctx, int ngraphs, const DPHead* dGs, const uint32_t* cb,
+                      uint8_t* arena, uint32_t* dqueue, uint64_t* launches) {
+  const int R = ctx->dp.tiles_per_lane;
+  // queue reset (a kernel, not a memset, so the pair can be captured) and
+  // the persistent launch, replayed from a hipGraph cached per batch shape
+  const int grid = ctx->prop.multiProcessorCount * ctx->dp.batch_wg_per_cu;
+  const int bblock = ctx->dp.batch_block;
+  auto launch = [&] {
+    hipLaunchKernelGGL(ResetCounter, dim3(1), dim3(64), 0, ctx->stream, dqueue);
+    hipLaunchKernelGGL(DPPersistentKernel<WB>, dim3(grid), dim3(bblock), 0,
+                       ctx->stream, dGs, cb, arena, ngraphs, dqueue, R);
+  };
+  if (!ctx->dp.use_graph) {
+    launch();
+    *launches += 2;
+  } else {
+    const td_ctx::GraphKey key{-ngraphs, WB, R, bblock * 64 + ctx->dp.batch_wg_per_cu};
+    const void* sig[3] = {arena, dGs, dqueue};
+    auto it = ctx->dp_graphs.find(key);
+    auto& p = ctx->dp_graph_ptrs[key];
+    if (it != ctx->dp_graphs.end() && (p.first != sig[0] || p.second != sig[1])) {
+      (void)hipGraphExecDestroy(it->second);
+      ctx->dp_graphs.erase(it);
+      it = ctx->dp_graphs.end();
+    }
+    if (it == ctx->dp_graphs.end()) {
+      hipGraph_t graph;
+      TD_HIP(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
+      launch();
+      TD_HIP(hipStreamEndCapture(ctx->stream, &graph));
+      hipGraphExec_t exec;
+      TD_HIP(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
+      (void)hipGraphDestroy(graph);
+      it = ctx->dp_graphs.emplace(key, exec).first;
+      p = {sig[0], sig[1]};
+    }
+    TD_HIP(hipGraphLaunch(it->second, ctx->stream));
+    *launches += 1;
+  }
+  TD_HIP(hipGetLastError());
+}
+
+// Modes 1 and 2 of a batch call.
+template <int WB>
 void LaunchBatch(td_ctx* ctx, int mode, int ngraphs,
                  const DPGraph* Gs, const DPGraph* dGs,
-                 const uint32_t* cb, uint8_t* arena, uint32_t* dqueue,
+                 const uint32_t* cb, uint8_t* arena,
                  uint64_t* launches) {
   const int R = ctx->dp.tiles_per_lane, block = ctx->dp.block;
-  if (mode == 0) {
-    // queue reset (a kernel, not a memset, so the pair can be captured) and
-    // the persistent launch, replayed from a hipGraph cached per batch shape
-    const int grid = ctx->prop.multiProcessorCount * ctx->dp.batch_wg_per_cu;
-    const int bblock = ctx->dp.batch_block;
-    auto launch = [&] {
-      hipLaunchKernelGGL(ResetCounter, dim3(1), dim3(64), 0, ctx->stream, dqueue);
-      hipLaunchKernelGGL(DPPersistentKernel<WB>, dim3(grid), dim3(bblock), 0,
-                         ctx->stream, dGs, cb, arena, ngraphs, dqueue, R);
-    };
-    if (!ctx->dp.use_graph) {
-      launch();
-      *launches += 2;
-    } else {
-      const td_ctx::GraphKey key{-ngraphs, WB, R, bblock * 64 + ctx->dp.batch_wg_per_cu};
-      const void* sig[3] = {arena, dGs, dqueue};
-      auto it = ctx->dp_graphs.find(key);
-      auto& p = ctx->dp_graph_ptrs[key];
-      if (it != ctx->dp_graphs.end() && (p.first != sig[0] || p.second != sig[1])) {
-        (void)hipGraphExecDestroy(it->second);
-        ctx->dp_graphs.erase(it);
-        it = ctx->dp_graphs.end();
-      }
-      if (it == ctx->dp_graphs.end()) {
-        hipGraph_t graph;
-        TD_HIP(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-        launch();
-        TD_HIP(hipStreamEndCapture(ctx->stream, &graph));
-        hipGraphExec_t exec;
-        TD_HIP(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
-        (void)hipGraphDestroy(graph);
-        it = ctx->dp_graphs.emplace(key, exec).first;
-        p = {sig[0], sig[1]};
-      }
-      TD_HIP(hipGraphLaunch(it->second, ctx->stream));
-      *launches += 1;
-    }
-  } else if (mode == 1) {
+  if (mode == 1) {
     int maxnh = 0;
     for (int i = 0; i < ngraphs; ++i) maxnh = std::max(maxnh, static_cast<int>(Gs[i].nh));
     const uint32_t chunk_tiles = static_cast<uint32_t>(block) * R * 2;
@@ -1555,11 +1569,22 @@ void SolveBatch(td_ctx* ctx, int ngraphs, const int32_t* ns,
   }
   // graphs above kMaxBatchN vertices go through the single-graph kernels;
   // the rest run largest first, so the persistent queue ends with short work
-  std::vector<int> large, perm;
-  for (int i = 0; i < ngraphs; ++i) (ns[i] > kMaxBatchN ? large : perm).push_back(i);
-  std::stable_sort(perm.begin(), perm.end(),
-                   [&](int a, int b) { return ns[a] > ns[b]; });
-  const int nsmall = static_cast<int>(perm.size());
+  std::vector<int> large;
+  int first[kMaxBatchN + 2] = {};  // first[n]: graphs of more than n vertices, <= kMaxBatchN
+  for (int i = 0; i < ngraphs; ++i) {
+    if (ns[i] > kMaxBatchN) large.push_back(i);
+    else ++first[ns[i] - 1];
+  }
+  for (int n = kMaxBatchN - 1; n >= 0; --n) first[n] += first[n + 1];
+  const int nsmall = first[0];
+  std::vector<int> perm(nsmall);
+  std::vector<uint32_t> sizes(nsmall);
+  for (int i = 0; i < ngraphs; ++i)
+    if (ns[i] <= kMaxBatchN) {
+      const int at = first[ns[i]]++;
+      perm[at] = i;
+      sizes[at] = static_cast<uint32_t>(ns[i]);
+    }
   // of these, mode 0 gives the last ones, of at most kLdsMaxN vertices, to
   // DPLdsKernel
   int nmid = nsmall;
@@ -1568,18 +1593,20 @@ void SolveBatch(td_ctx* ctx, int ngraphs, const int32_t* ns,
   int nbig = mode == 0 && FlowPays(ctx, nmid, ns, perm) ? 0 : nmid;
   // page-locked block of the small graphs' records and results; the kernels
   // write the results (and DPLdsKernel reads its graphs) there themselves
-  const size_t o_lds = sizeof(DPGraph) * nsmall;
+  const size_t record = mode == 0 ? sizeof(DPHead) : sizeof(DPGraph);
+  const size_t o_lds = record * nsmall;
   const size_t o_flow = o_lds + sizeof(LdsGraph) * (nsmall - nmid);
   const size_t o_par = (o_flow + sizeof(FlowGraph) * (nmid - nbig) + 63) / 64 * 64;
   const size_t o_td = o_par + 64ull * nsmall;
   uint8_t* block = static_cast<uint8_t*>(ctx->Pinned(o_td + 4ull * nsmall + 16, 1));
   int32_t* flow_status = reinterpret_cast<int32_t*>(block + o_td + 4ull * nsmall);
   *flow_status = 0;
-  DPGraph* Gs = reinterpret_cast<DPGraph*>(block);
+  DPGraph* Gs = reinterpret_cast<DPGraph*>(block);   // modes 1 and 2
+  DPHead* heads = reinterpret_cast<DPHead*>(block);  // mode 0
   LdsGraph* Ls = reinterpret_cast<LdsGraph*>(block + o_lds);
   FlowGraph* Fs = reinterpret_cast<FlowGraph*>(block + o_flow);
   // every graph is checked, and the small graphs' records are built, on the
-  // context's worker threads (about 0.3 us and 1 us a graph) before any GPU work;
+  // context's worker threads (about 0.3 us and 0.1 to 1 us a graph) before any GPU work;
   // a failure is reported for the lowest failing graph, as a serial check
   // would
   {
@@ -1596,12 +1623,18 @@ void SolveBatch(td_ctx* ctx, int ngraphs, const int32_t* ns,
       }
       for (int j = t; j < nsmall; j += T) {
         const int i = perm[j];
-        Gs[j] = MakeGraph(ns[i], adj_concat + row_off[i], WordBits(lb), 0, mode != 0);
-        if (j >= nmid) {
-          Ls[j - nmid].n = Gs[j].n;
-          std::memcpy(Ls[j - nmid].adj, Gs[j].adj, sizeof(Ls[0].adj));
-        } else if (j >= nbig) {
-          std::memcpy(Fs[j - nbig].adj, Gs[j].adj, sizeof(Fs[0].adj));
+        const uint64_t* rows = adj_concat + row_off[i];
+        if (mode != 0) {
+          Gs[j] = MakeGraph(ns[i], rows, WordBits(lb));
+        } else if (j < nmid) {
+          heads[j] = MakeHead(ns[i], rows, WordBits(lb));
+          if (j >= nbig)
+            for (int v = 0; v < kFlowMaxN; ++v) Fs[j - nbig].adj[v] = heads[j].adj[v];
+        } else {
+          LdsGraph& L = Ls[j - nmid];
+          L.n = sizes[j];
+          for (int v = 0; v < kLdsMaxN; ++v)
+            L.adj[v] = v < ns[i] ? static_cast<uint32_t>(rows[v]) : 0u;
         }
       }
     };
@@ -1645,15 +1678,25 @@ void SolveBatch(td_ctx* ctx, int ngraphs, const int32_t* ns,
     return;
   }
   ngraphs = nsmall;
+  // bytes used and claimed by a graph of n vertices
+  uint64_t used[kMaxBatchN + 1], claims[kMaxBatchN + 1];
+  const uint64_t none[kMaxBatchN] = {};
+  for (int n = 1; n <= kMaxBatchN; ++n) {
+    const DPHead H = MakeHead(n, none, WordBits(lb));
+    used[n] = (TableBytes(H) + 255) / 256 * 256;
+    claims[n] = (ClaimedBytes(H) + 255) / 256 * 256;
+  }
   uint64_t off = 0, claimed = 0;
+  auto place = [&](int j) {
+    (mode == 0 ? heads[j].table : Gs[j].table) = off;
+    off += used[sizes[j]];
+  };
   for (int j = 0; j < ngraphs; ++j) {
-    Gs[j].table = off;
-    if (j < nbig) off += (TableBytes(Gs[j]) + 255) / 256 * 256;
-    claimed += (ClaimedBytes(Gs[j]) + 255) / 256 * 256;
+    if (j < nbig) place(j);
+    claimed += claims[sizes[j]];
   }
   uint8_t* arena = static_cast<uint8_t*>(ctx->Buffer("dp.batch_arena", claimed));
-  DPGraph* dGs = static_cast<DPGraph*>(
-      ctx->Buffer("dp.batch_graphs", sizeof(DPGraph) * ngraphs));
+  void* drec = ctx->Buffer("dp.batch_graphs", sizeof(DPGraph) * ngraphs);
   const uint32_t* cb = PascalDevice(ctx);
   uint32_t* dq = static_cast<uint32_t*>(ctx->Buffer("dp.batch_queue", 256));
   int8_t* par = reinterpret_cast<int8_t*>(block + o_par);
@@ -1667,42 +1710,38 @@ void SolveBatch(td_ctx* ctx, int ngraphs, const int32_t* ns,
     // the first launch holds the largest graphs, but later ones more of them
     size_t most = 0;
     for (int j = nbig; j < nmid;) {
-      j += PlanFlow(ctx, nmid - j, &Gs[j].n, sizeof(DPGraph) / 4, &flow, &flow_words,
-                    &flow_planes, &flow_groups);
+      j += PlanFlow(ctx, nmid - j, &sizes[j], &flow, &flow_words, &flow_planes, &flow_groups);
       most = std::max(most, flow_words);
     }
     fbuf = FlowBuffer(ctx, most);
   }
   if (!fbuf) {
-    for (int j = nbig; j < nmid; ++j) {
-      Gs[j].table = off;
-      off += (TableBytes(Gs[j]) + 255) / 256 * 256;
-    }
+    for (int j = nbig; j < nmid; ++j) place(j);
     nbig = nmid;
   }
-  if (mode == 0) {
-    // the persistent kernel reads only each record's head and builds the
-    // tables itself: 288 of the 4512 bytes per graph go up
-    constexpr size_t kHead = offsetof(DPGraph, nbh);
-    if (nbig > 0)
-      TD_HIP(hipMemcpy2DAsync(dGs, sizeof(DPGraph), Gs, sizeof(DPGraph), kHead, nbig,
-                              hipMemcpyHostToDevice, ctx->stream));
-  } else {
-    TD_HIP(hipMemcpyAsync(dGs, Gs, sizeof(DPGraph) * ngraphs, hipMemcpyHostToDevice,
-                          ctx->stream));
-  }
+  if (nbig > 0)
+    TD_HIP(hipMemcpyAsync(drec, block, record * nbig, hipMemcpyHostToDevice, ctx->stream));
   uint64_t small_launches = 0;
   TD_HIP(hipEventRecord(ctx->ev[0], ctx->stream));
   if (nbig > 0) {
+    auto launch = [&](auto wb) {
+      constexpr int WB = decltype(wb)::value;
+      if (mode == 0)
+        LaunchPersistent<WB>(ctx, nbig, static_cast<const DPHead*>(drec), cb, arena, dq,
+                             &small_launches);
+      else
+        LaunchBatch<WB>(ctx, mode, nbig, Gs, static_cast<const DPGraph*>(drec), cb, arena,
+                        &small_launches);
+    };
     switch (WordBits(lb)) {
-      case 0: LaunchBatch<0>(ctx, mode, nbig, Gs, dGs, cb, arena, dq, &small_launches); break;
-      case 1: LaunchBatch<1>(ctx, mode, nbig, Gs, dGs, cb, arena, dq, &small_launches); break;
-      default: LaunchBatch<2>(ctx, mode, nbig, Gs, dGs, cb, arena, dq, &small_launches); break;
+      case 0: launch(std::integral_constant<int, 0>()); break;
+      case 1: launch(std::integral_constant<int, 1>()); break;
+      default: launch(std::integral_constant<int, 2>()); break;
     }
   }
   for (int j = nbig; j < nmid;) {
-    const int k = PlanFlow(ctx, nmid - j, &Gs[j].n, sizeof(DPGraph) / 4, &flow, &flow_words,
-                           &flow_planes, &flow_groups);
+    const int k = PlanFlow(ctx, nmid - j, &sizes[j], &flow, &flow_words, &flow_planes,
+                           &flow_groups);
     LaunchFlow(ctx, flow, k, flow_groups, Fs + (j - nbig), cb, arena + off, fbuf, par + 64ull * j,
                tds + j, flow_status, nullptr);
     off += (flow_planes + 255) / 256 * 256;
@@ -1716,8 +1755,12 @@ void SolveBatch(td_ctx* ctx, int ngraphs, const int32_t* ns,
   // else the launches
   level_kernels += mode == 0 ? 1 : small_launches;
   if (nbig > 0) {
-    hipLaunchKernelGGL(DPTreeKernel, dim3(nbig), dim3(64), 0, ctx->stream, dGs, cb, arena, par,
-                       tds);
+    if (mode == 0)
+      hipLaunchKernelGGL(DPTreeKernel<DPHead>, dim3(nbig), dim3(64), 0, ctx->stream,
+                         static_cast<const DPHead*>(drec), cb, arena, par, tds);
+    else
+      hipLaunchKernelGGL(DPTreeKernel<DPGraph>, dim3(nbig), dim3(64), 0, ctx->stream,
+                         static_cast<const DPGraph*>(drec), cb, arena, par, tds);
     TD_HIP(hipGetLastError());
     ++launches;
   }

@@ -1528,8 +1528,8 @@ bool FlowPays(const td_ctx* ctx, int count, const int32_t* ns, const std::vector
 // More graphs than CUs go in one launch per workgroup size, so that small
 // graphs do not hold the LDS and threads of large ones; fewer fit in one
 // launch, a CU each.
-uint64_t LaunchLdsBatch(td_ctx* ctx, int count, const LdsGraph* Ls, const uint32_t* cb,
-                        int8_t* parents, int32_t* tds) {
+uint64_t LaunchLdsBatch(td_ctx* ctx, hipStream_t st, int count, const LdsGraph* Ls,
+                        const uint32_t* cb, int8_t* parents, int32_t* tds) {
   uint64_t launches = 0;
   for (int at = 0; at < count;) {
     const int n = static_cast<int>(Ls[at].n), threads = LdsThreads(n);
@@ -1537,7 +1537,7 @@ uint64_t LaunchLdsBatch(td_ctx* ctx, int count, const LdsGraph* Ls, const uint32
     while (end < count && (count <= ctx->prop.multiProcessorCount ||
                            LdsThreads(static_cast<int>(Ls[end].n)) == threads))
       ++end;
-    hipLaunchKernelGGL(DPLdsKernel, dim3(end - at), dim3(threads), LdsBytes(n), ctx->stream,
+    hipLaunchKernelGGL(DPLdsKernel, dim3(end - at), dim3(threads), LdsBytes(n), st,
                        Ls + at, LdsGraph{}, cb, static_cast<uint32_t*>(nullptr),
                        parents + 64ull * at, tds + at,
                        static_cast<unsigned long long*>(nullptr));
@@ -1723,6 +1723,27 @@ void SolveBatch(td_ctx* ctx, int ngraphs, const int32_t* ns,
     TD_HIP(hipMemcpyAsync(drec, block, record * nbig, hipMemcpyHostToDevice, ctx->stream));
   uint64_t small_launches = 0;
   TD_HIP(hipEventRecord(ctx->ev[0], ctx->stream));
+  // Beside a persistent launch the graphs in LDS run on a stream of their own,
+  // started first: the persistent workgroups take what room they leave, and
+  // share the rest out by their queue (4096 graphs of 12..24 vertices: 3.48 ms
+  // instead of 3.61 one after the other).
+  hipStream_t lds_stream = ctx->stream;
+  struct Drain {  // the kernels write to the block: none may outlive an error
+    hipStream_t a, b;
+    ~Drain() {
+      if (a) (void)hipStreamSynchronize(a);
+      if (b) (void)hipStreamSynchronize(b);
+    }
+  } drain{ctx->stream, nullptr};
+  if (nmid < nsmall) {
+    if (nbig > 0) {
+      if (!ctx->side) TD_HIP(hipStreamCreateWithFlags(&ctx->side, hipStreamNonBlocking));
+      drain.b = lds_stream = ctx->side;
+    }
+    small_launches += LaunchLdsBatch(ctx, lds_stream, nsmall - nmid, Ls, cb, par + 64ull * nmid,
+                                     tds + nmid);
+    if (lds_stream != ctx->stream) TD_HIP(hipEventRecord(ctx->ev[3], lds_stream));
+  }
   if (nbig > 0) {
     auto launch = [&](auto wb) {
       constexpr int WB = decltype(wb)::value;
@@ -1748,8 +1769,7 @@ void SolveBatch(td_ctx* ctx, int ngraphs, const int32_t* ns,
     small_launches += 2;
     j += k;
   }
-  if (nmid < nsmall)
-    small_launches += LaunchLdsBatch(ctx, nsmall - nmid, Ls, cb, par + 64ull * nmid, tds + nmid);
+  if (lds_stream != ctx->stream) TD_HIP(hipStreamWaitEvent(ctx->stream, ctx->ev[3], 0));
   TD_HIP(hipEventRecord(ctx->ev[1], ctx->stream));
   // mode 0 counts as one level kernel however its graphs were shared out;
   // else the launches
@@ -1767,6 +1787,7 @@ void SolveBatch(td_ctx* ctx, int ngraphs, const int32_t* ns,
   launches += small_launches;
   TD_HIP(hipEventRecord(ctx->ev[2], ctx->stream));
   TD_HIP(hipStreamSynchronize(ctx->stream));
+  drain.a = drain.b = nullptr;
   // a wait was given up: those graphs one by one (SolveOne falls back itself)
   if (*flow_status)
     for (int j = nbig; j < nmid; ++j) {

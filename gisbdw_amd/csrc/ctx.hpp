@@ -65,6 +65,17 @@ constexpr int kTabNbh = 0, kTabIsoH = 512, kTabIsoL = 1024, kTabWords = 1056;
 static_assert(sizeof(DPGraph) == sizeof(DPHead) + 4 * kTabWords,
               "nbh, isoh and isol must follow each other and the head");
 
+// Whether row v of a graph of n vertices is one that ValidateGraph takes: no
+// vertex n or above, no self loop, and (rows[u] for every neighbour u < 64)
+// symmetric.  A row v >= n has to be empty.
+__device__ __forceinline__ bool RowFine(const uint64_t* rows, uint64_t row, int n, int v) {
+  if (v >= n) return row == 0ull;
+  if ((n < 64 && row >> n) || (row >> v & 1ull)) return false;
+  bool ok = true;
+  for (uint64_t m = row; m; m &= m - 1) ok = ok && (rows[__builtin_ctzll(m)] >> v & 1ull);
+  return ok;
+}
+
 // DP launch configuration (autotuned).
 struct DPConfig {
   int low_bits = 4;        // 2..5: tiles of 1, 1, 2 or 4 words

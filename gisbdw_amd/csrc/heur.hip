@@ -16,6 +16,7 @@
 // whose elimination created v's component.  The Variance score is computed
 // in the reference's arithmetic: double sums and square root, float E times
 // the component count, no fused multiply-add.
+#include <algorithm>
 #include <cstring>
 #include <vector>
 
@@ -28,6 +29,12 @@ constexpr int kMaxHeurN = 64;
 
 __device__ __forceinline__ uint64_t HBallot(bool p) {
   return static_cast<uint64_t>(__ballot(p));
+}
+
+// LDS written by a wave's lanes is read by its other lanes after this
+__device__ __forceinline__ void WaveSync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
 }
 
 // component of `from` inside X by ballot BFS (lane u holds row u)
@@ -100,8 +107,19 @@ __device__ double VarianceCoef(uint64_t C, int p, const uint64_t* s_adj, uint8_t
   while (rest) {
     uint64_t comp = rest & (0ull - rest), front = comp;
     while (front) {
-      uint64_t nb = 0;
-      for (uint64_t f = front; f; f &= f - 1) nb |= s_adj[__builtin_ctzll(f)];
+      // four rows at a time, so that their reads are in flight together
+      uint64_t nb = 0, f = front;
+      while (f) {
+        const int a = __builtin_ctzll(f);
+        f &= f - 1;
+        const int b = f ? __builtin_ctzll(f) : a;
+        f &= f - 1;
+        const int c = f ? __builtin_ctzll(f) : a;
+        f &= f - 1;
+        const int d = f ? __builtin_ctzll(f) : a;
+        f &= f - 1;
+        nb |= (s_adj[a] | s_adj[b]) | (s_adj[c] | s_adj[d]);
+      }
       nb &= rest & ~comp;
       comp |= nb;
       front = nb;
@@ -199,7 +217,7 @@ __device__ void SpanningForest(const uint64_t* s_adj, int n, uint64_t* s_st, int
   const int lane = threadIdx.x & 63;
   s_st[lane] = 0ull;
   s_uf[lane] = lane;
-  __syncthreads();
+  WaveSync();
   if (lane == 0) {
     for (int i = 0; i < n; ++i) {
       for (uint64_t m = s_adj[i] & ~((2ull << i) - 1ull); m; m &= m - 1) {
@@ -215,92 +233,68 @@ __device__ void SpanningForest(const uint64_t* s_adj, int n, uint64_t* s_st, int
       }
     }
   }
-  __syncthreads();
+  WaveSync();
 }
 
-struct HeurTree {
-  int td;
-  int8_t parent[64];
-};
-
 // kind: 1 = HighestDegree(SpanningTree(Variance(1.0, 0.2, 0.8))), 2 =
-// HighestDegree, 3 = SpanningTree, 4 = Variance(1.0, 0.2, 0.8).
-__global__ __launch_bounds__(64) void HeuristicKernel(const int32_t* __restrict__ ns,
-                                                      const uint64_t* __restrict__ adj64,
-                                                      int kind,
-                                                      const int32_t* __restrict__ inner_td,
-                                                      const int8_t* __restrict__ inner_par,
-                                                      int32_t* __restrict__ td_out,
-                                                      int8_t* __restrict__ parent_out) {
+// HighestDegree, 3 = SpanningTree, 4 = Variance(1.0, 0.2, 0.8), 5 and 6 the
+// chains over an inner result.
+//
+// One graph per workgroup, a wave for each heuristic of a chain: they do not
+// depend on each other, each is a chain of dependent LDS reads and ballots,
+// and a wave by itself leaves its SIMD idle for most of it.  The decorators
+// then compare the three trees.  Rows come from page-locked host memory (read
+// once) and are checked here; a graph that is not valid sets status and is
+// left out.  1024 sparse graphs of 40..64 vertices: see the launch.
+__global__ __launch_bounds__(192) void HeuristicKernel(
+    const int32_t* __restrict__ ns, const uint32_t* __restrict__ offs,
+    const uint64_t* __restrict__ rows, int kind, const int32_t* __restrict__ inner_td,
+    const int8_t* __restrict__ inner_par, int32_t* __restrict__ td_out,
+    int8_t* __restrict__ parent_out, int32_t* __restrict__ status) {
   __shared__ uint64_t s_adj[64], s_st[64];
-  __shared__ int s_uf[64];
+  __shared__ int s_uf[64], s_td[3];
   __shared__ uint8_t s_sizes[64 * 64];
-  __shared__ int8_t s_par[4][64];
-  const int gi = blockIdx.x, lane = threadIdx.x;
+  __shared__ int8_t s_par[3][64];
+  const int gi = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int n = ns[gi];
-  const uint64_t row = lane < n ? adj64[static_cast<size_t>(gi) * 64 + lane] : 0ull;
-  s_adj[lane] = row;
+  if (wave == 0) s_adj[lane] = lane < n ? rows[offs[gi] + lane] : 0ull;
   __syncthreads();
+  const uint64_t row = s_adj[lane];
+  const bool bad = __ballot(!RowFine(s_adj, row, n, lane)) != 0ull;  // in every wave alike
+  if (threadIdx.x == 0) status[gi] = bad ? 1 : 0;
+  if (bad) return;
+  // tree 0: Variance, 1: SpanningTree, 2: HighestDegree; -1 where the kind has none
   const float A = 1.0f, D = 0.2f, E = 0.8f;
-  int td = 0;
-  int8_t* out = s_par[0];
-  if (kind == 2) {
-    td = HighestDegree(row, n, s_par[0]);
-  } else if (kind == 3) {
-    SpanningForest(s_adj, n, s_st, s_uf);
-    td = SpanningTree(row, n, s_st, s_par[0]);
-  } else if (kind == 4) {
-    td = Variance(row, n, s_adj, s_sizes, A, D, E, s_par[0]);
-  } else if (kind == 6) {
-    // HighestDegree(Variance(inner)): decorators keep the inner result only
-    // when strictly shallower; a missing inner result (-1) never is
-    int tv = Variance(row, n, s_adj, s_sizes, A, D, E, s_par[0]);
-    int8_t* vt = s_par[0];
-    const int ti = inner_td[gi];
-    if (ti >= 0 && ti < tv) {
-      tv = ti;
-      s_par[3][lane] = lane < n ? inner_par[static_cast<size_t>(gi) * 64 + lane] : -1;
-      vt = s_par[3];
-    }
-    __syncthreads();
-    const int th = HighestDegree(row, n, s_par[2]);
-    td = th;
-    out = s_par[2];
-    if (tv < th) {
-      td = tv;
-      out = vt;
+  int td = -1;
+  if (wave == 0) {
+    if (kind != 2 && kind != 3) td = Variance(row, n, s_adj, s_sizes, A, D, E, s_par[0]);
+  } else if (wave == 1) {
+    if (kind == 1 || kind == 3 || kind == 5) {
+      SpanningForest(s_adj, n, s_st, s_uf);
+      td = SpanningTree(row, n, s_st, s_par[1]);
     }
   } else {
-    // kind 1: HighestDegree(SpanningTree(Variance)); kind 5: the same over an
-    // inner result.  Decorators keep the inner result only when strictly
-    // shallower.
-    int tv = Variance(row, n, s_adj, s_sizes, A, D, E, s_par[0]);
-    if (kind == 5) {
-      const int ti = inner_td[gi];
-      if (ti >= 0 && ti < tv) {
-        tv = ti;
-        s_par[0][lane] = lane < n ? inner_par[static_cast<size_t>(gi) * 64 + lane] : -1;
-      }
-      __syncthreads();
-    }
-    SpanningForest(s_adj, n, s_st, s_uf);
-    int ts = SpanningTree(row, n, s_st, s_par[1]);
-    int8_t* st = s_par[1];
-    if (tv < ts) {
-      ts = tv;
-      st = s_par[0];
-    }
-    const int th = HighestDegree(row, n, s_par[2]);
-    td = th;
-    out = s_par[2];
-    if (ts < th) {
-      td = ts;
-      out = st;
-    }
+    if (kind != 3 && kind != 4) td = HighestDegree(row, n, s_par[2]);
   }
+  if (lane == 0) s_td[wave] = td;
   __syncthreads();
-  if (lane < n) parent_out[static_cast<size_t>(gi) * 64 + lane] = out[lane];
-  if (lane == 0) td_out[gi] = td;
+  if (wave) return;
+  // decorators keep the inner result only when it is strictly shallower; a
+  // missing inner result (-1) never is
+  int best = s_td[0];
+  int8_t parent = s_par[0][lane];
+  if (kind >= 5 && inner_td[gi] >= 0 && inner_td[gi] < best) {
+    best = inner_td[gi];
+    parent = lane < n ? inner_par[static_cast<size_t>(gi) * 64 + lane] : -1;
+  }
+#pragma unroll
+  for (int w = 1; w < 3; ++w)
+    if (s_td[w] >= 0 && !(best >= 0 && best < s_td[w])) {
+      best = s_td[w];
+      parent = s_par[w][lane];
+    }
+  if (lane < n) parent_out[static_cast<size_t>(gi) * 64 + lane] = parent;
+  if (lane == 0) td_out[gi] = best;
 }
 
 template <typename F>
@@ -339,25 +333,20 @@ int td_heuristic_batch(td_ctx* ctx, int32_t ngraphs, const int32_t* n,
       TD_REQUIRE(n[i] >= 1 && n[i] <= kMaxHeurN, TD_E_INVALID, "graphs need n in [1, 64]");
       off[i + 1] = off[i] + static_cast<size_t>(n[i]);
     }
-    std::vector<uint64_t> rows(static_cast<size_t>(ngraphs) * 64, 0ull);
-    for (int i = 0; i < ngraphs; ++i) {
-      ValidateGraph(n[i], adj_concat + off[i], kMaxHeurN);
-      std::memcpy(rows.data() + static_cast<size_t>(i) * 64, adj_concat + off[i],
-                  sizeof(uint64_t) * n[i]);
-    }
-    auto* dn = static_cast<int32_t*>(ctx->Buffer("heur.n", 4ull * ngraphs));
-    auto* dadj = static_cast<uint64_t*>(ctx->Buffer("heur.adj", rows.size() * 8));
-    auto* dtd = static_cast<int32_t*>(ctx->Buffer("heur.td", 4ull * ngraphs));
-    auto* dpar = static_cast<int8_t*>(ctx->Buffer("heur.parent", 64ull * ngraphs));
-    TD_HIP(hipMemcpyAsync(dn, n, 4ull * ngraphs, hipMemcpyHostToDevice, ctx->stream));
-    TD_HIP(hipMemcpyAsync(dadj, rows.data(), rows.size() * 8, hipMemcpyHostToDevice,
-                          ctx->stream));
+    auto check = [&] {
+      for (int i = 0; i < ngraphs; ++i) ValidateGraph(n[i], adj_concat + off[i], kMaxHeurN);
+    };
     // kinds 5 and 6: the bottom-up heuristic is the innermost link; it runs
     // for graphs of at most 32 vertices (a larger graph's levels never fit,
     // so the reference's link returns UINT_MAX there)
-    std::vector<int32_t> itd(static_cast<size_t>(ngraphs), -1);
-    std::vector<int8_t> ipar(kind >= 5 ? 64ull * ngraphs : 1, -1);
+    int32_t* ditd = nullptr;
+    int8_t* dipar = nullptr;
+    constexpr int kChunk = 4096;
+    // (a call of several chunks must not write results ahead of an error)
+    if (kind >= 5 || ngraphs > kChunk) check();
     if (kind >= 5) {
+      std::vector<int32_t> itd(static_cast<size_t>(ngraphs), -1);
+      std::vector<int8_t> ipar(64ull * ngraphs, -1);
       for (int i = 0; i < ngraphs; ++i) {
         if (n[i] > 32) continue;
         int32_t t = -1;
@@ -366,21 +355,48 @@ int td_heuristic_batch(td_ctx* ctx, int32_t ngraphs, const int32_t* n,
         if (rc != TD_OK) throw Error{rc, ctx->err};
         itd[i] = t;
       }
+      ditd = static_cast<int32_t*>(ctx->Buffer("heur.inner_td", 4ull * ngraphs));
+      dipar = static_cast<int8_t*>(ctx->Buffer("heur.inner_parent", ipar.size()));
+      TD_HIP(hipMemcpyAsync(ditd, itd.data(), 4ull * ngraphs, hipMemcpyHostToDevice,
+                            ctx->stream));
+      TD_HIP(hipMemcpyAsync(dipar, ipar.data(), ipar.size(), hipMemcpyHostToDevice, ctx->stream));
+      TD_HIP(hipStreamSynchronize(ctx->stream));
     }
-    auto* ditd = static_cast<int32_t*>(ctx->Buffer("heur.inner_td", 4ull * ngraphs));
-    auto* dipar = static_cast<int8_t*>(ctx->Buffer("heur.inner_parent", ipar.size()));
-    TD_HIP(hipMemcpyAsync(ditd, itd.data(), 4ull * ngraphs, hipMemcpyHostToDevice, ctx->stream));
-    TD_HIP(hipMemcpyAsync(dipar, ipar.data(), ipar.size(), hipMemcpyHostToDevice, ctx->stream));
-    hipLaunchKernelGGL(HeuristicKernel, dim3(ngraphs), dim3(64), 0, ctx->stream, dn, dadj,
-                       kind, ditd, dipar, dtd, dpar);
-    TD_HIP(hipGetLastError());
-    std::vector<int8_t> par(64ull * ngraphs);
-    TD_HIP(hipMemcpyAsync(td_out, dtd, 4ull * ngraphs, hipMemcpyDeviceToHost, ctx->stream));
-    TD_HIP(hipMemcpyAsync(par.data(), dpar, par.size(), hipMemcpyDeviceToHost, ctx->stream));
-    TD_HIP(hipStreamSynchronize(ctx->stream));
-    if (parent_concat)
-      for (int i = 0; i < ngraphs; ++i)
-        std::memcpy(parent_concat + off[i], par.data() + 64ull * i, n[i]);
+    // Graphs, status and results in page-locked memory, kChunk graphs at a
+    // time.  1024 sparse graphs of 40..64 vertices: 650 us a call with checks
+    // and pageable copies on the host and one wave per graph (kernel 330),
+    // 248 now (kernel 224, its rows over PCIe included).
+    const size_t most = static_cast<size_t>(std::min(ngraphs, kChunk));
+    size_t most_rows = 0;
+    for (int at = 0; at < ngraphs; at += kChunk)
+      most_rows = std::max(most_rows, off[std::min(ngraphs, at + kChunk)] - off[at]);
+    uint8_t* p = static_cast<uint8_t*>(ctx->Pinned(8 * most_rows + (16 + 64) * most));
+    uint64_t* prows = reinterpret_cast<uint64_t*>(p);
+    int32_t* pn = reinterpret_cast<int32_t*>(prows + most_rows);
+    uint32_t* poff = reinterpret_cast<uint32_t*>(pn + most);
+    int32_t* ptd = reinterpret_cast<int32_t*>(poff + most);
+    int32_t* pstatus = ptd + most;
+    int8_t* ppar = reinterpret_cast<int8_t*>(pstatus + most);
+    for (int at = 0; at < ngraphs; at += kChunk) {
+      const int c = std::min(ngraphs - at, kChunk);
+      std::memcpy(prows, adj_concat + off[at], 8 * (off[at + c] - off[at]));
+      std::memcpy(pn, n + at, 4ull * c);
+      for (int i = 0; i < c; ++i) poff[i] = static_cast<uint32_t>(off[at + i] - off[at]);
+      hipLaunchKernelGGL(HeuristicKernel, dim3(c), dim3(192), 0, ctx->stream, pn, poff, prows,
+                         kind, ditd ? ditd + at : nullptr,
+                         dipar ? dipar + 64ull * at : nullptr, ptd, ppar, pstatus);
+      TD_HIP(hipGetLastError());
+      TD_HIP(hipStreamSynchronize(ctx->stream));
+      for (int i = 0; i < c; ++i)
+        if (pstatus[i]) {
+          check();  // throws the first error
+          throw Error{TD_E_INVALID, "invalid graph"};
+        }
+      std::memcpy(td_out + at, ptd, 4ull * c);
+      if (parent_concat)
+        for (int i = 0; i < c; ++i)
+          std::memcpy(parent_concat + off[at + i], ppar + 64ull * i, n[at + i]);
+    }
   });
 }
 

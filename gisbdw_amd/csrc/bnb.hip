@@ -39,6 +39,15 @@ namespace {
 constexpr int kMaxBnBN = 64;
 constexpr int kTagWord = 16;  // queue word holding the memo tag base (own 64 bytes)
 constexpr int kStack = 72;  // Feasible(C, k) nests at most k + 1 <= 65 frames
+// A graph of at most kFinishMaxN vertices that kFinishNodes search nodes have
+// not settled is finished by the subset DP, where the node budget is above
+// kFinishBudget (or 0, none).  The DP's 2^n subsets cost the same whatever the
+// graph: 30 us on one CU for n = 18, 95 us on the device for n = 24, what a
+// workgroup of 16 waves spends on 100 to 400 nodes, while a refutation on 20
+// vertices of a random cubic graph takes 3e5 nodes (80 ms).  Past 1024 nodes
+// (0.3 ms) the search is the worse bet.
+constexpr int kFinishMaxN = 24;
+constexpr uint64_t kFinishNodes = 1024, kFinishBudget = 32768;
 constexpr uint32_t kBudgetChunk = 64;  // search nodes a wave takes from its graph's budget at once
 
 struct BnBGraph {
@@ -1027,8 +1036,8 @@ __host__ __device__ constexpr size_t WaveLds(int dp_small) {
 __global__ __launch_bounds__(64 * kMaxWaves)
 __attribute__((amdgpu_waves_per_eu(6, 6))) void BnBKernel(
     const BnBGraph* __restrict__ gs, BnBOut* __restrict__ outs,
-    uint4* __restrict__ memo_base, int memo_log2, uint64_t node_budget, int dp_small,
-    int ngraphs, uint32_t* __restrict__ queue) {
+    uint4* __restrict__ memo_base, int memo_log2, uint64_t node_budget, uint64_t small_budget,
+    int dp_small, int ngraphs, uint32_t* __restrict__ queue) {
   // queue[0]: the next graph; queue[kTagWord]: this call's memo tag base,
   // written before the launch (a captured launch replays with new tags)
   const uint32_t tag_base = queue[kTagWord];
@@ -1078,7 +1087,7 @@ __attribute__((amdgpu_waves_per_eu(6, 6))) void BnBKernel(
     S.nodes = 0;
     S.hits = 0;
     // the node budget is per graph; the waves draw on it in chunks
-    S.budget = node_budget;
+    S.budget = n <= kFinishMaxN ? small_budget : node_budget;
     S.pool = &s_pool;
     S.left = 0;
     S.aborted = false;
@@ -1322,7 +1331,85 @@ int64_t Param(td_ctx* ctx, const char* k, int64_t dflt) {
 
 void SolveBnBSearch(td_ctx* ctx, int ngraphs, const int32_t* ns, const uint64_t* adj_concat,
                     const int32_t* ub_seed, const float* scores, uint8_t* td_out,
-                    int8_t* parent_concat, uint8_t* certified_out, td_bnb_stats* stats) {
+                    int8_t* parent_concat, uint8_t* certified_out, td_bnb_stats* stats,
+                    bool finish = true);
+
+// The graphs of at most kFinishMaxN vertices that the search has left
+// uncertified, by the subset DP (whose single-solve tables and queries stay
+// as they are), in calls of at most 2^30 subsets; where the device or the
+// byte budget has no room for that, by the search without its early stop.
+void FinishSmall(td_ctx* ctx, const int32_t* ns, const uint64_t* adj_concat,
+                 const std::vector<size_t>& off, const int32_t* ub_seed, const float* scores,
+                 std::vector<BnBOut>& out, double* ms) {
+  auto arena = ctx->bufs.find("dp.batch_arena");
+  const bool held = arena != ctx->bufs.end() && arena->second.p;
+  std::vector<int> left;
+  for (size_t i = 0; i < out.size(); ++i)
+    if (ns[i] <= kFinishMaxN && !out[i].certified) left.push_back(static_cast<int>(i));
+  for (size_t at = 0; at < left.size();) {
+    std::vector<int32_t> n, seed;
+    std::vector<uint64_t> adj;
+    std::vector<float> score;
+    uint64_t subsets = 0;
+    size_t end = at;
+    for (; end < left.size(); ++end) {
+      const int i = left[end];
+      if (end > at && subsets + (1ull << ns[i]) > (1ull << 30)) break;
+      subsets += 1ull << ns[i];
+      n.push_back(ns[i]);
+      adj.insert(adj.end(), adj_concat + off[i], adj_concat + off[i + 1]);
+      seed.push_back(ub_seed ? ub_seed[i] : 0);
+      if (scores) score.insert(score.end(), scores + off[i], scores + off[i + 1]);
+    }
+    const int count = static_cast<int>(n.size());
+    std::vector<uint8_t> td(count);
+    std::vector<int8_t> par(adj.size());
+    td_dp_stats st{};
+    const int rc = KeepDP(ctx, [&] {
+      return td_dp_solve_batch(ctx, count, n.data(), adj.data(), td.data(), par.data(), 0, &st);
+    });
+    if (rc == TD_OK) {
+      *ms += st.level_ms + st.tree_ms;
+      size_t r = 0;
+      for (int j = 0; j < count; ++j) {
+        BnBOut& o = out[left[at + j]];
+        o.td = o.lb = td[j];
+        o.certified = 1;
+        std::memcpy(o.parent, par.data() + r, n[j]);
+        r += n[j];
+      }
+    } else {
+      TD_REQUIRE(rc == TD_E_NOMEM, rc, ctx->err);
+      std::vector<uint8_t> cert(count);
+      td_bnb_stats bst{};
+      SolveBnBSearch(ctx, count, n.data(), adj.data(), ub_seed ? seed.data() : nullptr,
+                     scores ? score.data() : nullptr, td.data(), par.data(), cert.data(), &bst,
+                     false);
+      *ms += bst.kernel_ms;
+      size_t r = 0;
+      for (int j = 0; j < count; ++j) {
+        BnBOut& o = out[left[at + j]];
+        const td_ctx::BnBDetail& d = ctx->bnb_last[j];
+        o.td = td[j];
+        o.lb = d.lb;
+        o.certified = cert[j];
+        o.nodes += d.nodes;
+        o.last_k = d.last_k;
+        o.last_nodes = d.last_nodes;
+        std::memcpy(o.parent, par.data() + r, n[j]);
+        r += n[j];
+      }
+    }
+    at = end;
+  }
+  // a byte budget is the caller's to spend on other calls
+  if (ctx->budget && !held && !left.empty()) ctx->Release("dp.batch_arena");
+}
+
+void SolveBnBSearch(td_ctx* ctx, int ngraphs, const int32_t* ns, const uint64_t* adj_concat,
+                    const int32_t* ub_seed, const float* scores, uint8_t* td_out,
+                    int8_t* parent_concat, uint8_t* certified_out, td_bnb_stats* stats,
+                    bool finish) {
   const auto t0 = std::chrono::steady_clock::now();
   TD_REQUIRE(ngraphs >= 1 && ns && adj_concat, TD_E_INVALID, "empty batch or null pointer");
   std::vector<size_t> off(ngraphs + 1, 0);
@@ -1344,6 +1431,8 @@ void SolveBnBSearch(td_ctx* ctx, int ngraphs, const int32_t* ns, const uint64_t*
     }
   }
   const uint64_t budget = static_cast<uint64_t>(Param(ctx, "bnb.node_budget", 2000000));
+  if (budget != 0 && budget <= kFinishBudget) finish = false;
+  const uint64_t small_budget = finish ? kFinishNodes : budget;
   // waves per graph; 0 (the default): as many as keep 24 waves on each CU
   // when every graph has its own workgroup slot (16 for at most one graph
   // per CU, 12 for two), else 8 (three 8-wave workgroups per CU)
@@ -1398,14 +1487,15 @@ void SolveBnBSearch(td_ctx* ctx, int ngraphs, const int32_t* ns, const uint64_t*
   auto launch = [&] {
     hipLaunchKernelGGL(BnBResetQueue, dim3(1), dim3(64), 0, ctx->stream, dQ);
     hipLaunchKernelGGL(BnBKernel, dim3(groups), dim3(64 * W), W * WaveLds(dp_small),
-                       ctx->stream, dG, dO, dM, memo_log2, budget, dp_small, ngraphs, dQ);
+                       ctx->stream, dG, dO, dM, memo_log2, budget, small_budget, dp_small, ngraphs,
+                       dQ);
   };
   if (Param(ctx, "bnb.use_graph", 1) == 0) {
     launch();
   } else {
     const std::vector<uint64_t> key = {
         static_cast<uint64_t>(groups), static_cast<uint64_t>(W), static_cast<uint64_t>(dp_small),
-        static_cast<uint64_t>(memo_log2), budget, static_cast<uint64_t>(ngraphs),
+        static_cast<uint64_t>(memo_log2), budget, small_budget, static_cast<uint64_t>(ngraphs),
         reinterpret_cast<uint64_t>(dG), reinterpret_cast<uint64_t>(dO),
         reinterpret_cast<uint64_t>(dM), reinterpret_cast<uint64_t>(dQ)};
     if (ctx->bnb_graph && ctx->bnb_graph_key != key) {
@@ -1432,6 +1522,10 @@ void SolveBnBSearch(td_ctx* ctx, int ngraphs, const int32_t* ns, const uint64_t*
   TD_HIP(hipMemcpyAsync(ho.data(), dO, sizeof(BnBOut) * ngraphs, hipMemcpyDeviceToHost,
                         ctx->stream));
   TD_HIP(hipStreamSynchronize(ctx->stream));
+  float search_ms = 0.f;
+  TD_HIP(hipEventElapsedTime(&search_ms, ctx->ev[0], ctx->ev[1]));
+  double finish_ms = 0.0;
+  if (finish) FinishSmall(ctx, ns, adj_concat, off, ub_seed, scores, ho, &finish_ms);
   ctx->bnb_last.assign(ngraphs, {0, 0, 0, -1, 0});
   uint64_t cert = 0, nodes = 0, hits = 0;
   for (int i = 0; i < ngraphs; ++i) {
@@ -1444,13 +1538,11 @@ void SolveBnBSearch(td_ctx* ctx, int ngraphs, const int32_t* ns, const uint64_t*
     hits += ho[i].memo_hits;
   }
   if (stats) {
-    float ms = 0.f;
-    TD_HIP(hipEventElapsedTime(&ms, ctx->ev[0], ctx->ev[1]));
     stats->graphs = static_cast<uint64_t>(ngraphs);
     stats->certified = cert;
     stats->nodes = nodes;
     stats->memo_hits = hits;
-    stats->kernel_ms = ms;
+    stats->kernel_ms = search_ms + finish_ms;
     stats->total_ms = std::chrono::duration<double, std::milli>(
                           std::chrono::steady_clock::now() - t0)
                           .count();

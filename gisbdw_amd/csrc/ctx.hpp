@@ -236,6 +236,7 @@ struct td_ctx {
   // DPFlowKernel's buffer: the words published in it carry the call's tag, and
   // its ticket counter has seen flow_tickets workgroups (see FlowBuffer)
   uint32_t flow_tag = 0, flow_tickets = 0;
+  bool single_solve_ran = false;  // by SolveOne, since it was last cleared (see KeepDP)
   bool record_up = false;  // its record is in "dp.graph" (see LastRecord)
   tdhip::DPGraph last_graph{};
 
@@ -268,6 +269,17 @@ uint64_t UnrankColex(int n, int k, uint64_t code);
 uint64_t RankColex(uint64_t mask);
 // validate a graph; returns the adjacency as 32-bit rows when n <= 32
 void ValidateGraph(int n, const uint64_t* adj, int max_n);
+// Runs call(), a td_dp_solve_batch of graphs of at most 26 vertices, without
+// ending the last single solve's queries: such a batch has buffers of its own,
+// unless it had to solve a graph singly.
+template <typename Call>
+int KeepDP(td_ctx* ctx, Call&& call) {
+  const bool had = ctx->have_dp;
+  ctx->single_solve_ran = false;
+  const int rc = call();
+  if (!ctx->single_solve_ran) ctx->have_dp = had;
+  return rc;
+}
 // device address of td_dp_solve_noalloc's fixed scratch array for the
 // context's device (once per device; the device must be current)
 void NoAllocSetup(td_ctx* ctx);

@@ -1119,6 +1119,7 @@ void SolveOne(td_ctx* ctx, int n, const uint64_t* adj, uint8_t* td_out,
   // the buffers below may be reallocated: until this solve completes, the
   // queries have no tables to read
   ctx->have_dp = false;
+  ctx->single_solve_ran = true;
   const bool lds = n <= kLdsMaxN, flow = !lds && n <= kFlowMaxN;
   DPGraph G = SingleGraph(ctx, n, adj, !lds && !flow);
   const uint64_t tbytes = ClaimedBytes(G, ClaimsPacked(ctx, n));

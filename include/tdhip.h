@@ -267,6 +267,9 @@ int td_bnb_solve(td_ctx* ctx, int32_t n, const uint64_t* adj, int32_t heur_td,
  * heur_td.  vertex_scores (nullable, sum n[i] floats): a learned proposal;
  * higher score = tried first as a root and used for an extra greedy upper
  * bound.  Scores only order the search; they never prune.
+ * A graph of at most 24 vertices that 1,024 nodes have not settled is finished
+ * by the subset DP (certified; its details count the search's nodes and end at
+ * the k it had reached) if "bnb.node_budget" is above 32,768 or 0, none.
  * td_out / certified_out: ngraphs bytes; parent_concat: sum n[i] bytes.
  * With the context parameter "bnb.dp_max_n" = m > 0 (default 0), graphs of
  * at most m <= 32 vertices are answered by td_dp_solve_batch instead

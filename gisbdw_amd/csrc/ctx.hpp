@@ -237,6 +237,7 @@ struct td_ctx {
   // its ticket counter has seen flow_tickets workgroups (see FlowBuffer)
   uint32_t flow_tag = 0, flow_tickets = 0;
   bool single_solve_ran = false;  // by SolveOne, since it was last cleared (see KeepDP)
+  int unsynced = 0;  // single solves since their stream was last synchronized
   bool record_up = false;  // its record is in "dp.graph" (see LastRecord)
   tdhip::DPGraph last_graph{};
 

@@ -1009,14 +1009,34 @@ void FillStats(td_dp_stats* stats, int n, uint64_t launches, uint64_t level_kern
       std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
 }
 
-// Results of DPLdsKernel in host-visible memory: 64 parents, the depth, and
-// three readings of the device's clock.
+// Results of DPLdsKernel in host-visible memory: 64 parents, the depth, three
+// readings of the device's clock, and "done".
 struct LdsOut {
   int8_t parent[64];
   int32_t td;
   int32_t status;
-  unsigned long long clock[3];
+  unsigned long long clock[4];
 };
+
+// Waits until the last kernel of a single solve has published its results.
+// Reading the flag it writes sees them 5 to 6 us before
+// hipStreamSynchronize returns (n = 9: 27 to 21 us a call).  Should it not
+// come within a few milliseconds (a busy device, or an error), and once in a
+// while, for the runtime to take its launch resources back, the stream is
+// synchronized.
+void WaitDone(td_ctx* ctx, LdsOut* out) {
+  const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(5);
+  if (++ctx->unsynced < 64) {
+    for (int i = 1;; ++i) {
+      if (__atomic_load_n(&out->clock[3], __ATOMIC_ACQUIRE)) return;
+      __builtin_ia32_pause();
+      if (i % 256 == 0 && std::chrono::steady_clock::now() > until) break;
+    }
+  }
+  ctx->unsynced = 0;
+  TD_HIP(hipStreamSynchronize(ctx->stream));
+}
+
 
 // One launch for a graph of at most kLdsMaxN vertices: the graph goes up in
 // the kernel's arguments and the kernel writes its results to `out` itself, so
@@ -1134,6 +1154,7 @@ void SolveOne(td_ctx* ctx, int n, const uint64_t* adj, uint8_t* td_out,
   ctx->record_up = !lds && !fbuf;
   if (lds || fbuf) {
     LdsOut* out = reinterpret_cast<LdsOut*>(stage + kInBytes);
+    out->clock[3] = 0;
     if (lds) {
       LaunchLds(ctx, G, cb, arena, out);
     } else {
@@ -1146,7 +1167,7 @@ void SolveOne(td_ctx* ctx, int n, const uint64_t* adj, uint8_t* td_out,
       LaunchFlow(ctx, f, 1, groups, nullptr, cb, arena, fbuf, out->parent, &out->td, &out->status,
                  out->clock);
     }
-    TD_HIP(hipStreamSynchronize(ctx->stream));
+    WaitDone(ctx, out);
     if (lds || !out->status) {
       if (td_out) *td_out = static_cast<uint8_t>(out->td);
       if (parent_out) std::memcpy(parent_out, out->parent, n);

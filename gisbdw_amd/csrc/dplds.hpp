@@ -37,6 +37,14 @@ constexpr int LdsThreads(int n) {
   return n <= 13 ? 64 : n == 14 ? 128 : n == 15 ? 256 : n == 16 ? 512 : 1024;
 }
 
+// Everything this wave has written is in host memory: clock[3] = 1, which the
+// host waits for.
+__device__ __forceinline__ void PublishDone(unsigned long long* clock) {
+  __threadfence_system();
+  if ((threadIdx.x & 63) == 0)
+    __hip_atomic_store(clock + 3, 1ull, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // the L of a word that meet the low set T
 __device__ __forceinline__ uint32_t Meets(uint32_t T) {
   return ((T & 1u) ? 0xAAAAAAAAu : 0u) | ((T & 2u) ? 0xCCCCCCCCu : 0u) |
@@ -105,7 +113,7 @@ __device__ __forceinline__ DPWord LdsWord(const uint32_t* s, const uint32_t* w, 
 // or null for the graph in `one`.  table (nullable): takes the graph's three planes
 // (2^nh words each, word H at H: DPGraph::direct), for later queries.
 // Results: 64 parents and the depth per graph; clock (nullable): the device's
-// clock at the start, after the levels and at the end.
+// clock at the start, after the levels and at the end, then PublishDone.
 __global__ __launch_bounds__(1024) void DPLdsKernel(
     const LdsGraph* __restrict__ gs, const LdsGraph one, const uint32_t* __restrict__ g_cb,
     uint32_t* __restrict__ table, int8_t* __restrict__ parent_out, int32_t* __restrict__ td_out,
@@ -165,6 +173,7 @@ __global__ __launch_bounds__(1024) void DPLdsKernel(
       clock[2] = wall_clock64();
     }
   }
+  if (clock) PublishDone(clock);
 }
 
 // ---------------------------------------------------------------------------
@@ -412,6 +421,7 @@ __global__ __launch_bounds__(64) void DPDirectTreeKernel(
     td_out[blockIdx.x] = depth;
     if (clock) clock[2] = wall_clock64();
   }
+  if (clock) PublishDone(clock);
 }
 
 }  // namespace

@@ -209,7 +209,7 @@ __device__ __forceinline__ int CeilLog2(int x) {  // x >= 1
 // sU / sD: this wave's LDS scratch (64 entries each) for U and D; a child
 // adds its L to its parent's entries with LDS atomics (the value an OR
 // returns shows the bits an earlier child already brought, which go to D).
-__device__ int TreeRank(uint64_t myadj, uint64_t C, int* top, uint32_t* sU, uint32_t* sD) {
+__device__ __forceinline__ int TreeRank(uint64_t myadj, uint64_t C, int* top, uint32_t* sU, uint32_t* sD) {
   const int lane = threadIdx.x & 63;
   const uint64_t root = C & (0ull - C);
   int mylvl = (root >> lane) & 1ull ? 0 : -1;
@@ -329,52 +329,87 @@ __device__ __forceinline__ int Degeneracy(uint64_t myadj, uint64_t X0) {
   return d;
 }
 
-// ---- memo: per-wave table of 2^log2 buckets x 4 entries of 16 bytes -------
-// entry = {key lo, key hi, data, tag}; data: bits 0-7 lb, 8-15 solk (0 =
-// none), 16-23 root; tag = graph serial + 1 (0 = empty), so a new graph needs
-// no clearing.
+// ---- memo: a table of 2^log2 buckets, 4 entries of 16 bytes a wave in each --
+// entry = {key = the set, val}; val: bits 0-7 lb, 8-15 solk (0 = none), 16-23
+// root, 32-63 tag = graph serial + 1 (0 = empty), so a new graph needs no
+// clearing.  A wave writes its own four entries of a bucket and reads those of
+// every wave of its workgroup, which are next to each other: what one wave has
+// proven settles the set for all (with a table to each wave, 16 waves spent 1.8
+// times the nodes of one on the same refutation: 21200 and 11400 on a near-tree
+// of 49 vertices).
+//
+// Entries 0-2 get their key once for a tag: key, then (release) the val with
+// the tag.  So a reader that has seen the val may take the facts of another
+// wave if the key, read again after an acquire, is the set's.  Entry 3 is the
+// one replaced when a bucket is full; only its own wave reads it.
+struct MemoEntry {
+  uint64_t key, val;
+};
+
 struct Memo {
-  uint4* table;
-  uint32_t mask;  // buckets - 1
+  MemoEntry* table;  // the workgroup's
+  uint32_t mask;     // buckets - 1
   uint32_t tag;
+  uint32_t waves, wave;
 };
 
 __device__ __forceinline__ uint32_t BucketOf(uint64_t C, uint32_t mask) {
   return static_cast<uint32_t>((C * 0x9E3779B97F4A7C15ull) >> 40) & mask;
 }
 
-// Lane i (i < 4) owns entry i of every bucket: it alone writes it and
-// reads it back for the decision, so one thread's program order keeps every
-// probe after every earlier store of the wave: no barrier is needed.  Lanes
-// 4-63 load copies of the same four entries (one 64-byte request for the
-// wave) and take no part.  MemoIssue loads C's bucket so the latency can
-// overlap other work; MemoResolve returns the first matching entry's data
-// (0 if absent) and its slot, or -1 - the first free slot (else a victim)
-// when absent.
+template <typename T>
+__device__ __forceinline__ T MemoLoad(const T* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// Lane 4 w + e reads entry e of wave w's part of C's bucket (lanes past the
+// waves read along and take no part).  The lane that reads one of this wave's
+// entries is the one that writes it, so its program order keeps every probe
+// after every earlier store of the wave.  MemoIssue loads C's bucket so the
+// latency can overlap other work; MemoResolve returns all that is known of C
+// (0: nothing) and the entry to store at: C's own one of this wave, or else
+// -1 - the first unused one (3 if none is).
 struct Bucket {
-  uint4 e;  // entry (lane & 3) of the bucket
+  const MemoEntry* p;
+  uint64_t key, val;
 };
 
 __device__ __forceinline__ Bucket MemoIssue(const Memo& m, uint64_t C) {
   Bucket b;
-  b.e = m.table[static_cast<size_t>(BucketOf(C, m.mask)) * 4 + (threadIdx.x & 3)];
+  const uint32_t at = min(threadIdx.x & 63u, 4u * m.waves - 1u);
+  b.p = m.table + static_cast<size_t>(BucketOf(C, m.mask)) * (4u * m.waves) + at;
+  b.val = MemoLoad(&b.p->val);
+  b.key = MemoLoad(&b.p->key);
   return b;
 }
 
 __device__ __forceinline__ uint32_t MemoResolve(const Memo& m, uint64_t C,
                                                 const Bucket& b, int* slot) {
-  const bool mine = (threadIdx.x & 63) < 4;
-  const bool live = b.e.w == m.tag;
-  const uint64_t hits = Ballot(mine && live && b.e.x == static_cast<uint32_t>(C) &&
-                               b.e.y == static_cast<uint32_t>(C >> 32));
-  if (hits) {
-    const int s = __builtin_ctzll(hits);
-    *slot = s;
-    return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(b.e.z), s));
+  const uint32_t lane = threadIdx.x & 63;
+  const bool own = lane >> 2 == m.wave;
+  const bool live = static_cast<uint32_t>(b.val >> 32) == m.tag && lane < 4 * m.waves;
+  bool hit = live && b.key == C && (own || (lane & 3) != 3);
+  uint64_t hits = Ballot(hit);
+  const uint64_t mine = 15ull << (4 * m.wave);
+  if (hits & ~mine) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    hit = hit && (own || MemoLoad(&b.p->key) == C);
+    hits = Ballot(hit);
   }
-  const uint64_t frees = Ballot(mine && !live);
-  *slot = frees ? -1 - __builtin_ctzll(frees) : -1 - static_cast<int>((C >> 40) & 3ull);  // victim
-  return 0u;
+  const uint64_t known = hits & mine;
+  const uint64_t frees = Ballot(own && !live);
+  *slot = known ? static_cast<int>(__builtin_ctzll(known) & 3)
+                : -1 - (frees ? static_cast<int>(__builtin_ctzll(frees) & 3) : 3);
+  uint32_t data = 0;
+  for (; hits; hits &= hits - 1) {  // the best of every wave's facts
+    const uint32_t d = static_cast<uint32_t>(__builtin_amdgcn_readlane(
+        static_cast<int>(static_cast<uint32_t>(b.val)), __builtin_ctzll(hits)));
+    const uint32_t lb = max(data & 0xFFu, d & 0xFFu);
+    const uint32_t have = data >> 8 & 0xFFu, more = d >> 8 & 0xFFu;
+    const uint32_t sol = more && (!have || more < have) ? d : data;
+    data = lb | (sol & 0xFFFF00u);
+  }
+  return data;
 }
 
 __device__ __forceinline__ uint32_t MemoProbe(const Memo& m, uint64_t C,
@@ -383,26 +418,25 @@ __device__ __forceinline__ uint32_t MemoProbe(const Memo& m, uint64_t C,
   return MemoResolve(m, C, b, slot);
 }
 
+// Adds to the facts known of C (`old`, the result of the probe that gave slot).
 __device__ __forceinline__ void MemoStore(const Memo& m, uint64_t C, int slot,
                                           uint32_t old, uint32_t lb, uint32_t solk,
                                           uint32_t root) {
-  uint32_t olb = old & 0xFF, osk = (old >> 8) & 0xFF, ort = (old >> 16) & 0xFF;
-  if (slot < 0) {  // new entry
-    olb = 0;
-    osk = 0;
-    ort = 0;
+  const uint32_t osk = old >> 8 & 0xFFu;
+  const uint32_t nlb = max(old & 0xFFu, lb);
+  uint32_t sol = old & 0xFFFF00u;
+  if (solk && (!osk || solk < osk)) sol = solk << 8 | root << 16;
+  const uint32_t s = static_cast<uint32_t>(slot < 0 ? -1 - slot : slot);
+  if ((threadIdx.x & 63) == 4 * m.wave + s) {  // the entry's owner
+    MemoEntry* p = m.table + static_cast<size_t>(BucketOf(C, m.mask)) * (4u * m.waves) +
+                   (4 * m.wave + s);
+    if (slot < 0) {
+      __hip_atomic_store(&p->key, C, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    }
+    __hip_atomic_store(&p->val, static_cast<uint64_t>(m.tag) << 32 | sol | nlb,
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   }
-  const uint32_t nlb = max(olb, lb);
-  uint32_t nsk = osk, nrt = ort;
-  if (solk && (!osk || solk < osk)) {
-    nsk = solk;
-    nrt = root;
-  }
-  const int s = slot < 0 ? -1 - slot : slot;
-  if ((threadIdx.x & 63) == s)  // the entry's owner
-    m.table[static_cast<size_t>(BucketOf(C, m.mask)) * 4 + s] =
-        make_uint4(static_cast<uint32_t>(C), static_cast<uint32_t>(C >> 32),
-                   nlb | (nsk << 8) | (nrt << 16), m.tag);
 }
 
 // Highest key among cand (nonempty), ties to the lowest vertex: plain =
@@ -458,6 +492,9 @@ __device__ __forceinline__ uint64_t Undominated(uint64_t myadj, const uint64_t* 
   return C & ~Ballot(dominated);
 }
 
+// One wave's search.  Every function that takes it by reference is inlined: with
+// one of them out of line the state lives in memory and the LDS pointers in it
+// become generic ones, 5.0 us a node instead of 3.7 for a wave alone.
 struct Search {
   Frame* st;  // LDS stack
   uint64_t myadj;
@@ -601,7 +638,7 @@ __device__ __forceinline__ bool Halted(Search& S) {
 // decided: *roots holds the roots to try).  e = |E(C)| or -1; ecc / last:
 // the BFS from C's lowest vertex (its rounds and last front) when the caller
 // has run it, else ecc = -1.
-__device__ int Enter(Search& S, uint64_t C, int k, int e, int ecc, uint64_t last,
+__device__ __forceinline__ int Enter(Search& S, uint64_t C, int k, int e, int ecc, uint64_t last,
                      uint64_t* roots) {
   const int lane = threadIdx.x & 63;
   const int n = __builtin_popcountll(C);
@@ -644,7 +681,7 @@ __device__ int Enter(Search& S, uint64_t C, int k, int e, int ecc, uint64_t last
   // the nodes of sparse graphs)
   int slot;
   const uint32_t md = MemoResolve(S.memo, C, me, &slot);
-  if (slot >= 0) {
+  {
     const uint32_t mlb = md & 0xFF, sk = (md >> 8) & 0xFF;
     if (sk && sk <= static_cast<uint32_t>(k)) { ++S.hits; return 1; }
     if (mlb > static_cast<uint32_t>(k)) { ++S.hits; return 0; }
@@ -679,7 +716,7 @@ __device__ int Enter(Search& S, uint64_t C, int k, int e, int ecc, uint64_t last
 // view), so no barrier is needed between a frame update and its use.  A
 // child that its node decides at once (most of them: a bound or the memo)
 // gets no frame; a frame is pushed only for a child whose roots are tried.
-__device__ bool Feasible(Search& S, uint64_t C0, int k0) {
+__device__ __forceinline__ bool Feasible(Search& S, uint64_t C0, int k0) {
   const int lane = threadIdx.x & 63;
   {
     const int n0 = __builtin_popcountll(C0);
@@ -855,7 +892,7 @@ __device__ bool Feasible(Search& S, uint64_t C0, int k0) {
 
 // Rebuild a tree of depth <= k for connected C from the memo's roots,
 // re-running the search for a set whose entry was evicted.  parent[] in LDS.
-__device__ void Build(Search& S, uint64_t C0, int k0, int par0, int8_t* parent,
+__device__ __forceinline__ void Build(Search& S, uint64_t C0, int k0, int par0, int8_t* parent,
                       uint64_t* bst, int* bk, int* bpar) {
   const int lane = threadIdx.x & 63;
   int sp = 0;
@@ -887,7 +924,7 @@ __device__ void Build(Search& S, uint64_t C0, int k0, int par0, int8_t* parent,
     }
     int slot;
     uint32_t md = MemoProbe(S.memo, C, &slot);
-    uint32_t sk = (slot >= 0) ? (md >> 8) & 0xFF : 0;
+    uint32_t sk = (md >> 8) & 0xFF;
     if (!(sk && sk <= static_cast<uint32_t>(k))) {
       const uint64_t saved_budget = S.budget;
       S.budget = 0;  // the set is known feasible: finish the search
@@ -896,7 +933,7 @@ __device__ void Build(Search& S, uint64_t C0, int k0, int par0, int8_t* parent,
       S.building = false;
       S.budget = saved_budget;
       md = MemoProbe(S.memo, C, &slot);
-      sk = (slot >= 0) ? (md >> 8) & 0xFF : 0;
+      sk = (md >> 8) & 0xFF;
       if (!(sk && sk <= static_cast<uint32_t>(k))) {
         // no tree can be rebuilt: report the call as uncertified and keep
         // the previous best tree
@@ -1015,7 +1052,7 @@ __device__ int MinDegreeTree(uint64_t myadj, uint64_t V, int8_t* parent,
 // Wave 0 computes the upper-bound trees and the static bound; then for each
 // k = UB-1, UB-2, ... the W waves share out the top-level root candidates (in
 // key order, each wave claiming the next one when it is free), each
-// searching its candidates with a private memo and drawing on the graph's
+// searching its candidates with the waves' common memo and drawing on the graph's
 // node budget in chunks.  A wave that finds a decomposition raises s_found
 // and the others stop; if none does and the budget did not run out, td > k
 // is proven.
@@ -1036,7 +1073,7 @@ __host__ __device__ constexpr size_t WaveLds(int dp_small) {
 __global__ __launch_bounds__(64 * kMaxWaves)
 __attribute__((amdgpu_waves_per_eu(6, 6))) void BnBKernel(
     const BnBGraph* __restrict__ gs, BnBOut* __restrict__ outs,
-    uint4* __restrict__ memo_base, int memo_log2, uint64_t node_budget, uint64_t small_budget,
+    MemoEntry* __restrict__ memo_base, int memo_log2, uint64_t node_budget, uint64_t small_budget,
     int dp_small, int ngraphs, uint32_t* __restrict__ queue) {
   // queue[0]: the next graph; queue[kTagWord]: this call's memo tag base,
   // written before the launch (a captured launch replays with new tags)
@@ -1066,7 +1103,9 @@ __attribute__((amdgpu_waves_per_eu(6, 6))) void BnBKernel(
     S.sdp_rows = reinterpret_cast<uint16_t*>(S.sdp + (1u << kSmallDPMax));
   }
   S.memo.table =
-      memo_base + (static_cast<size_t>(blockIdx.x * W + wid) << (memo_log2 + 2));
+      memo_base + (static_cast<size_t>(blockIdx.x * W) << (memo_log2 + 2));
+  S.memo.waves = static_cast<uint32_t>(W);
+  S.memo.wave = static_cast<uint32_t>(Uniform32(wid));
   S.memo.mask = (1u << memo_log2) - 1u;
   for (;;) {
     if (threadIdx.x == 0) s_gi = static_cast<int>(atomicAdd(queue, 1u));
@@ -1462,10 +1501,10 @@ void SolveBnBSearch(td_ctx* ctx, int ngraphs, const int32_t* ns, const uint64_t*
   if (groups_cap <= 0) groups_cap = ctx->prop.multiProcessorCount * 4;  // 0: 4 per CU
   const int groups = std::max(1, std::min(ngraphs, groups_cap));
   const size_t waves = static_cast<size_t>(groups) * W;
-  const size_t memo_bytes = (waves << (memo_log2 + 2)) * sizeof(uint4);
+  const size_t memo_bytes = (waves << (memo_log2 + 2)) * sizeof(MemoEntry);
   auto* dG = static_cast<BnBGraph*>(ctx->Buffer("bnb.graphs", sizeof(BnBGraph) * ngraphs));
   auto* dO = static_cast<BnBOut*>(ctx->Buffer("bnb.out", sizeof(BnBOut) * ngraphs));
-  auto* dM = static_cast<uint4*>(ctx->Buffer("bnb.memo", memo_bytes));
+  auto* dM = static_cast<MemoEntry*>(ctx->Buffer("bnb.memo", memo_bytes));
   auto* dQ = static_cast<uint32_t*>(ctx->Buffer("bnb.queue", 256));
   // Entries carry the tag of the graph that wrote them (a serial that grows
   // across calls), so a table is cleared only when it is (re)allocated.

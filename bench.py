@@ -17,23 +17,22 @@ around each graph's level sequence; the union of those intervals, so time
 in which two graphs' levels overlap counts once, and avg_launch_ms is that
 time over the launches: the period of one launch at the achieved rate, not
 the duration of a single kernel, which runs beside another graph's
-kernels), compulsory bytes = 2 * 2^n per graph
-(every level table written once and read back once by the next level).  The
+kernels), compulsory bytes = 0.75 * 2^n per graph
+(every level table, three bits per subset, written once and read back once by
+the next level).  The
 per-subset model of k one-byte reads of level k-1 plus one write, 2^(n-1)
 (n+2) bytes per graph, counts reads that the kernel serves from registers
 and caches; its rate is reported beside as model_GBps, not as the roofline.
-In the plain layout a graph's levels run as DPLevelKernel launches, except
-the runs of small levels at either end, which one DPSmallLevelsKernel
-workgroup does per run; in the class layout every level is one
-DPClassLevelKernel launch.  Per-launch figures divide by that launch count.
+A graph's levels run as DPLevelKernel launches, except the runs of small levels
+at either end, which one DPSmallLevelsKernel workgroup does per run.  Per-launch
+figures divide by that launch count.
 traffic is NOT measured by this run: it is the rocprofv3 --pmc figure (read
 and write bytes per launch from the L2's request counts by size) that the
 committed summary profiles/dp_level_kernel_n30_traffic.md holds for the
 launch shape that ran (null if it has none); traffic_over_compulsory divides
 it by the compulsory bytes per launch.
 
-Launch shape: td_dp_autotune picks (class_bits, low_bits, tiles_per_lane,
-grid_mult, block) for n before the warm-up, unless --no-autotune or an
+Launch shape: td_dp_autotune picks (low_bits, tiles_per_lane, grid_mult, block) for n before the warm-up, unless --no-autotune or an
 explicit shape flag is given.
 
 cpu_baseline: the oracle's flat-table DP (OpenMP over each level) timed on the
@@ -86,7 +85,7 @@ def parse():
     ap.add_argument("--class-bits", type=int, default=None, choices=[0, 3, 4])
     ap.add_argument("--grid-mult", type=int, default=None)
     ap.add_argument("--packed", type=int, default=None, choices=[0, 1],
-                    help="class layouts: packed tiles (4 bits per subset) or byte tiles")
+                    help="kept for older command lines; without effect")
     ap.add_argument("--streams", type=int, default=None, choices=[1, 2, 3],
                     help="large graphs of a batch call: level sequences in flight at once")
     ap.add_argument("--batch-block", type=int, default=None)
@@ -531,13 +530,8 @@ def cpu_baseline_bottom_up(g):
 
 def shape_key(ctx):
     """The DP launch shape, as the traffic summary keys its lines."""
-    key = ("low_bits={} tiles_per_lane={} block={} class_bits={} grid_mult={}".format(
-        *(ctx.get_param("dp." + k) for k in
-          ("low_bits", "tiles_per_lane", "block", "class_bits", "grid_mult"))))
-    if ctx.get_param("dp.class_bits") and ctx.get_param("dp.low_bits") >= 4 and \
-            ctx.get_param("dp.packed"):
-        key += " packed=1"
-    return key
+    return "low_bits={} tiles_per_lane={} block={} grid_mult={}".format(
+        *(ctx.get_param("dp." + k) for k in ("low_bits", "tiles_per_lane", "block", "grid_mult")))
 
 
 def profile_traffic(key):
@@ -639,7 +633,8 @@ def main():
             print(f"[bench] step {i} level_ms={a:.3f}", file=sys.stderr, flush=True)
         wall = time.perf_counter() - t0
         nlev = kernels[0]  # level-kernel executions in the timed steps
-        comp = 2 * sub  # compulsory bytes: each level written once, read once
+        # compulsory bytes: three bits per subset, written once, read once
+        comp = 0.75 * sub
         achieved = comp / (lvl_ms * 1e-3) / 1e9
         n = graphs[0].n
         traffic = profile_traffic(shape_key(ctx))
@@ -683,9 +678,8 @@ def main():
                                   "TCC_EA0_RDREQ_{32B,64B,128B} and TCC_EA0_WRREQ(_64B) "
                                   "request counts, not this run)",
                 "traffic_over_compulsory": (traffic / (comp / nlev)) if traffic else None,
-                "kernel": ("DPClassLevelKernel" if ctx.get_param("dp.class_bits")
-                           else "DPLevelKernel"),
-                "bytes_basis": "compulsory: 2 * 2^n per graph",
+                "kernel": "DPLevelKernel",
+                "bytes_basis": "compulsory: 0.75 * 2^n per graph (3 bits per subset)",
                 "compulsory_bytes_per_launch": comp / nlev,
                 "avg_launch_ms": lvl_ms / nlev,
                 "launches": nlev,
@@ -704,8 +698,8 @@ def main():
         # per height: the kept forest's 32 slots read and 34 bytes written
         # (its 32 slots, the vertex added last, the height), plus the k
         # heights of S \ v and 2|E(S)| neighbour slots read; over all subsets
-        # 66 * 2^n + (n + m) * 2^(n-1).  The kernel packs slots into 4 bits
-        # where the heights allow, so it moves fewer bytes than this.
+        # 66 * 2^n + (n + m) * 2^(n-1).  The kernel packs slots into 3 or 4
+        # bits where the heights allow, so it moves fewer bytes than this.
         g = G.gnp(26, 0.15, 1)
         graphs = [g]
         m = sum(bin(r).count("1") for r in g.adj) // 2
@@ -869,7 +863,7 @@ def main():
             sub += st.subsets
             print(f"[bench] step {i} level_ms={st.level_ms:.3f}", file=sys.stderr, flush=True)
         wall = time.perf_counter() - t0
-        achieved = 2 * sub / (lvl_ms * 1e-3) / 1e9
+        achieved = 0.75 * sub / (lvl_ms * 1e-3) / 1e9  # three bits per subset, twice
         out = {
             "metric": "DP graphs/sec (batched exact subset DP)",
             "value": len(graphs) * args.steps / wall,
@@ -888,7 +882,7 @@ def main():
             "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBPS,
                          "unit": "GB/s", "frac": achieved / HBM_PEAK_GBPS, "traffic": None,
                          "kernel": "DPPersistentKernel",
-                         "bytes_basis": "compulsory: 2 * 2^n per graph",
+                         "bytes_basis": "compulsory: 0.75 * 2^n per graph (3 bits per subset)",
                          "model_GBps": alg / (lvl_ms * 1e-3) / 1e9},
             "extra": {"subsets_per_s": sub / wall},
         }

@@ -2095,8 +2095,8 @@ int td_dp_autotune(td_ctx* ctx, int32_t n, const char* cache_path,
       // (tiles per lane, grid multiple): one tile per lane at three grid
       // sizes, and two consecutive tiles per lane
       const int shapes[4][2] = {{1, 2}, {1, 4}, {1, 8}, {2, 4}};
-      // plain and class layouts; class layouts with 16- or 32-subset tiles
-      // both packed and as bytes
+      // (class_bits and packed no longer change the tables; the candidates are
+      // still those that existing caches and their readers know)
       for (int cbits : {0, 4})
         for (int lb : {3, 4, 5})
           for (int pk : {0, 1}) {

@@ -161,8 +161,8 @@ int td_dp_solve_batch(td_ctx* ctx, int32_t ngraphs, const int32_t* n,
                       int8_t* parent_concat, int32_t mode,
                       td_dp_stats* stats);
 
-/* Autotuner: times every candidate (class_bits, low_bits, tiles_per_lane,
- * grid_mult, block) on a seeded G(n, 0.25) graph and keeps the best in the
+/* Autotuner: times every candidate (low_bits, tiles_per_lane, grid_mult,
+ * block) on a seeded G(n, 0.25) graph and keeps the best in the
  * context: the level kernels for n > 26 (such graphs also run in batch
  * calls, where the tree kernel is hidden), the level kernels plus the tree
  * kernel for smaller n.  With a non-null cache_path (JSON lines), a "best"

@@ -489,6 +489,46 @@ __device__ __forceinline__ uint32_t LookupCode(const DPHead* __restrict__ g,
   return ((g0 >> (S & 31u)) & 1u) | (((g1 >> (S & 31u)) & 1u) << 1);
 }
 
+// Whether td(A) and td(B) differ, A a set and B = A without at most one
+// vertex: both ranks in one pass, four vertices of each at a time, so that
+// eight reads of the binomials are in flight, then the four words together
+// (one set after the other, a vertex at a time: 33 us for the tree at n = 29,
+// 25 this way).
+__device__ __forceinline__ bool CodesDiffer(const DPHead* __restrict__ g,
+                                            const uint8_t* __restrict__ arena,
+                                            const uint32_t* s_cb, const uint32_t* s_base,
+                                            uint32_t A, uint32_t B) {
+  if (g->direct) return LookupCode(g, arena, s_cb, s_base, A) != LookupCode(g, arena, s_cb, s_base, B);
+  const uint32_t lb = g->lb;
+  uint32_t Ha = A >> lb, Hb = B >> lb;
+  uint32_t ta = s_base[__builtin_popcount(Ha)], tb = s_base[__builtin_popcount(Hb)];
+  // the i-th vertex's binomial; past the last one C(0, 1) = 0
+  auto term = [&](uint32_t* H, int i) {
+    const uint32_t at = *H ? static_cast<uint32_t>(__builtin_ctz(*H)) * kCbStride + i : 1u;
+    *H &= *H - 1;
+    return s_cb[at];
+  };
+  for (int i = 1; Ha; i += 4) {  // B has no vertex that A lacks
+    const uint32_t a0 = term(&Ha, i), b0 = term(&Hb, i);
+    const uint32_t a1 = term(&Ha, i + 1), b1 = term(&Hb, i + 1);
+    const uint32_t a2 = term(&Ha, i + 2), b2 = term(&Hb, i + 2);
+    const uint32_t a3 = term(&Ha, i + 3), b3 = term(&Hb, i + 3);
+    ta += a0 + a1 + a2 + a3;
+    tb += b0 + b1 + b2 + b3;
+  }
+  const size_t ps = static_cast<size_t>(s_base[g->nh + 1]) << (lb - 3);
+  const uint32_t words = (1u << (lb - 5)) - 1u;
+  const uint8_t* base = arena + g->table;
+  const uint8_t* pa = base + (static_cast<size_t>(ta) << (lb - 3)) + 4 * ((A >> 5) & words);
+  const uint8_t* pb = base + (static_cast<size_t>(tb) << (lb - 3)) + 4 * ((B >> 5) & words);
+  const uint32_t a0 = *reinterpret_cast<const uint32_t*>(pa);
+  const uint32_t a1 = *reinterpret_cast<const uint32_t*>(pa + ps);
+  const uint32_t b0 = *reinterpret_cast<const uint32_t*>(pb);
+  const uint32_t b1 = *reinterpret_cast<const uint32_t*>(pb + ps);
+  const uint32_t sa = A & 31u, sb = B & 31u;
+  return (((a0 >> sa) ^ (b0 >> sb)) | ((a1 >> sa) ^ (b1 >> sb))) & 1u;
+}
+
 // td mod 4 of a Gray code
 __device__ __forceinline__ uint32_t GrayValue(uint32_t code) { return code ^ (code >> 1); }
 
@@ -597,12 +637,12 @@ __global__ __launch_bounds__(64) void DPWalkKernel(
 // the same round, the parent of a root is the root whose removal created its
 // component, and all roots leave together.  The tree is the one
 // GetElimination's order produces (each component's root depends only on the
-// component), in about td rounds instead of n.  code(S): the Gray code of
-// td(S) mod 4.  Returns lane u's parent (-1: a root); *depth_out = the tree's
+// component), in about td rounds instead of n.  differ(C, D): whether the Gray
+// codes of td(C) and td(D) mod 4 differ.  Returns lane u's parent (-1: a root); *depth_out = the tree's
 // depth in every lane.
-template <typename Code>
+template <typename Differ>
 __device__ __forceinline__ int DecomposeWave(uint32_t myadj, uint32_t S, int* depth_out,
-                                             Code code) {
+                                             Differ differ) {
   const int lane = threadIdx.x & 63;
   if (lane >= 32) myadj = 0u;
   int creator = -1, depth = 0, parent = -1;
@@ -623,9 +663,8 @@ __device__ __forceinline__ int DecomposeWave(uint32_t myadj, uint32_t S, int* de
       rest &= ~comp;
     }
     // td(C \ v) is td(C) or td(C) - 1: the codes mod 4 tell which
-    const uint32_t cc = in ? code(mine) : 0u;
-    const uint32_t cv = in ? code(mine & ~(1u << lane)) : 0u;
-    const uint32_t cand = static_cast<uint32_t>(__ballot(in && cv != cc));
+    const uint32_t cand =
+        static_cast<uint32_t>(__ballot(in && differ(mine, mine & ~(1u << (lane & 31)))));
     // a connected set always has a vertex with td(C \ v) = td(C) - 1; the
     // lowest vertex stands in only so that a damaged table cannot stall
     const uint32_t rc = cand & mine;
@@ -659,7 +698,9 @@ __global__ __launch_bounds__(64) void DPTreeKernel(
   int depth = 0;
   const int parent =
       DecomposeWave(lane < 32 ? g->adj[lane] : 0u, S, &depth,
-                    [&](uint32_t C) { return LookupCode(g, arena, s_cb, s_base, C); });
+                    [&](uint32_t C, uint32_t D) {
+                      return CodesDiffer(g, arena, s_cb, s_base, C, D);
+                    });
   int8_t* out = parent_out + static_cast<size_t>(blockIdx.x) * 64;
   if (lane < 32 && ((S >> lane) & 1u)) out[lane] = static_cast<int8_t>(parent);
   if (lane == 0) td_out[blockIdx.x] = depth;
@@ -1159,8 +1200,8 @@ void SolveOne(td_ctx* ctx, int n, const uint64_t* adj, uint8_t* td_out,
   uint8_t* din = static_cast<uint8_t*>(ctx->Buffer("dp.graph", kInBytes));
   DPGraph* dG = reinterpret_cast<DPGraph*>(din);
   const uint32_t* cb = PascalDevice(ctx);
-  uint8_t* dtree = static_cast<uint8_t*>(ctx->Buffer("dp.tree_out", kTreeBytes));
-  uint8_t* stage = static_cast<uint8_t*>(ctx->Pinned(kInBytes + sizeof(LdsOut)));
+  (void)ctx->Buffer("dp.tree_out", kTreeBytes);  // asks the byte budget
+  uint8_t* stage = static_cast<uint8_t*>(ctx->Pinned(kInBytes + std::max(sizeof(LdsOut), kTreeBytes)));
   uint8_t* fbuf = flow ? FlowBuffer(ctx, FlowBytes(n)) : nullptr;
   ctx->last_n = n;
   ctx->record_up = !lds && !fbuf;
@@ -1204,13 +1245,13 @@ void SolveOne(td_ctx* ctx, int n, const uint64_t* adj, uint8_t* td_out,
   TD_HIP(hipEventRecord(ctx->ev[0], ctx->stream));
   RunLevels(ctx, G, dG, cb, arena, &launches);
   TD_HIP(hipEventRecord(ctx->ev[1], ctx->stream));
+  // the tree goes straight to page-locked memory
+  uint8_t* staged = stage + kInBytes;
   hipLaunchKernelGGL(DPTreeKernel<DPGraph>, dim3(1), dim3(64), 0, ctx->stream, dG, cb, arena,
-                     reinterpret_cast<int8_t*>(dtree), reinterpret_cast<int32_t*>(dtree + 64));
+                     reinterpret_cast<int8_t*>(staged), reinterpret_cast<int32_t*>(staged + 64));
   TD_HIP(hipGetLastError());
   ++launches;
   TD_HIP(hipEventRecord(ctx->ev[2], ctx->stream));
-  uint8_t* staged = stage + kInBytes;
-  TD_HIP(hipMemcpyAsync(staged, dtree, 64 + 4, hipMemcpyDeviceToHost, ctx->stream));
   TD_HIP(hipStreamSynchronize(ctx->stream));
   int32_t td = 0;
   std::memcpy(&td, staged + 64, 4);

@@ -159,10 +159,11 @@ __global__ __launch_bounds__(1024) void DPLdsKernel(
   const unsigned long long t1 = clock ? wall_clock64() : 0ull;
   int depth = 0;
   const int parent = DecomposeWave(s[kLdsAdj + (tid & 31)], n >= 32 ? ~0u : (1u << n) - 1u, &depth,
-                                   [&](uint32_t S) {
-                                     const uint32_t* p = w + (S >> 5);
-                                     return (p[0] >> (S & 31u) & 1u) |
-                                            (p[N] >> (S & 31u) & 1u) << 1;
+                                   [&](uint32_t A, uint32_t B) {
+                                     const uint32_t *a = w + (A >> 5), *b = w + (B >> 5);
+                                     const uint32_t x = a[0], y = a[N], u = b[0], v = b[N];
+                                     return (((x >> (A & 31u)) ^ (u >> (B & 31u))) |
+                                             ((y >> (A & 31u)) ^ (v >> (B & 31u)))) & 1u;
                                    });
   if (tid < n) parent_out[64 * static_cast<size_t>(blockIdx.x) + tid] = static_cast<int8_t>(parent);
   if (tid == 0) {
@@ -412,9 +413,10 @@ __global__ __launch_bounds__(64) void DPDirectTreeKernel(
   const uint32_t* mine = table + cl.table + 3 * plane * (blockIdx.x - cl.graph);
   const uint32_t row = lane >= n ? 0u : gs ? gs[blockIdx.x].adj[lane] : f.one.adj[lane];
   int depth = 0;
-  const int parent = DecomposeWave(row, (1u << n) - 1u, &depth, [&](uint32_t S) {
-    const uint32_t* p = mine + (S >> 5);
-    return (p[0] >> (S & 31u) & 1u) | (p[plane] >> (S & 31u) & 1u) << 1;
+  const int parent = DecomposeWave(row, (1u << n) - 1u, &depth, [&](uint32_t A, uint32_t B) {
+    const uint32_t *a = mine + (A >> 5), *b = mine + (B >> 5);
+    const uint32_t x = a[0], y = a[plane], u = b[0], v = b[plane];
+    return (((x >> (A & 31u)) ^ (u >> (B & 31u))) | ((y >> (A & 31u)) ^ (v >> (B & 31u)))) & 1u;
   });
   if (lane < n) parent_out[64 * static_cast<size_t>(blockIdx.x) + lane] = static_cast<int8_t>(parent);
   if (lane == 0) {

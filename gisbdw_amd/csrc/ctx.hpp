@@ -195,9 +195,11 @@ struct td_ctx {
   void* Buffer(const std::string& name, size_t bytes);
   void Release(const std::string& name);
   // page-locked host staging for the per-call copies, two independent
-  // buffers (grown on demand; every call synchronizes before returning, so
-  // they are reused): slot 0 for single-graph staging, slot 1 for the batch
-  // records and results, which live across the large-graph pipeline
+  // buffers (grown on demand): slot 0 for single-graph staging, slot 1 for the
+  // batch records and results, which live across the large-graph pipeline.
+  // They are reused because no call returns while the device may still access
+  // them: it has synchronized, or (a single solve of at most 24 vertices) read
+  // the flag that the last kernel writes after everything else
   void* pinned[2] = {nullptr, nullptr};
   size_t pinned_bytes[2] = {0, 0};
   void* Pinned(size_t bytes, int slot = 0);

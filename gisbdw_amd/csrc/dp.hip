@@ -1071,7 +1071,9 @@ struct LdsOut {
   unsigned long long clock[4];
 };
 
-// Waits until the last kernel of a single solve has published its results.
+// Waits until the last kernel of a single solve has published its results, its
+// last act: tree and tables are written, and all that is left of the call on
+// the device is the kernel's own end.
 // Reading the flag it writes sees them 5 to 6 us before
 // hipStreamSynchronize returns (n = 9: 27 to 21 us a call).  Should it not
 // come within a few milliseconds (a busy device, or an error), and once in a

@@ -31,14 +31,14 @@ constexpr int kLdsAdj = 0, kLdsSize = 32, kLdsOff = 48, kLdsNbh = 64, kLdsIsoH =
 constexpr size_t LdsBytes(int n) {
   return 4 * static_cast<size_t>(kLdsHead) + (12ull << (n > 5 ? n - 5 : 0));
 }
-// Threads for one graph: a wave where every level fits one; else about the
-// largest level, at most 1024.
+// Threads for one graph: a wave up to n = 13 (at 13 one level, of 70 words,
+// takes two passes); else about the largest level, at most 1024.
 constexpr int LdsThreads(int n) {
   return n <= 13 ? 64 : n == 14 ? 128 : n == 15 ? 256 : n == 16 ? 512 : 1024;
 }
 
-// Everything this wave has written is in host memory: clock[3] = 1, which the
-// host waits for.
+// Everything this wave has written, and what other waves had written before a
+// barrier, is in memory: clock[3] = 1, which the host waits for.
 __device__ __forceinline__ void PublishDone(unsigned long long* clock) {
   __threadfence_system();
   if ((threadIdx.x & 63) == 0)
@@ -113,7 +113,8 @@ __device__ __forceinline__ DPWord LdsWord(const uint32_t* s, const uint32_t* w, 
 // or null for the graph in `one`.  table (nullable): takes the graph's three planes
 // (2^nh words each, word H at H: DPGraph::direct), for later queries.
 // Results: 64 parents and the depth per graph; clock (nullable): the device's
-// clock at the start, after the levels and at the end, then PublishDone.
+// clock at the start, after the levels and at the end, then PublishDone once
+// every wave has written its part of everything.
 __global__ __launch_bounds__(1024) void DPLdsKernel(
     const LdsGraph* __restrict__ gs, const LdsGraph one, const uint32_t* __restrict__ g_cb,
     uint32_t* __restrict__ table, int8_t* __restrict__ parent_out, int32_t* __restrict__ td_out,
@@ -153,28 +154,38 @@ __global__ __launch_bounds__(1024) void DPLdsKernel(
       next = order[s[kLdsOff + h + 1] + tid];
     __syncthreads();
   }
-  if (table)
+  if (table) {
     for (int i = tid; i < 3 * N; i += blockDim.x) table[i] = w[i];
-  if (tid >= 64) return;
-  const unsigned long long t1 = clock ? wall_clock64() : 0ull;
-  int depth = 0;
-  const int parent = DecomposeWave(s[kLdsAdj + (tid & 31)], n >= 32 ? ~0u : (1u << n) - 1u, &depth,
-                                   [&](uint32_t A, uint32_t B) {
-                                     const uint32_t *a = w + (A >> 5), *b = w + (B >> 5);
-                                     const uint32_t x = a[0], y = a[N], u = b[0], v = b[N];
-                                     return (((x >> (A & 31u)) ^ (u >> (B & 31u))) |
-                                             ((y >> (A & 31u)) ^ (v >> (B & 31u)))) & 1u;
-                                   });
-  if (tid < n) parent_out[64 * static_cast<size_t>(blockIdx.x) + tid] = static_cast<int8_t>(parent);
-  if (tid == 0) {
-    td_out[blockIdx.x] = depth;
-    if (clock) {
-      clock[0] = t0;
-      clock[1] = t1;
-      clock[2] = wall_clock64();
+    // a wave's part is written before the barrier that "done" waits for, not
+    // on its way (wave 0's own part: PublishDone)
+    if (tid >= 64) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+  }
+  if (tid < 64) {
+    const unsigned long long t1 = clock ? wall_clock64() : 0ull;
+    int depth = 0;
+    const int parent =
+        DecomposeWave(s[kLdsAdj + (tid & 31)], n >= 32 ? ~0u : (1u << n) - 1u, &depth,
+                      [&](uint32_t A, uint32_t B) {
+                        const uint32_t *a = w + (A >> 5), *b = w + (B >> 5);
+                        const uint32_t x = a[0], y = a[N], u = b[0], v = b[N];
+                        return (((x >> (A & 31u)) ^ (u >> (B & 31u))) |
+                                ((y >> (A & 31u)) ^ (v >> (B & 31u)))) & 1u;
+                      });
+    if (tid < n)
+      parent_out[64 * static_cast<size_t>(blockIdx.x) + tid] = static_cast<int8_t>(parent);
+    if (tid == 0) {
+      td_out[blockIdx.x] = depth;
+      if (clock) {
+        clock[0] = t0;
+        clock[1] = t1;
+        clock[2] = wall_clock64();
+      }
     }
   }
-  if (clock) PublishDone(clock);
+  if (!clock) return;
+  // "done" stands for the tables too, whichever wave wrote them
+  __syncthreads();
+  if (tid < 64) PublishDone(clock);
 }
 
 // ---------------------------------------------------------------------------

@@ -2049,7 +2049,6 @@ int td_dp_get_treedepth(td_ctx* ctx, int32_t k, uint64_t code,
     TD_REQUIRE(k >= 0 && k <= n && code < Binom(n, k), TD_E_STATE,
                "subset code out of range");
     // one subset of level k, as td_dp_get_level reads them
-    (void)ctx->Buffer("dp.walk_order", 64 * 4);  // asks the byte budget
     uint8_t* d = static_cast<uint8_t*>(ctx->Pinned(4));
     hipLaunchKernelGGL(DPExportLevelKernel, dim3(1), dim3(64), 0, ctx->stream,
                        static_cast<const DPHead&>(ctx->last_graph), PascalDevice(ctx),

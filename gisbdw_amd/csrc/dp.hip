@@ -574,30 +574,25 @@ __device__ __forceinline__ uint32_t WaveMax(uint32_t v) {
   return v;
 }
 
-// GetElimination (dynamic_gpu.hpp:49-64) for one start set per wave: pop the
-// root stored for the current set and repeat.  The root of a connected C is
+// GetElimination (dynamic_gpu.hpp:49-64) from S, by one wave: pop the root
+// stored for the current set and repeat, `steps` times.  The root of a connected C is
 // the smallest v with td(C \ v) = td(C) - 1 (the strict < over ascending v of
 // dynamic_gpu.cu:84-87); a disconnected set stores the root of its first
 // component (lowest vertex order) of largest td (dynamic_gpu.cu:90-104).
 __global__ __launch_bounds__(64) void DPWalkKernel(
-    const DPGraph* __restrict__ gs, const uint32_t* __restrict__ g_cb,
-    const uint8_t* __restrict__ arena, const uint32_t* __restrict__ start,
-    const int32_t* __restrict__ nsteps, int32_t* __restrict__ orders,
-    int order_stride) {
+    const DPGraph* __restrict__ g, const uint32_t* __restrict__ g_cb,
+    const uint8_t* __restrict__ arena, uint32_t S, int steps, int32_t* __restrict__ out) {
   __shared__ uint32_t s_cb[32 * kCbStride];
   __shared__ uint32_t s_base[kLookupWords];
-  const DPGraph* g = gs + blockIdx.x;
   LoadLookupTables(g, g_cb, s_cb, s_base);
   const int lane = threadIdx.x;
   const uint32_t myadj = lane < 32 ? g->adj[lane] : 0u;
-  uint32_t S = start[blockIdx.x];
-  const int steps = nsteps[blockIdx.x];
-  int32_t* out = orders + static_cast<size_t>(blockIdx.x) * order_stride;
   for (int step = 0; step < steps && S != 0u; ++step) {
-    // component of every vertex of S, by ballot BFS from each lowest vertex,
-    // and its td: lane i reads the code of the component's vertices 0..i, and
-    // td is the number of places where that code changes
-    uint32_t rest = S, C = 0u, T = 0u;
+    // C = the first component of largest td, components by ballot BFS from each
+    // lowest vertex.  A td takes up to 11 reads all over the table, so it is
+    // looked up only where sizes leave it open: td of a component is at most
+    // its size, and at least 2 if it has an edge.
+    uint32_t rest = S, C = 0u, T = 0u;  // T = td(C) once it is needed
     while (rest) {
       uint32_t comp = rest & (0u - rest), front = comp;
       for (;;) {
@@ -607,24 +602,24 @@ __global__ __launch_bounds__(64) void DPWalkKernel(
         comp |= nb;
         front = nb;
       }
-      const uint32_t upto = lane < 31 ? (2u << lane) - 1u : ~0u;
-      const uint32_t code =
-          lane < 32 ? LookupCode(g, arena, s_cb, s_base, comp & upto) : 0u;
-      const uint32_t below = __shfl_up(code, 1);
-      const uint32_t td = static_cast<uint32_t>(
-          __popcll(__ballot(lane < 32 && code != (lane ? below : 0u))));
-      if (td > T) {
-        T = td;
-        C = comp;
-      }
       rest &= ~comp;
+      const int most = __builtin_popcount(comp);
+      if (!C) {
+        C = comp;
+      } else if (most > (T ? static_cast<int>(T) : min(__builtin_popcount(C), 2))) {
+        if (!T) T = LookupTd(g, arena, s_cb, s_base, C);
+        const uint32_t td = LookupTd(g, arena, s_cb, s_base, comp);
+        if (td > T) {
+          T = td;
+          C = comp;
+        }
+      }
     }
-    // the root: the lowest v of the first component C of largest td whose
-    // removal lowers td, that is, changes the code
+    // the root: the lowest v of C whose removal lowers td, that is, changes
+    // the code
     const bool inC = lane < 32 && ((C >> lane) & 1u);
-    const uint32_t cc = inC ? LookupCode(g, arena, s_cb, s_base, C) : 0u;
-    const uint32_t cv = inC ? LookupCode(g, arena, s_cb, s_base, C & ~(1u << lane)) : 0u;
-    const unsigned long long rb = __ballot(inC && cv != cc);
+    const unsigned long long rb =
+        __ballot(inC && CodesDiffer(g, arena, s_cb, s_base, C, C & ~(1u << lane)));
     const int root = __ffsll(static_cast<long long>(rb)) - 1;
     if (lane == 0) out[step] = root;
     S &= ~(1u << root);
@@ -2161,16 +2156,11 @@ int td_dp_get_elimination(td_ctx* ctx, int32_t nverts, int32_t subset_size,
                "order_out is null");
     if (subset_size == 0) return;
     const uint32_t S = static_cast<uint32_t>(UnrankColex(n, subset_size, subset_code));
-    const int32_t steps = subset_size;
-    uint32_t* dstart = static_cast<uint32_t*>(ctx->Buffer("dp.walk_start", 8));
-    int32_t* dsteps = static_cast<int32_t*>(ctx->Buffer("dp.walk_steps", 8));
     int32_t* dorder = static_cast<int32_t*>(ctx->Buffer("dp.walk_order", 64 * 4));
-    TD_HIP(hipMemcpyAsync(dstart, &S, 4, hipMemcpyHostToDevice, ctx->stream));
-    TD_HIP(hipMemcpyAsync(dsteps, &steps, 4, hipMemcpyHostToDevice, ctx->stream));
     const DPGraph* dG = LastRecord(ctx);
     const uint8_t* arena = static_cast<const uint8_t*>(ctx->bufs["dp.arena"].p);
     hipLaunchKernelGGL(DPWalkKernel, dim3(1), dim3(64), 0, ctx->stream, dG,
-                       PascalDevice(ctx), arena, dstart, dsteps, dorder, 64);
+                       PascalDevice(ctx), arena, S, subset_size, dorder);
     TD_HIP(hipGetLastError());
     TD_HIP(hipMemcpyAsync(order_out, dorder, 4 * subset_size,
                           hipMemcpyDeviceToHost, ctx->stream));

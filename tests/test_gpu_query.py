@@ -1,5 +1,7 @@
-"""Queries over tables of two and four words to a tile, and of every number of
-three-vertex steps: a subset's treedepth equals its entry of the level read."""
+"""Queries over tables of every kind: a subset's treedepth (every number of
+three-vertex steps, two and four words to a tile) equals its entry of the level
+read, and the eliminations of sparse, mostly disconnected sets are the
+reference's."""
 import math
 import random
 
@@ -7,6 +9,7 @@ import pytest
 
 from gisbdw_amd import api
 from gisbdw_amd import graphs as G
+from test_gpu_dp import mask_of, ref_elimination
 
 pytestmark = pytest.mark.gpu
 
@@ -25,3 +28,17 @@ def test_single_reads_equal_level(n, low_bits):
             assert dp.GetTreedepth(n, k, code) == level[code], (k, code)
     assert math.comb(n, n) == 1 and dp.GetTreedepth(n, n, 0) == dp.treedepth
     ctx.close()
+
+
+@pytest.mark.parametrize("n,p", [(16, 0.1), (22, 0.09), (25, 0.08), (25, 0.2)])
+def test_elimination_of_disconnected_sets(ctx, oracle, n, p):
+    g = G.gnp(n, p, n + 1)
+    levels = oracle.dp_fast(g, levels=True)[2]
+    dp = api.DynamicGPU(ctx)
+    dp(g)
+    rng = random.Random(n)
+    for k in (1, 2, 3, 5, n // 2, n - 2, n):
+        code = rng.randrange(math.comb(n, k))
+        S = mask_of(oracle.decode(n, k, code))
+        print("eliminate", n, k, code, flush=True)
+        assert dp.GetElimination(n, k, code) == ref_elimination(g, levels, S, k)

@@ -703,11 +703,11 @@ constexpr int kChunk = 4096;
 struct Staging {
   uint64_t *adj, *tgt;
   int32_t *ns, *status;
-  float* out;  // the larger of kChunk score rows, and kChunk losses and the gradient
+  float* out;  // kChunk graphs' rows of `floats`, or their losses and the gradient
 };
-Staging StagingBuffers(td_ctx* ctx, int ngraphs) {
+Staging StagingBuffers(td_ctx* ctx, int ngraphs, size_t floats) {
   const size_t c = static_cast<size_t>(std::min(ngraphs, kChunk));
-  const size_t out = std::max<size_t>(256 * c, 4 * c + 4 * kNParams);
+  const size_t out = std::max<size_t>(4 * floats * c, 4 * c + 4 * kNParams);
   uint8_t* p = static_cast<uint8_t*>(ctx->Pinned(528 * c + out));
   Staging s;
   s.adj = reinterpret_cast<uint64_t*>(p);
@@ -741,7 +741,7 @@ void CheckIntake(const Uploaded& u, int ngraphs, const int32_t* ns, const uint64
 // there: the caller synchronizes and calls CheckIntake before it hands out any
 // result.
 Uploaded Intake(td_ctx* ctx, const char* tag, int ngraphs, const int32_t* ns,
-                const uint64_t* adj64, const uint64_t* targets) {
+                const uint64_t* adj64, const uint64_t* targets, size_t out_floats = 64) {
   TD_REQUIRE(ngraphs >= 1 && ns && adj64, TD_E_INVALID, "empty batch or null pointer");
   for (int i = 0; i < ngraphs; ++i)
     if (ns[i] < 1 || ns[i] > 64) CheckGraphs(ngraphs, ns, adj64);  // throws the first error
@@ -751,7 +751,7 @@ Uploaded Intake(td_ctx* ctx, const char* tag, int ngraphs, const int32_t* ns,
   u.adj = static_cast<uint64_t*>(ctx->Buffer(t + ".adj", 512ull * ngraphs));
   u.feat = static_cast<float*>(ctx->Buffer(t + ".feat", 1024ull * ngraphs));
   u.tgt = targets ? static_cast<uint64_t*>(ctx->Buffer(t + ".tgt", 8ull * ngraphs)) : nullptr;
-  u.st = StagingBuffers(ctx, ngraphs);
+  u.st = StagingBuffers(ctx, ngraphs, out_floats);
   u.last = 0;
   for (int at = 0; at < ngraphs; at += kChunk) {
     const size_t c = static_cast<size_t>(std::min(ngraphs - at, kChunk));
@@ -837,12 +837,22 @@ int td_mlp_get_weights(td_ctx* ctx, float* w, int64_t count) {
 int td_mlp_features(td_ctx* ctx, int32_t ngraphs, const int32_t* ns, const uint64_t* adj64,
                     float* feat_out) {
   return Guard(ctx, [&] {
-    Uploaded u = Intake(ctx, "mlp.in", ngraphs, ns, adj64, nullptr);
+    TD_REQUIRE(feat_out != nullptr, TD_E_INVALID, "features_out is null");
+    // up to kChunk graphs' features wait in page-locked memory for the check,
+    // so that one synchronization serves both
+    const bool staged = ngraphs <= kChunk;
+    const size_t bytes = 1024ull * ngraphs;
+    Uploaded u = Intake(ctx, "mlp.in", ngraphs, ns, adj64, nullptr, 256);
+    if (staged)
+      TD_HIP(hipMemcpyAsync(u.st.out, u.feat, bytes, hipMemcpyDeviceToHost, ctx->stream));
     TD_HIP(hipStreamSynchronize(ctx->stream));
     CheckIntake(u, ngraphs, ns, adj64);
-    TD_HIP(hipMemcpyAsync(feat_out, u.feat, 1024ull * ngraphs, hipMemcpyDeviceToHost,
-                          ctx->stream));
-    TD_HIP(hipStreamSynchronize(ctx->stream));
+    if (staged) {
+      std::memcpy(feat_out, u.st.out, bytes);
+    } else {
+      TD_HIP(hipMemcpyAsync(feat_out, u.feat, bytes, hipMemcpyDeviceToHost, ctx->stream));
+      TD_HIP(hipStreamSynchronize(ctx->stream));
+    }
   });
 }
 

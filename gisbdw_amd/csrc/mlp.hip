@@ -859,6 +859,7 @@ int td_mlp_features(td_ctx* ctx, int32_t ngraphs, const int32_t* ns, const uint6
 int td_mlp_scores(td_ctx* ctx, int32_t ngraphs, const int32_t* ns, const uint64_t* adj64,
                   float* scores_out) {
   return Guard(ctx, [&] {
+    TD_REQUIRE(scores_out != nullptr, TD_E_INVALID, "scores_out is null");
     DevNet d = NetBuffers(ctx);
     Uploaded u = Intake(ctx, "mlp.in", ngraphs, ns, adj64, nullptr);
     // up to kChunk graphs' scores go straight to host memory

@@ -11,7 +11,7 @@ from gisbdw_amd import graphs as G
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("call", ["td_mlp_features"])
+@pytest.mark.parametrize("call", ["td_mlp_features", "td_mlp_scores"])
 def test_null_output(call):
     ctx = api.Context()
     prop = learn.Proposal(ctx)

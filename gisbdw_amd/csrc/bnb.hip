@@ -1346,23 +1346,6 @@ __global__ void BnBResetQueue(uint32_t* q) {
   if (threadIdx.x == 0) *q = 0u;
 }
 
-template <typename F>
-int Guard(td_ctx* ctx, F&& f) {
-  if (!ctx) return TD_E_INVALID;
-  try {
-    TD_HIP(hipSetDevice(ctx->device));
-    f();
-    ctx->err.clear();
-    return TD_OK;
-  } catch (const Error& e) {
-    ctx->err = e.msg;
-    return e.code;
-  } catch (const std::exception& e) {
-    ctx->err = e.what();
-    return TD_E_INVALID;
-  }
-}
-
 int64_t Param(td_ctx* ctx, const char* k, int64_t dflt) {
   auto it = ctx->params.find(k);
   return it == ctx->params.end() ? dflt : it->second;

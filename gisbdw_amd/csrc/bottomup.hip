@@ -352,23 +352,6 @@ __global__ __launch_bounds__(64) void BottomUpWalkKernel(
   }
 }
 
-template <typename F>
-int BGuard(td_ctx* ctx, F&& f) {
-  if (!ctx) return TD_E_INVALID;
-  try {
-    TD_HIP(hipSetDevice(ctx->device));
-    f();
-    ctx->err.clear();
-    return TD_OK;
-  } catch (const Error& e) {
-    ctx->err = e.msg;
-    return e.code;
-  } catch (const std::exception& e) {
-    ctx->err = e.what();
-    return TD_E_INVALID;
-  }
-}
-
 const uint32_t* BuPascal(td_ctx* ctx) {
   auto it = ctx->bufs.find("bu.pascal");
   if (it != ctx->bufs.end() && it->second.p) return static_cast<const uint32_t*>(it->second.p);
@@ -434,7 +417,7 @@ extern "C" {
 
 int td_bottom_up(td_ctx* ctx, int32_t n, const uint64_t* adj, int32_t iterations,
                  int32_t* treedepth_out, int8_t* parent_out, int32_t* iterations_out) {
-  return BGuard(ctx, [&] {
+  return Guard(ctx, [&] {
     ValidateGraph(n, adj, 32);
     TD_REQUIRE(treedepth_out != nullptr, TD_E_INVALID, "treedepth_out is null");
     TD_REQUIRE(iterations == -1 || (iterations >= 1 && iterations <= n + 1), TD_E_INVALID,
@@ -546,7 +529,7 @@ int td_bottom_up(td_ctx* ctx, int32_t n, const uint64_t* adj, int32_t iterations
 }
 
 int td_bottom_up_get_treedepth(td_ctx* ctx, int32_t k, uint64_t code, uint32_t* td_out) {
-  return BGuard(ctx, [&] {
+  return Guard(ctx, [&] {
     TD_REQUIRE(ctx->have_bu, TD_E_STATE, "no td_bottom_up result to query");
     TD_REQUIRE(td_out != nullptr, TD_E_INVALID, "td_out is null");
     TD_REQUIRE(k >= 0 && k <= ctx->bu_n && code < Binom(ctx->bu_n, k), TD_E_INVALID,
@@ -565,7 +548,7 @@ int td_bottom_up_get_treedepth(td_ctx* ctx, int32_t k, uint64_t code, uint32_t* 
 
 int td_bottom_up_get_level(td_ctx* ctx, int32_t k, int8_t* last_out, uint8_t* height_out,
                            uint64_t out_len) {
-  return BGuard(ctx, [&] {
+  return Guard(ctx, [&] {
     TD_REQUIRE(ctx->have_bu, TD_E_STATE, "no td_bottom_up result to query");
     TD_REQUIRE(k >= 0 && k < ctx->bu_iters, TD_E_STATE, "level not run");
     const uint64_t cnt = Binom(ctx->bu_n, k);
@@ -580,7 +563,7 @@ int td_bottom_up_get_level(td_ctx* ctx, int32_t k, int8_t* last_out, uint8_t* he
 }
 
 int td_bottom_up_get_elimination(td_ctx* ctx, int32_t k, uint64_t code, int32_t* order_out) {
-  return BGuard(ctx, [&] {
+  return Guard(ctx, [&] {
     TD_REQUIRE(ctx->have_bu, TD_E_STATE, "no td_bottom_up result to query");
     TD_REQUIRE(order_out != nullptr || k == 0, TD_E_INVALID, "order_out is null");
     TD_REQUIRE(k >= 0 && k <= ctx->bu_n && code < Binom(ctx->bu_n, k), TD_E_INVALID,

@@ -67,6 +67,13 @@ void ValidateGraph(int n, const uint64_t* adj, int max_n) {
 
 }  // namespace tdhip
 
+void td_ctx::Settle() {
+  (void)hipStreamSynchronize(stream);
+  if (side) (void)hipStreamSynchronize(side);
+  for (hipStream_t q : lvl)
+    if (q) (void)hipStreamSynchronize(q);
+}
+
 void* td_ctx::Pinned(size_t bytes, int slot) {
   void*& p = pinned[slot];
   if (p && pinned_bytes[slot] >= bytes) return p;
@@ -118,10 +125,7 @@ void td_ctx::Release(const std::string& name) {
   auto it = bufs.find(name);
   if (it == bufs.end()) return;
   if (it->second.p) {
-    (void)hipStreamSynchronize(stream);
-    if (side) (void)hipStreamSynchronize(side);
-    for (hipStream_t q : lvl)
-      if (q) (void)hipStreamSynchronize(q);
+    Settle();
     (void)hipFree(it->second.p);
     allocated -= it->second.bytes;
   }
@@ -211,10 +215,7 @@ int td_ctx_create(td_ctx** out, int device, uint64_t mem_budget_bytes) {
 void td_ctx_destroy(td_ctx* c) {
   if (!c) return;
   (void)hipSetDevice(c->device);
-  if (c->stream) (void)hipStreamSynchronize(c->stream);
-  if (c->side) (void)hipStreamSynchronize(c->side);
-  for (hipStream_t q : c->lvl)
-    if (q) (void)hipStreamSynchronize(q);
+  if (c->stream) c->Settle();
   for (auto& kv : c->dp_graphs) (void)hipGraphExecDestroy(kv.second);
   if (c->bnb_graph) (void)hipGraphExecDestroy(c->bnb_graph);
   for (auto& kv : c->bufs)

@@ -203,6 +203,8 @@ struct td_ctx {
   void* pinned[2] = {nullptr, nullptr};
   size_t pinned_bytes[2] = {0, 0};
   void* Pinned(size_t bytes, int slot = 0);
+  // waits for everything this context has launched
+  void Settle();
 
   hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
   tdhip::WorkerPool workers;  // host threads for per-graph setup work
@@ -270,6 +272,28 @@ uint64_t Binom(int n, int k);
 // colex unrank on the host (n vertices, k-subset)
 uint64_t UnrankColex(int n, int k, uint64_t code);
 uint64_t RankColex(uint64_t mask);
+// The body of an entry point: f() with the context's device current, its errors
+// as a td_status and a message.  An error can leave f() with kernels in flight
+// that read and write the page-locked staging: they end before the caller has
+// the context back, whose next call uses that memory again.
+template <typename F>
+int Guard(td_ctx* ctx, F&& f) {
+  if (!ctx) return TD_E_INVALID;
+  int code = TD_E_INVALID;
+  try {
+    TD_HIP(hipSetDevice(ctx->device));
+    f();
+    ctx->err.clear();
+    return TD_OK;
+  } catch (const Error& e) {
+    ctx->err = e.msg;
+    code = e.code;
+  } catch (const std::exception& e) {
+    ctx->err = e.what();
+  }
+  ctx->Settle();
+  return code;
+}
 // validate a graph; returns the adjacency as 32-bit rows when n <= 32
 void ValidateGraph(int n, const uint64_t* adj, int max_n);
 // Runs call(), a td_dp_solve_batch of graphs of at most 26 vertices, without

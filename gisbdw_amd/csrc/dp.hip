@@ -1033,23 +1033,6 @@ void RunLevels(td_ctx* ctx, const DPGraph& G, const DPGraph* dG,
   ++*launches;
 }
 
-template <typename F>
-int Guard(td_ctx* ctx, F&& f) {
-  if (!ctx) return TD_E_INVALID;
-  try {
-    TD_HIP(hipSetDevice(ctx->device));
-    f();
-    ctx->err.clear();
-    return TD_OK;
-  } catch (const Error& e) {
-    ctx->err = e.msg;
-    return e.code;
-  } catch (const std::exception& e) {
-    ctx->err = e.what();
-    return TD_E_INVALID;
-  }
-}
-
 float Elapsed(hipEvent_t a, hipEvent_t b) {
   float ms = 0.f;
   TD_HIP(hipEventElapsedTime(&ms, a, b));

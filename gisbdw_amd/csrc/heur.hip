@@ -297,23 +297,6 @@ __global__ __launch_bounds__(192) void HeuristicKernel(
   if (lane == 0) td_out[gi] = best;
 }
 
-template <typename F>
-int HGuard(td_ctx* ctx, F&& f) {
-  if (!ctx) return TD_E_INVALID;
-  try {
-    TD_HIP(hipSetDevice(ctx->device));
-    f();
-    ctx->err.clear();
-    return TD_OK;
-  } catch (const Error& e) {
-    ctx->err = e.msg;
-    return e.code;
-  } catch (const std::exception& e) {
-    ctx->err = e.what();
-    return TD_E_INVALID;
-  }
-}
-
 }  // namespace
 }  // namespace tdhip
 
@@ -324,7 +307,7 @@ extern "C" {
 int td_heuristic_batch(td_ctx* ctx, int32_t ngraphs, const int32_t* n,
                        const uint64_t* adj_concat, int32_t kind, int32_t* td_out,
                        int8_t* parent_concat) {
-  return HGuard(ctx, [&] {
+  return Guard(ctx, [&] {
     TD_REQUIRE(ngraphs >= 1 && n && adj_concat && td_out, TD_E_INVALID,
                "empty batch or null pointer");
     TD_REQUIRE(kind >= 1 && kind <= 6, TD_E_INVALID, "kind must be in [1, 6]");

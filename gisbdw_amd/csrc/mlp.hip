@@ -635,23 +635,6 @@ __global__ __launch_bounds__(64) void LabelKernel(DPLookup L, const uint32_t* __
 // ---------------------------------------------------------------------------
 // host
 // ---------------------------------------------------------------------------
-template <typename F>
-int Guard(td_ctx* ctx, F&& f) {
-  if (!ctx) return TD_E_INVALID;
-  try {
-    TD_HIP(hipSetDevice(ctx->device));
-    f();
-    ctx->err.clear();
-    return TD_OK;
-  } catch (const Error& e) {
-    ctx->err = e.msg;
-    return e.code;
-  } catch (const std::exception& e) {
-    ctx->err = e.what();
-    return TD_E_INVALID;
-  }
-}
-
 struct DevNet {
   float* w;
   uint16_t* wb;

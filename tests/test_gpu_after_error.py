@@ -1,0 +1,40 @@
+"""A call that fails after it has launched something leaves nothing behind that
+the next call's staging memory could meet."""
+import numpy as np
+import pytest
+
+from gisbdw_amd import api, learn
+from gisbdw_amd import graphs as G
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("count", [8, 512])
+def test_call_after_no_memory(oracle, count):
+    """The gradient's rows (about 100 KB a graph) do not fit the budget when the
+    graphs are on their way already; the same memory then stages a solve's
+    record and the next scores."""
+    graphs = [G.tree_plus_edges(20 + i % 40, 0.1, i) for i in range(count)]
+    ns, adj = learn.pad_adj(graphs)
+    tgt = np.ones(count, np.uint64)
+    g = G.gnp(25, 0.2, 3)
+    want = oracle.dp_fast(g)
+    with api.Context() as free:
+        prop = learn.Proposal(free)
+        prop.init(1)
+        scores = prop.scores_padded(ns, adj)
+    # the solve's table, the other DP and network buffers, 1548 bytes a graph
+    ctx = api.Context(mem_budget_bytes=(1 << 25) + 650000 + 1600 * count)
+    prop = learn.Proposal(ctx)
+    prop.init(1)
+    dp = api.DynamicGPU(ctx)
+    dp(g)
+    for rep in range(4):
+        print("no memory", count, rep, flush=True)
+        with pytest.raises(api.TDError) as e:
+            prop.loss_grad(ns, adj, tgt)
+        assert e.value.code == api.TD_E_NOMEM
+        dp(g)
+        assert (dp.treedepth, dp.parent) == want
+        assert np.array_equal(prop.scores_padded(ns, adj), scores)
+    ctx.close()

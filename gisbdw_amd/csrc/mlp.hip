@@ -672,6 +672,20 @@ void CheckGraphs(int ngraphs, const int32_t* ns, const uint64_t* adj64) {
   }
 }
 
+// Guard for a call whose graphs are checked on the device: where there is no
+// memory to get them there, an invalid one is still the error that comes first.
+template <typename F>
+int GuardGraphs(td_ctx* ctx, int ngraphs, const int32_t* ns, const uint64_t* adj64, F&& f) {
+  return Guard(ctx, [&] {
+    try {
+      f();
+    } catch (const Error& e) {
+      if (e.code == TD_E_NOMEM) CheckGraphs(ngraphs, ns, adj64);
+      throw;
+    }
+  });
+}
+
 void CheckTargets(int ngraphs, const int32_t* ns, const uint64_t* targets) {
   for (int i = 0; i < ngraphs; ++i) {
     const uint64_t V = ns[i] >= 64 ? ~0ull : ((1ull << ns[i]) - 1ull);
@@ -819,7 +833,7 @@ int td_mlp_get_weights(td_ctx* ctx, float* w, int64_t count) {
 
 int td_mlp_features(td_ctx* ctx, int32_t ngraphs, const int32_t* ns, const uint64_t* adj64,
                     float* feat_out) {
-  return Guard(ctx, [&] {
+  return GuardGraphs(ctx, ngraphs, ns, adj64, [&] {
     TD_REQUIRE(feat_out != nullptr, TD_E_INVALID, "features_out is null");
     // up to kChunk graphs' features wait in page-locked memory for the check,
     // so that one synchronization serves both
@@ -841,7 +855,7 @@ int td_mlp_features(td_ctx* ctx, int32_t ngraphs, const int32_t* ns, const uint6
 
 int td_mlp_scores(td_ctx* ctx, int32_t ngraphs, const int32_t* ns, const uint64_t* adj64,
                   float* scores_out) {
-  return Guard(ctx, [&] {
+  return GuardGraphs(ctx, ngraphs, ns, adj64, [&] {
     TD_REQUIRE(scores_out != nullptr, TD_E_INVALID, "scores_out is null");
     DevNet d = NetBuffers(ctx);
     Uploaded u = Intake(ctx, "mlp.in", ngraphs, ns, adj64, nullptr);
@@ -867,7 +881,7 @@ int td_mlp_scores(td_ctx* ctx, int32_t ngraphs, const int32_t* ns, const uint64_
 // Mean loss over the graphs and (grad_out non-null) its gradient.
 int td_mlp_loss_grad(td_ctx* ctx, int32_t ngraphs, const int32_t* ns, const uint64_t* adj64,
                      const uint64_t* targets, float* loss_out, float* grad_out) {
-  return Guard(ctx, [&] {
+  return GuardGraphs(ctx, ngraphs, ns, adj64, [&] {
     TD_REQUIRE(ngraphs >= 1 && ns && adj64, TD_E_INVALID, "empty batch or null pointer");
     if (!targets) CheckGraphs(ngraphs, ns, adj64);
     TD_REQUIRE(targets != nullptr, TD_E_INVALID, "targets is null");
@@ -913,7 +927,7 @@ int td_mlp_loss_grad(td_ctx* ctx, int32_t ngraphs, const int32_t* ns, const uint
 int td_mlp_train(td_ctx* ctx, int32_t ngraphs, const int32_t* ns, const uint64_t* adj64,
                  const uint64_t* targets, int32_t epochs, int32_t batch, float lr,
                  uint64_t seed, float* epoch_loss_out) {
-  return Guard(ctx, [&] {
+  return GuardGraphs(ctx, ngraphs, ns, adj64, [&] {
     TD_REQUIRE(ngraphs >= 1 && ns && adj64, TD_E_INVALID, "empty batch or null pointer");
     const bool args = targets && epochs >= 1 && batch >= 1 && lr > 0.f;
     if (!args) CheckGraphs(ngraphs, ns, adj64);  // an invalid graph comes first

@@ -38,3 +38,23 @@ def test_call_after_no_memory(oracle, count):
         assert (dp.treedepth, dp.parent) == want
         assert np.array_equal(prop.scores_padded(ns, adj), scores)
     ctx.close()
+
+
+def test_invalid_graph_comes_before_no_memory():
+    ctx = api.Context(mem_budget_bytes=1 << 20)
+    prop = learn.Proposal(ctx)
+    prop.init(1)
+    ns, adj = learn.pad_adj([G.path(9) for _ in range(2000)])
+    tgt = np.ones(2000, np.uint64)
+    calls = {"features": lambda: prop.features(ns, adj),
+             "scores": lambda: prop.scores_padded(ns, adj),
+             "gradient": lambda: prop.loss_grad(ns, adj, tgt),
+             "train": lambda: prop.train(ns, adj, tgt, 1, 256)}
+    for code in (api.TD_E_NOMEM, api.TD_E_INVALID):
+        for name, call in calls.items():
+            print(name, code, flush=True)
+            with pytest.raises(api.TDError) as e:
+                call()
+            assert e.value.code == code, name
+        adj[1500, 3] |= np.uint64(1 << 3)  # a self loop
+    ctx.close()

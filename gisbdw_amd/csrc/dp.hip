@@ -1123,10 +1123,13 @@ void LaunchLds(td_ctx* ctx, const DPGraph& G, const uint32_t* cb, uint8_t* arena
 // the ticket counter: null where the byte budget or the device has no room for
 // it (the other kernels do without).  It is cleared when it is new and
 // (LaunchFlow) when the 16-bit tags have come round, so no word in it carries
-// a tag that is still to come.
+// a tag that is still to come.  The tag is kFlowStale while it is not known
+// what the buffer holds, an error included: the next call clears it.
 constexpr size_t kFlowHead = 256;
+constexpr uint32_t kFlowStale = 0xFFFFu;
 void ClearFlow(td_ctx* ctx) {
   const auto& b = ctx->bufs["dp.flow"];
+  ctx->flow_tag = kFlowStale;
   TD_HIP(hipMemsetAsync(b.p, 0, b.bytes, ctx->stream));
   ctx->flow_tag = 0;
   ctx->flow_tickets = 0;
@@ -1173,9 +1176,13 @@ int PlanFlow(const td_ctx* ctx, int count, const uint32_t* ns, FlowCall* f, size
 void LaunchFlow(td_ctx* ctx, FlowCall& f, int count, uint32_t groups, const FlowGraph* gs,
                 const uint32_t* cb, uint8_t* planes, uint8_t* buf, int8_t* parents, int32_t* tds,
                 int32_t* status, unsigned long long* clock) {
-  if (ctx->flow_tag >= 0xFFFFu) ClearFlow(ctx);
+  if (ctx->flow_tag >= kFlowStale) ClearFlow(ctx);
   f.ticket0 = ctx->flow_tickets;
-  f.tag = ++ctx->flow_tag;
+  f.tag = ctx->flow_tag + 1;
+  // the kernel's indexes come from its tickets: a launch check that fails (for
+  // an error of some earlier call of this thread, too, with the kernel on its
+  // way) must not leave them out of step
+  ctx->flow_tag = kFlowStale;
   f.spin = static_cast<uint32_t>(ctx->dp.flow_spin);
   uint32_t* ticket = reinterpret_cast<uint32_t*>(buf);
   auto* ex = reinterpret_cast<unsigned long long*>(buf + kFlowHead);
@@ -1193,6 +1200,7 @@ void LaunchFlow(td_ctx* ctx, FlowCall& f, int count, uint32_t groups, const Flow
     default: launch(DPFlowKernel<8>); break;
   }
   TD_HIP(hipGetLastError());
+  ctx->flow_tag = f.tag;
   ctx->flow_tickets += groups;
   hipLaunchKernelGGL(DPDirectTreeKernel, dim3(count), dim3(64), 0, ctx->stream, f, gs, table,
                      parents, tds, clock);

@@ -1,5 +1,7 @@
 """A call that fails after it has launched something leaves nothing behind that
 the next call's staging memory could meet."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -57,4 +59,27 @@ def test_invalid_graph_comes_before_no_memory():
                 call()
             assert e.value.code == code, name
         adj[1500, 3] |= np.uint64(1 << 3)  # a self loop
+    ctx.close()
+
+
+@pytest.mark.parametrize("n", [9, 20, 24, 26])
+def test_solve_after_an_error_of_another_call(oracle, n):
+    """An error that an earlier HIP call of the thread has left may end a solve
+    at its launch check; the solves after it are right."""
+    hip = C.CDLL("libamdhip64.so.7")
+    g = G.gnp(n, 0.25, n)
+    want = oracle.dp_fast(g)
+    ctx = api.Context()
+    dp = api.DynamicGPU(ctx)
+    for rep in range(3):
+        print("left-over error", n, rep, flush=True)
+        assert hip.hipSetDevice(1 << 20) != 0
+        try:
+            dp(g)
+        except api.TDError as e:
+            assert e.code == api.TD_E_HIP
+        for _ in range(2):
+            dp(g)
+            assert (dp.treedepth, dp.parent) == want
+        assert api.dp_solve_batch(ctx, [g, g], 0)[0] == [want[0]] * 2
     ctx.close()

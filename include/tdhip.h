@@ -165,9 +165,13 @@ int td_dp_solve_batch(td_ctx* ctx, int32_t ngraphs, const int32_t* n,
  * block) on a seeded G(n, 0.25) graph and keeps the best in the
  * context: the level kernels for n > 26 (such graphs also run in batch
  * calls, where the tree kernel is hidden), the level kernels plus the tree
- * kernel for smaller n.  With a non-null cache_path (JSON lines), a "best"
- * line for this n and device arch is applied without timing anything;
- * otherwise the sweep runs and every candidate plus the best are appended.
+ * kernel for smaller n.  Candidates that launch the same are timed once, and a
+ * parameter that makes no difference to the best launch stays as it is; so do
+ * "dp.class_bits" and "dp.packed", and for n <= 24, whose one launch reads
+ * none of these parameters, all of them.  With a non-null cache_path (JSON
+ * lines), a "best" line for this n and device arch is applied (n > 24) without
+ * timing anything; otherwise the sweep runs and every candidate plus the best
+ * are appended.
  * best_ms_out (nullable) receives the best time.  No reference counterpart:
  * the reference hard-codes 4096 x 128 threads per chunk
  * (Treedepth/src/dynamic_gpu/dynamic_gpu.cu:123-124). */
@@ -175,7 +179,8 @@ int td_dp_autotune(td_ctx* ctx, int32_t n, const char* cache_path,
                    double* best_ms_out);
 /* Autotuner of the persistent batch launch (td_dp_solve_batch mode 0):
  * sweeps (low_bits, tiles_per_lane, batch_block, batch_wg_per_cu) on the
- * given batch itself and keeps the best; the cache key is the batch's
+ * given batch itself and keeps the best (the present ones for a batch whose
+ * graphs all go to other kernels); the cache key is the batch's
  * (graph count, largest n, sum of n).  Same cache rules as td_dp_autotune. */
 int td_dp_autotune_batch(td_ctx* ctx, int32_t ngraphs, const int32_t* n,
                          const uint64_t* adj_concat, const char* cache_path,

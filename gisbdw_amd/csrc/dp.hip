@@ -796,7 +796,9 @@ struct LowMasks {
 int WordBits(int low_bits) { return low_bits >= 5 ? 2 : low_bits == 4 ? 1 : 0; }
 
 // Tile offsets of each high level, each level padded to a 128-byte boundary
-// of its plane so no cache line holds tiles of two levels.  Vertices n and
+// of its plane so no cache line holds tiles of two levels (32 bytes below 8
+// high vertices: such tables fit a few lines, and with more padding they
+// would take more bytes than a byte per subset did).  Vertices n and
 // up, where a tile has more than n, count as isolated.
 DPHead MakeHead(int n, const uint64_t* adj, int wb) {
   DPHead G;
@@ -805,7 +807,7 @@ DPHead MakeHead(int n, const uint64_t* adj, int wb) {
   G.n = n;
   G.lb = lb;
   G.nh = n > lb ? n - lb : 0;
-  const uint32_t pad_tiles = 128u >> (lb - 3);
+  const uint32_t pad_tiles = (G.nh < 8 ? 32u : 128u) >> (lb - 3);
   uint64_t off = 0;
   for (uint32_t h = 0; h <= G.nh; ++h) {
     G.lvl[h] = static_cast<uint32_t>(off);
@@ -1054,8 +1056,8 @@ DPGraph SingleGraph(td_ctx* ctx, int n, const uint64_t* adj, bool tables = true)
 
 // Whether the context claims a packed table's bytes for this graph.
 bool ClaimsPacked(const td_ctx* ctx, int n) {
-  return ctx->dp.packed && ctx->dp.class_bits > 0 && ctx->dp.low_bits >= 4 &&
-         n - ctx->dp.low_bits >= ctx->dp.class_min_nh;
+  const int lb = std::max(ctx->dp.low_bits, n - 28);  // of the byte tables
+  return ctx->dp.packed && ctx->dp.class_bits > 0 && lb >= 4 && n - lb >= ctx->dp.class_min_nh;
 }
 
 // The descriptor goes up from page-locked staging in one copy; the tree (64

@@ -1,4 +1,6 @@
 """What a byte budget admits: calls that fit it exactly, one after another."""
+import math
+
 import pytest
 
 from gisbdw_amd import api
@@ -33,4 +35,54 @@ def test_treedepth_query_needs_no_room(oracle, n):
     dp = api.DynamicGPU(ctx)
     dp(g)
     assert dp.GetTreedepth(n, n, 0) == dp.treedepth == oracle.dp_fast(g)[0]
+    ctx.close()
+
+
+# Bytes that a table of one byte per subset takes in tiles of 2^low subsets,
+# each level of tiles padded to 256 bytes, with the buffers beside it.
+def byte_table(n, low):
+    high, pad, tiles = max(n - low, 0), max(1, 256 >> low), 0
+    for h in range(high + 1):
+        tiles += -(-math.comb(high, h) // pad) * pad
+    return tiles << low
+
+
+RECORD, PASCAL = 4648, 139648
+
+
+@pytest.mark.parametrize("low_bits", [2, 3, 4, 5])
+def test_small_graphs_fit_where_byte_tables_did(oracle, low_bits):
+    """Padding of the bit planes' levels does not outgrow the byte tables."""
+    for n in range(1, 13):
+        g = G.gnp(n, 0.4, n)
+        want = oracle.dp_fast(g)
+        print("budget", low_bits, n, flush=True)
+        ctx = api.Context(mem_budget_bytes=byte_table(n, low_bits) + RECORD + 24 + PASCAL + 80)
+        ctx.set_param("dp.low_bits", low_bits)
+        dp = api.DynamicGPU(ctx)
+        dp(g)
+        assert (dp.treedepth, dp.parent) == want
+        ctx.close()
+        count = 16
+        for mode in (0, 1, 2):
+            rows = -(-byte_table(n, low_bits) // 256) * 256 + RECORD + 72
+            chunks = 16 * (max(n - low_bits, 0) + 1) if mode == 1 else 0
+            ctx = api.Context(mem_budget_bytes=count * (rows + chunks) + PASCAL + 256)
+            ctx.set_param("dp.low_bits", low_bits)
+            tds, pars, _ = api.dp_solve_batch(ctx, [g] * count, mode)
+            assert list(zip(tds, pars)) == [want] * count, mode
+            ctx.close()
+
+
+@pytest.mark.parametrize("low_bits", [3, 4])
+def test_packed_claim_at_32_vertices(low_bits):
+    """17/32 of a byte per subset, as tiles of 16 subsets and more took."""
+    n = 32
+    ctx = api.Context(mem_budget_bytes=(17 << 27) + (1 << 20) + (64 << 20))
+    for k, v in (("low_bits", low_bits), ("class_bits", 4), ("packed", 1)):
+        ctx.set_param("dp." + k, v)
+    dp = api.DynamicGPU(ctx)
+    print("packed", low_bits, flush=True)
+    dp(G.path(n))
+    assert dp.treedepth == 6
     ctx.close()

@@ -86,3 +86,24 @@ def test_packed_claim_at_32_vertices(low_bits):
     dp(G.path(n))
     assert dp.treedepth == 6
     ctx.close()
+
+
+def test_bottom_up_has_the_room_of_published_words(oracle):
+    """The words that a solve of 19..24 vertices publishes are no claim on the
+    budget: the bottom-up heuristic still gets all its levels."""
+    g, h = G.gnp(20, 0.3, 20), G.gnp(16, 0.3, 1)
+    want = oracle.dp_fast(g)[0]
+    single = (1 << 20) + RECORD + 24 + PASCAL + 80
+    bottom_up = least(lambda c: api.BottomUpHeuristicGPU(c)(h, h.n + 1), 1 << 24)
+    for iterations in (-1, h.n + 1):
+        # what is left over is less than the 0.5 MB of published words
+        ctx = api.Context(mem_budget_bytes=single + bottom_up + (8 << 10))
+        dp = api.DynamicGPU(ctx)
+        print("bottom up", iterations, flush=True)
+        dp(g)
+        bu = api.BottomUpHeuristicGPU(ctx)
+        bu(h, iterations)
+        assert bu.GetIterationsPerformed() == h.n + 1
+        dp(g)
+        assert dp.treedepth == want
+        ctx.close()

@@ -240,7 +240,6 @@ struct td_ctx {
   // DPFlowKernel's buffer: the words published in it carry the call's tag, and
   // its ticket counter has seen flow_tickets workgroups (see FlowBuffer)
   uint32_t flow_tag = 0, flow_tickets = 0;
-  bool single_solve_ran = false;  // by SolveOne, since it was last cleared (see KeepDP)
   int unsynced = 0;  // single solves since their stream was last synchronized
   bool record_up = false;  // its record is in "dp.graph" (see LastRecord)
   tdhip::DPGraph last_graph{};
@@ -297,14 +296,12 @@ int Guard(td_ctx* ctx, F&& f) {
 // validate a graph; returns the adjacency as 32-bit rows when n <= 32
 void ValidateGraph(int n, const uint64_t* adj, int max_n);
 // Runs call(), a td_dp_solve_batch of graphs of at most 26 vertices, without
-// ending the last single solve's queries: such a batch has buffers of its own,
-// unless it had to solve a graph singly.
+// ending the last single solve's queries: such a batch has buffers of its own.
 template <typename Call>
 int KeepDP(td_ctx* ctx, Call&& call) {
   const bool had = ctx->have_dp;
-  ctx->single_solve_ran = false;
   const int rc = call();
-  if (!ctx->single_solve_ran) ctx->have_dp = had;
+  ctx->have_dp = had;
   return rc;
 }
 // device address of td_dp_solve_noalloc's fixed scratch array for the

@@ -1219,7 +1219,6 @@ void SolveOne(td_ctx* ctx, int n, const uint64_t* adj, uint8_t* td_out,
   // the buffers below may be reallocated: until this solve completes, the
   // queries have no tables to read
   ctx->have_dp = false;
-  ctx->single_solve_ran = true;
   const bool lds = n <= kLdsMaxN, flow = !lds && n <= kFlowMaxN;
   DPGraph G = SingleGraph(ctx, n, adj, !lds && !flow);
   const uint64_t tbytes = ClaimedBytes(G, ClaimsPacked(ctx, n));
@@ -1874,7 +1873,7 @@ void SolveBatch(td_ctx* ctx, int ngraphs, const int32_t* ns,
     if (lds_stream != ctx->stream) TD_HIP(hipEventRecord(ctx->ev[3], lds_stream));
   }
   if (persistent) *persistent = mode == 0 && nbig > 0;
-  if (nbig > 0) {
+  auto launch_levels = [&] {
     auto launch = [&](auto wb) {
       constexpr int WB = decltype(wb)::value;
       if (mode == 0)
@@ -1889,7 +1888,18 @@ void SolveBatch(td_ctx* ctx, int ngraphs, const int32_t* ns,
       case 1: launch(std::integral_constant<int, 1>()); break;
       default: launch(std::integral_constant<int, 2>()); break;
     }
-  }
+  };
+  auto launch_trees = [&] {
+    if (mode == 0)
+      hipLaunchKernelGGL(DPTreeKernel<DPHead>, dim3(nbig), dim3(64), 0, ctx->stream,
+                         static_cast<const DPHead*>(drec), cb, arena, par, tds);
+    else
+      hipLaunchKernelGGL(DPTreeKernel<DPGraph>, dim3(nbig), dim3(64), 0, ctx->stream,
+                         static_cast<const DPGraph*>(drec), cb, arena, par, tds);
+    TD_HIP(hipGetLastError());
+    ++small_launches;
+  };
+  if (nbig > 0) launch_levels();
   for (int j = nbig; j < nmid;) {
     const int k = PlanFlow(ctx, nmid - j, &sizes[j], &flow, &flow_words, &flow_planes,
                            &flow_groups);
@@ -1904,35 +1914,35 @@ void SolveBatch(td_ctx* ctx, int ngraphs, const int32_t* ns,
   // mode 0 counts as one level kernel however its graphs were shared out;
   // else the launches
   level_kernels += mode == 0 ? 1 : small_launches;
-  if (nbig > 0) {
-    if (mode == 0)
-      hipLaunchKernelGGL(DPTreeKernel<DPHead>, dim3(nbig), dim3(64), 0, ctx->stream,
-                         static_cast<const DPHead*>(drec), cb, arena, par, tds);
-    else
-      hipLaunchKernelGGL(DPTreeKernel<DPGraph>, dim3(nbig), dim3(64), 0, ctx->stream,
-                         static_cast<const DPGraph*>(drec), cb, arena, par, tds);
-    TD_HIP(hipGetLastError());
-    ++launches;
-  }
-  launches += small_launches;
+  if (nbig > 0) launch_trees();
   TD_HIP(hipEventRecord(ctx->ev[2], ctx->stream));
   TD_HIP(hipStreamSynchronize(ctx->stream));
+  level_ms += Elapsed(ctx->ev[0], ctx->ev[1]);
+  tree_ms += Elapsed(ctx->ev[1], ctx->ev[2]);
+  if (*flow_status) {
+    // a wait was given up: the persistent kernel takes those graphs instead,
+    // as it does without room for the published words; the arena holds them
+    nbig = nmid;
+    off = 0;
+    for (int j = 0; j < nbig; ++j) place(j);
+    TD_HIP(hipMemcpyAsync(drec, block, record * nbig, hipMemcpyHostToDevice, ctx->stream));
+    TD_HIP(hipEventRecord(ctx->ev[0], ctx->stream));
+    launch_levels();
+    ++level_kernels;
+    TD_HIP(hipEventRecord(ctx->ev[1], ctx->stream));
+    launch_trees();
+    TD_HIP(hipEventRecord(ctx->ev[2], ctx->stream));
+    TD_HIP(hipStreamSynchronize(ctx->stream));
+    level_ms += Elapsed(ctx->ev[0], ctx->ev[1]);
+    tree_ms += Elapsed(ctx->ev[1], ctx->ev[2]);
+  }
   drain.a = drain.b = nullptr;
-  // a wait was given up: those graphs one by one (SolveOne falls back itself)
-  if (*flow_status)
-    for (int j = nbig; j < nmid; ++j) {
-      uint8_t td = 0;
-      SolveOne(ctx, ns[perm[j]], adj_concat + row_off[perm[j]], &td, par + 64ull * j, nullptr);
-      tds[j] = td;
-    }
-  if (*flow_status) ctx->have_dp = false;
+  launches += small_launches;
   for (int j = 0; j < ngraphs; ++j) {
     const int i = perm[j];
     if (td_out) td_out[i] = static_cast<uint8_t>(tds[j]);
     if (parent_concat) std::memcpy(parent_concat + row_off[i], par + 64ull * j, ns[i]);
   }
-  level_ms += Elapsed(ctx->ev[0], ctx->ev[1]);
-  tree_ms += Elapsed(ctx->ev[1], ctx->ev[2]);
   finish();
 }
 

@@ -1356,6 +1356,10 @@ void SolveBnBSearch(td_ctx* ctx, int ngraphs, const int32_t* ns, const uint64_t*
                     int8_t* parent_concat, uint8_t* certified_out, td_bnb_stats* stats,
                     bool finish = true);
 
+// Device buffers of td_dp_solve_batch for graphs of at most 26 vertices.
+constexpr const char* kBatchBuffers[] = {"dp.batch_arena", "dp.batch_graphs", "dp.batch_queue",
+                                         "dp.pascal", "dp.flow"};
+
 // The graphs of at most kFinishMaxN vertices that the search has left
 // uncertified, by the subset DP (whose single-solve tables and queries stay
 // as they are), in calls of at most 2^30 subsets; where the device or the
@@ -1363,8 +1367,8 @@ void SolveBnBSearch(td_ctx* ctx, int ngraphs, const int32_t* ns, const uint64_t*
 void FinishSmall(td_ctx* ctx, const int32_t* ns, const uint64_t* adj_concat,
                  const std::vector<size_t>& off, const int32_t* ub_seed, const float* scores,
                  std::vector<BnBOut>& out, double* ms) {
-  auto arena = ctx->bufs.find("dp.batch_arena");
-  const bool held = arena != ctx->bufs.end() && arena->second.p;
+  std::map<std::string, size_t> held;
+  for (const char* k : kBatchBuffers) held[k] = ctx->Held(k);
   std::vector<int> left;
   for (size_t i = 0; i < out.size(); ++i)
     if (ns[i] <= kFinishMaxN && !out[i].certified) left.push_back(static_cast<int>(i));
@@ -1424,8 +1428,16 @@ void FinishSmall(td_ctx* ctx, const int32_t* ns, const uint64_t* adj_concat,
     }
     at = end;
   }
-  // a byte budget is the caller's to spend on other calls
-  if (ctx->budget && !held && !left.empty()) ctx->Release("dp.batch_arena");
+  // a byte budget is the caller's to spend on other calls: what the DP has taken
+  // goes back, and captured launches with it, which know its addresses
+  if (!ctx->budget) return;
+  bool released = false;
+  for (const char* k : kBatchBuffers)
+    if (ctx->Held(k) > held[k]) {
+      ctx->Release(k);
+      released = true;
+    }
+  if (released) ctx->DropDPGraphs();
 }
 
 void SolveBnBSearch(td_ctx* ctx, int ngraphs, const int32_t* ns, const uint64_t* adj_concat,

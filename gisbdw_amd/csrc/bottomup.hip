@@ -430,8 +430,7 @@ int td_bottom_up(td_ctx* ctx, int32_t n, const uint64_t* adj, int32_t iterations
     uint64_t avail;
     if (ctx->budget) {
       // the subset DP's published words make room (td_ctx::Buffer)
-      const auto flow = ctx->bufs.find("dp.flow");
-      const uint64_t room = held + (flow != ctx->bufs.end() ? flow->second.bytes : 0);
+      const uint64_t room = held + ctx->Held("dp.flow");
       avail = ctx->budget - std::min(ctx->budget, ctx->allocated - room);
     } else {
       size_t free_b = 0, total_b = 0;

@@ -121,6 +121,17 @@ void* td_ctx::Buffer(const std::string& name, size_t bytes) {
   return b.p;
 }
 
+size_t td_ctx::Held(const std::string& name) const {
+  const auto it = bufs.find(name);
+  return it != bufs.end() && it->second.p ? it->second.bytes : 0;
+}
+
+void td_ctx::DropDPGraphs() {
+  for (auto& kv : dp_graphs) (void)hipGraphExecDestroy(kv.second);
+  dp_graphs.clear();
+  dp_graph_ptrs.clear();
+}
+
 void td_ctx::Release(const std::string& name) {
   auto it = bufs.find(name);
   if (it == bufs.end()) return;
@@ -216,7 +227,7 @@ void td_ctx_destroy(td_ctx* c) {
   if (!c) return;
   (void)hipSetDevice(c->device);
   if (c->stream) c->Settle();
-  for (auto& kv : c->dp_graphs) (void)hipGraphExecDestroy(kv.second);
+  c->DropDPGraphs();
   if (c->bnb_graph) (void)hipGraphExecDestroy(c->bnb_graph);
   for (auto& kv : c->bufs)
     if (kv.second.p) (void)hipFree(kv.second.p);
@@ -286,8 +297,7 @@ int td_ctx_set_param(td_ctx* c, const char* key, int64_t v) {
     return bad("unknown parameter");
   }
   // a change of DP launch shape invalidates the captured level graphs
-  for (auto& kv : c->dp_graphs) (void)hipGraphExecDestroy(kv.second);
-  c->dp_graphs.clear();
+  c->DropDPGraphs();
   return TD_OK;
 }
 

@@ -194,6 +194,7 @@ struct td_ctx {
   std::map<std::string, tdhip::DeviceBuffer> bufs;
   void* Buffer(const std::string& name, size_t bytes);
   void Release(const std::string& name);
+  size_t Held(const std::string& name) const;  // bytes of a buffer, 0 if there is none
   // page-locked host staging for the per-call copies, two independent
   // buffers (grown on demand): slot 0 for single-graph staging, slot 1 for the
   // batch records and results, which live across the large-graph pipeline.
@@ -263,6 +264,7 @@ struct td_ctx {
   std::map<GraphKey, hipGraphExec_t> dp_graphs;
   // buffer addresses baked into each captured graph (arena, descriptor)
   std::map<GraphKey, std::pair<const void*, const void*>> dp_graph_ptrs;
+  void DropDPGraphs();
 };
 
 namespace tdhip {

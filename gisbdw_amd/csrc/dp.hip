@@ -2020,9 +2020,7 @@ void ApplyTuned(td_ctx* ctx, const DPConfig& best) {
   const int use_graph = ctx->dp.use_graph;
   ctx->dp = best;
   ctx->dp.use_graph = use_graph;
-  for (auto& kv : ctx->dp_graphs) (void)hipGraphExecDestroy(kv.second);
-  ctx->dp_graphs.clear();
-  ctx->dp_graph_ptrs.clear();
+  ctx->DropDPGraphs();
 }
 
 // Times run() (level-kernel ms) under each candidate: one warm-up, then the

@@ -107,3 +107,34 @@ def test_bottom_up_has_the_room_of_published_words(oracle):
         dp(g)
         assert dp.treedepth == want
         ctx.close()
+
+
+def test_search_gives_the_dp_s_memory_back(oracle):
+    """Small graphs that the search hands to the subset DP leave nothing of it
+    on the budget: what fits after a search without the DP still fits."""
+    hard = [G.random_cubic(20, 5), G.gnp(18, 0.6, 3)]
+    g = G.gnp(21, 0.25, 8)
+    want = oracle.dp_fast(g)
+
+    def search(ctx, nodes):
+        for k, v in (("waves_per_graph", 1), ("memo_log2", 10), ("node_budget", nodes)):
+            ctx.set_param("bnb." + k, v)
+        return api.bnb_solve_batch(ctx, hard)
+
+    def alone(ctx):
+        search(ctx, 20000)  # too few for the DP to step in
+        api.DynamicGPU(ctx)(g)
+
+    ctx = api.Context(mem_budget_bytes=least(alone, 1 << 24))
+    dp = api.DynamicGPU(ctx)
+    print("search, then solve", flush=True)
+    tds, _, cert, _ = search(ctx, 50000)
+    assert all(cert) and tds == [oracle.dp_fast(h)[0] for h in hard]
+    dp(g)
+    assert (dp.treedepth, dp.parent) == want
+    # beside a solve that fills the budget the search does without the DP, and
+    # the solve's queries go on
+    tds, pars, _, _ = search(ctx, 50000)
+    assert all(oracle.certify(h, p, t) for h, p, t in zip(hard, pars, tds))
+    assert dp.GetTreedepth(g.n, g.n, 0) == want[0]
+    ctx.close()

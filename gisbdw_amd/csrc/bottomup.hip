@@ -367,7 +367,7 @@ const uint32_t* BuPascal(td_ctx* ctx) {
       if (__builtin_popcount(mask) == k) tail[off++] = static_cast<uint16_t>(mask);
   }
   void* d = ctx->Buffer("bu.pascal", cb.size() * 4);
-  TD_HIP(hipMemcpy(d, cb.data(), cb.size() * 4, hipMemcpyHostToDevice));
+  ctx->Copy(d, cb.data(), cb.size() * 4, hipMemcpyHostToDevice);
   return static_cast<const uint32_t*>(d);
 }
 
@@ -541,9 +541,8 @@ int td_bottom_up_get_treedepth(td_ctx* ctx, int32_t k, uint64_t code, uint32_t* 
       return;
     }
     uint8_t h = 0;
-    TD_HIP(hipMemcpy(&h,
-                     static_cast<const uint8_t*>(ctx->bufs["bu.height"].p) + ctx->bu_off[k] + code,
-                     1, hipMemcpyDeviceToHost));
+    ctx->Copy(&h, static_cast<const uint8_t*>(ctx->bufs["bu.height"].p) + ctx->bu_off[k] + code, 1,
+              hipMemcpyDeviceToHost);
     *td_out = h;
   });
 }
@@ -556,11 +555,11 @@ int td_bottom_up_get_level(td_ctx* ctx, int32_t k, int8_t* last_out, uint8_t* he
     const uint64_t cnt = Binom(ctx->bu_n, k);
     TD_REQUIRE(out_len >= cnt, TD_E_INVALID, "output shorter than the level");
     if (last_out)
-      TD_HIP(hipMemcpy(last_out, static_cast<const int8_t*>(ctx->bufs["bu.last"].p) +
-                                     ctx->bu_off[k], cnt, hipMemcpyDeviceToHost));
+      ctx->Copy(last_out, static_cast<const int8_t*>(ctx->bufs["bu.last"].p) + ctx->bu_off[k], cnt,
+                hipMemcpyDeviceToHost);
     if (height_out)
-      TD_HIP(hipMemcpy(height_out, static_cast<const uint8_t*>(ctx->bufs["bu.height"].p) +
-                                       ctx->bu_off[k], cnt, hipMemcpyDeviceToHost));
+      ctx->Copy(height_out, static_cast<const uint8_t*>(ctx->bufs["bu.height"].p) + ctx->bu_off[k],
+                cnt, hipMemcpyDeviceToHost);
   });
 }
 

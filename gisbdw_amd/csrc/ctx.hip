@@ -74,6 +74,11 @@ void td_ctx::Settle() {
     if (q) (void)hipStreamSynchronize(q);
 }
 
+void td_ctx::Copy(void* dst, const void* src, size_t bytes, hipMemcpyKind kind) {
+  TD_HIP(hipMemcpyAsync(dst, src, bytes, kind, stream));
+  TD_HIP(hipStreamSynchronize(stream));
+}
+
 void* td_ctx::Pinned(size_t bytes, int slot) {
   void*& p = pinned[slot];
   if (p && pinned_bytes[slot] >= bytes) return p;

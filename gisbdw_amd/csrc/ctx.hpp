@@ -206,6 +206,9 @@ struct td_ctx {
   void* Pinned(size_t bytes, int slot = 0);
   // waits for everything this context has launched
   void Settle();
+  // hipMemcpy on the context's stream: one on the null stream fails while some
+  // other thread captures a launch sequence, and ends that capture
+  void Copy(void* dst, const void* src, size_t bytes, hipMemcpyKind kind);
 
   hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
   tdhip::WorkerPool workers;  // host threads for per-graph setup work

@@ -885,7 +885,7 @@ const uint32_t* PascalDevice(td_ctx* ctx) {
     return static_cast<const uint32_t*>(it->second.p);
   const std::vector<uint32_t> cb = PascalTable();
   void* d = ctx->Buffer("dp.pascal", cb.size() * 4);
-  TD_HIP(hipMemcpy(d, cb.data(), cb.size() * 4, hipMemcpyHostToDevice));
+  ctx->Copy(d, cb.data(), cb.size() * 4, hipMemcpyHostToDevice);
   return static_cast<const uint32_t*>(d);
 }
 
@@ -2085,8 +2085,8 @@ void NoAllocSetup(td_ctx* ctx) {
   TD_HIP(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)));
   TD_REQUIRE(p != nullptr, TD_E_HIP, "hipGetSymbolAddress returned no address");
   const std::vector<uint32_t> cb = PascalTable();
-  TD_HIP(hipMemcpy(static_cast<uint8_t*>(p) + kNoAllocPascalOff, cb.data(), cb.size() * 4,
-                   hipMemcpyHostToDevice));
+  ctx->Copy(static_cast<uint8_t*>(p) + kNoAllocPascalOff, cb.data(), cb.size() * 4,
+            hipMemcpyHostToDevice);
   g_noalloc_ptr[ctx->device] = static_cast<uint8_t*>(p);
 }
 

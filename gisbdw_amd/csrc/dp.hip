@@ -2025,37 +2025,47 @@ void ApplyTuned(td_ctx* ctx, const DPConfig& best) {
 
 // Times run() (level-kernel ms) under each candidate: one warm-up, then the
 // mean of three.  Candidates under which run() launches the same, by
-// same(a, b), are timed once and share the time.  Returns the best time; *best
-// receives its configuration: the present one where that launches the same,
-// else the present one with adopt(&present, winner).
+// same(a, b), share the least of their times (a shape timed once can lose to a
+// worse one by noise); where all do, the first is timed alone.  Returns the best
+// time; *best receives its configuration: the present one where that launches
+// the same, else the present one with adopt(&present, winner).
 template <typename Run, typename Same, typename Adopt>
 double Sweep(td_ctx* ctx, const std::string& key, const std::vector<DPConfig>& cands,
              const char* cache_path, DPConfig* best, Run run, Same same, Adopt adopt) {
   const DPConfig saved = ctx->dp;
-  double best_ms = 1e30;
-  std::string log;
-  DPConfig winner = saved;
-  std::vector<std::pair<DPConfig, double>> timed;
+  const bool alike = std::all_of(cands.begin(), cands.end(),
+                                 [&](const DPConfig& c) { return same(cands.front(), c); });
+  std::vector<std::pair<DPConfig, double>> timed;  // by launch
+  auto at = [&](const DPConfig& c) {
+    return std::find_if(timed.begin(), timed.end(),
+                        [&](const auto& t) { return same(t.first, c); });
+  };
   try {
     for (const DPConfig& c : cands) {
-      auto it = std::find_if(timed.begin(), timed.end(),
-                             [&](const auto& t) { return same(t.first, c); });
-      if (it == timed.end()) {
-        ctx->dp = c;
-        run();
-        double t = 0;
-        for (int rep = 0; rep < 3; ++rep) t += run();
-        it = timed.insert(timed.end(), {c, t / 3});
-      }
-      log += JsonLine(key, c, it->second, false, ctx->prop.gcnArchName);
-      if (it->second < best_ms) {
-        best_ms = it->second;
-        winner = c;
-      }
+      auto it = at(c);
+      if (alike && it != timed.end()) break;
+      ctx->dp = c;
+      run();
+      double t = 0;
+      for (int rep = 0; rep < 3; ++rep) t += run();
+      t /= 3;
+      if (it == timed.end()) timed.push_back({c, t});
+      else it->second = std::min(it->second, t);
     }
   } catch (...) {
     ctx->dp = saved;
     throw;
+  }
+  double best_ms = 1e30;
+  std::string log;
+  DPConfig winner = saved;
+  for (const DPConfig& c : cands) {
+    const double t = at(c)->second;
+    log += JsonLine(key, c, t, false, ctx->prop.gcnArchName);
+    if (t < best_ms) {
+      best_ms = t;
+      winner = c;
+    }
   }
   ctx->dp = saved;
   *best = saved;

@@ -165,7 +165,7 @@ int td_dp_solve_batch(td_ctx* ctx, int32_t ngraphs, const int32_t* n,
  * block) on a seeded G(n, 0.25) graph and keeps the best in the
  * context: the level kernels for n > 26 (such graphs also run in batch
  * calls, where the tree kernel is hidden), the level kernels plus the tree
- * kernel for smaller n.  Candidates that launch the same are timed once, and a
+ * kernel for smaller n.  Candidates that launch the same share a time, and a
  * parameter that makes no difference to the best launch stays as it is; so do
  * "dp.class_bits" and "dp.packed", and for n <= 24, whose one launch reads
  * none of these parameters, all of them.  With a non-null cache_path (JSON

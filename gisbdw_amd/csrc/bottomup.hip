@@ -387,10 +387,8 @@ uint64_t BuBytes(int n, int K) {
 uint64_t BuHeld(td_ctx* ctx) {
   uint64_t b = 0;
   for (const char* k : {"bu.rec0", "bu.rec1", "bu.last", "bu.height", "bu.off", "bu.adj",
-                        "bu.pascal", "bu.walk", "bu.maxh"}) {
-    auto it = ctx->bufs.find(k);
-    if (it != ctx->bufs.end()) b += it->second.bytes;
-  }
+                        "bu.pascal", "bu.walk", "bu.maxh"})
+    b += ctx->Held(k);
   return b;
 }
 

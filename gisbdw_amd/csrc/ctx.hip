@@ -1,5 +1,6 @@
 // ctx.hip -- context lifetime, device buffers, parameters and host-side
 // combinatorics shared by the DP and the branch-and-bound.
+#include <algorithm>
 #include <cstring>
 
 #include "ctx.hpp"
@@ -94,24 +95,21 @@ void* td_ctx::Pinned(size_t bytes, int slot) {
   return p;
 }
 
-void* td_ctx::Buffer(const std::string& name, size_t bytes) {
+void* td_ctx::Buffer(const std::string& name, size_t bytes, size_t claim) {
+  claim = std::max(claim, bytes);
   auto& b = bufs[name];
-  if (b.bytes >= bytes && b.p) return b.p;
+  if (b.bytes >= bytes && b.claimed >= claim && b.p) return b.p;
   if (b.p) {
-    TD_HIP(hipStreamSynchronize(stream));
-    if (side) TD_HIP(hipStreamSynchronize(side));
-    for (hipStream_t q : lvl)
-      if (q) TD_HIP(hipStreamSynchronize(q));
+    Settle();
     TD_HIP(hipFree(b.p));
-    allocated -= b.bytes;
-    b.p = nullptr;
-    b.bytes = 0;
+    allocated -= b.claimed;
+    b = {};
   }
   // DPFlowKernel's buffer is a help, not a need: it makes room
-  if (budget && allocated + bytes > budget && name != "dp.flow") Release("dp.flow");
-  if (budget && allocated + bytes > budget)
+  if (budget && allocated + claim > budget && name != "dp.flow") Release("dp.flow");
+  if (budget && allocated + claim > budget)
     throw tdhip::Error{TD_E_NOMEM, "buffer '" + name + "' of " +
-                                       std::to_string(bytes) +
+                                       std::to_string(claim) +
                                        " bytes exceeds the context budget"};
   hipError_t e = hipMalloc(&b.p, bytes ? bytes : 1);
   if (e != hipSuccess) {
@@ -122,13 +120,14 @@ void* td_ctx::Buffer(const std::string& name, size_t bytes) {
                                        "' failed: " + hipGetErrorString(e)};
   }
   b.bytes = bytes;
-  allocated += bytes;
+  b.claimed = claim;
+  allocated += claim;
   return b.p;
 }
 
 size_t td_ctx::Held(const std::string& name) const {
   const auto it = bufs.find(name);
-  return it != bufs.end() && it->second.p ? it->second.bytes : 0;
+  return it != bufs.end() && it->second.p ? it->second.claimed : 0;
 }
 
 void td_ctx::DropDPGraphs() {
@@ -143,7 +142,7 @@ void td_ctx::Release(const std::string& name) {
   if (it->second.p) {
     Settle();
     (void)hipFree(it->second.p);
-    allocated -= it->second.bytes;
+    allocated -= it->second.claimed;
   }
   bufs.erase(it);
 }

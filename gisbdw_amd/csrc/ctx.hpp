@@ -96,6 +96,7 @@ struct DPConfig {
 struct DeviceBuffer {
   void* p = nullptr;
   size_t bytes = 0;
+  size_t claimed = 0;  // of the byte budget, at least bytes
 };
 
 }  // namespace tdhip
@@ -183,18 +184,19 @@ struct td_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
   uint64_t budget = 0;
-  uint64_t allocated = 0;
+  uint64_t allocated = 0;  // bytes claimed of the budget
   std::string err;
   hipDeviceProp_t prop{};
   double clock_khz = 1e5;  // rate of the device's wall clock
   tdhip::DPConfig dp;
   std::map<std::string, int64_t> params;
 
-  // named device buffers (grown on demand, freed with the context)
+  // named device buffers (grown on demand, freed with the context); a buffer
+  // takes `claim` bytes of the budget if that is more than its own
   std::map<std::string, tdhip::DeviceBuffer> bufs;
-  void* Buffer(const std::string& name, size_t bytes);
+  void* Buffer(const std::string& name, size_t bytes, size_t claim = 0);
   void Release(const std::string& name);
-  size_t Held(const std::string& name) const;  // bytes of a buffer, 0 if there is none
+  size_t Held(const std::string& name) const;  // bytes that a buffer claims, 0 if there is none
   // page-locked host staging for the per-call copies, two independent
   // buffers (grown on demand): slot 0 for single-graph staging, slot 1 for the
   // batch records and results, which live across the large-graph pipeline.

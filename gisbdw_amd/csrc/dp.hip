@@ -851,9 +851,9 @@ uint64_t TableBytes(const DPHead& G) {
   return 3 * (static_cast<uint64_t>(G.lvl[G.nh + 1]) << (G.lb - 3));
 }
 
-// Bytes that a graph's table takes from the context's budget: one per subset,
-// though only 3/8 are used, or (dp.packed with dp.class_bits) 17/32, so that a
-// byte budget admits and refuses the same calls as with byte tables.
+// Bytes that a graph's table claims of the context's budget: one per subset,
+// though only 3/8 are allocated, or (dp.packed with dp.class_bits) 17/32, so
+// that a byte budget admits and refuses the same calls as with byte tables.
 uint64_t ClaimedBytes(const DPHead& G, bool packed = false) {
   const uint64_t subsets = 1ull << G.n;
   return std::max(TableBytes(G), packed ? subsets / 2 + subsets / 32 : subsets);
@@ -1221,8 +1221,8 @@ void SolveOne(td_ctx* ctx, int n, const uint64_t* adj, uint8_t* td_out,
   ctx->have_dp = false;
   const bool lds = n <= kLdsMaxN, flow = !lds && n <= kFlowMaxN;
   DPGraph G = SingleGraph(ctx, n, adj, !lds && !flow);
-  const uint64_t tbytes = ClaimedBytes(G, ClaimsPacked(ctx, n));
-  uint8_t* arena = static_cast<uint8_t*>(ctx->Buffer("dp.arena", tbytes));
+  uint8_t* arena = static_cast<uint8_t*>(
+      ctx->Buffer("dp.arena", TableBytes(G), ClaimedBytes(G, ClaimsPacked(ctx, n))));
   uint8_t* din = static_cast<uint8_t*>(ctx->Buffer("dp.graph", kInBytes));
   DPGraph* dG = reinterpret_cast<DPGraph*>(din);
   const uint32_t* cb = PascalDevice(ctx);
@@ -1442,14 +1442,16 @@ void SolveLarge(td_ctx* ctx, const std::vector<int>& idx, const int32_t* ns,
   for (auto& e : ctx->pev)
     if (!e) TD_HIP(hipEventCreate(&e));
   // every buffer at its final size before the first launch
-  uint64_t tmax = 0;
-  for (int i : idx)
-    tmax = std::max(tmax, ClaimedBytes(SingleGraph(ctx, ns[i], adj_concat + row_off[i], false),
-                                       ClaimsPacked(ctx, ns[i])));
+  uint64_t tmax = 0, cmax = 0;
+  for (int i : idx) {
+    const DPGraph G = SingleGraph(ctx, ns[i], adj_concat + row_off[i], false);
+    tmax = std::max(tmax, TableBytes(G));
+    cmax = std::max(cmax, ClaimedBytes(G, ClaimsPacked(ctx, ns[i])));
+  }
   uint8_t *arena[kSlots], *din[kSlots], *dtree[kSlots];
   for (int s = 0; s < S; ++s) {
     const std::string sfx = s ? std::to_string(s) : std::string();
-    arena[s] = static_cast<uint8_t*>(ctx->Buffer("dp.arena" + sfx, tmax));
+    arena[s] = static_cast<uint8_t*>(ctx->Buffer("dp.arena" + sfx, tmax, cmax));
     din[s] = static_cast<uint8_t*>(ctx->Buffer("dp.graph" + sfx, kInBytes));
     dtree[s] = static_cast<uint8_t*>(ctx->Buffer("dp.tree_out" + sfx, kTreeBytes));
   }
@@ -1814,17 +1816,18 @@ void SolveBatch(td_ctx* ctx, int ngraphs, const int32_t* ns,
     used[n] = (TableBytes(H) + 255) / 256 * 256;
     claims[n] = (ClaimedBytes(H) + 255) / 256 * 256;
   }
-  uint64_t off = 0, claimed = 0;
+  uint64_t off = 0, room = 0, claimed = 0;
   auto place = [&](int j) {
     (mode == 0 ? heads[j].table : Gs[j].table) = off;
     off += used[sizes[j]];
   };
   for (int j = 0; j < ngraphs; ++j) {
     if (j < nbig) place(j);
+    if (j < nmid) room += used[sizes[j]];  // the persistent kernel may have to take any of them
     claimed += claims[sizes[j]];
   }
-  uint8_t* arena = static_cast<uint8_t*>(ctx->Buffer("dp.batch_arena", claimed));
-  void* drec = ctx->Buffer("dp.batch_graphs", sizeof(DPGraph) * ngraphs);
+  uint8_t* arena = static_cast<uint8_t*>(ctx->Buffer("dp.batch_arena", room, claimed));
+  void* drec = ctx->Buffer("dp.batch_graphs", record * ngraphs, sizeof(DPGraph) * ngraphs);
   const uint32_t* cb = PascalDevice(ctx);
   uint32_t* dq = static_cast<uint32_t*>(ctx->Buffer("dp.batch_queue", 256));
   int8_t* par = reinterpret_cast<int8_t*>(block + o_par);

@@ -45,7 +45,13 @@ constexpr int kStack = 72;  // Feasible(C, k) nests at most k + 1 <= 65 frames
 // graph: 30 us on one CU for n = 18, 95 us on the device for n = 24, what a
 // workgroup of 16 waves spends on 100 to 400 nodes, while a refutation on 20
 // vertices of a random cubic graph takes 3e5 nodes (80 ms).  Past 1024 nodes
-// (0.3 ms) the search is the worse bet.
+// (0.3 ms) the search is the worse bet.  Fewer would be faster on dense graphs
+// (256 of 20..24 vertices: 7.0 ms, and 1.6 with the DP at once, which
+// bnb.dp_max_n asks for), but sparse ones are settled by then, with the search's
+// own trees and details.  kFinishBudget is no speed limit: a budget of some
+// thousand nodes asks for an answer that may be uncertified after that much
+// search (sweeps of the budget use 1e3 to 3e4), and keeps that meaning; the line
+// lies between those and the budgets meant for certificates (5e4 and up).
 constexpr int kFinishMaxN = 24;
 constexpr uint64_t kFinishNodes = 1024, kFinishBudget = 32768;
 constexpr uint32_t kBudgetChunk = 64;  // search nodes a wave takes from its graph's budget at once

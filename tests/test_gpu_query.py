@@ -5,6 +5,7 @@ reference's."""
 import math
 import random
 
+import numpy as np
 import pytest
 
 from gisbdw_amd import api
@@ -42,3 +43,16 @@ def test_elimination_of_disconnected_sets(ctx, oracle, n, p):
         S = mask_of(oracle.decode(n, k, code))
         print("eliminate", n, k, code, flush=True)
         assert dp.GetElimination(n, k, code) == ref_elimination(g, levels, S, k)
+
+
+# 4 MiB of a level at a time: the last whole part, two parts, three
+@pytest.mark.parametrize("n,ks", [(24, (11, 12)), (25, (11, 12)), (26, (12, 13))])
+def test_levels_in_parts(ctx, oracle, n, ks):
+    g = G.gnp(n, 0.2, n)
+    levels = oracle.dp_fast(g, levels=True)[2]
+    dp = api.DynamicGPU(ctx)
+    dp(g)
+    for k in ks:
+        print("level", n, k, flush=True)
+        at = sum(math.comb(n, i) for i in range(k))
+        assert np.array_equal(dp.level(k), levels[at: at + math.comb(n, k)])

@@ -1373,11 +1373,12 @@ constexpr const char* kBatchBuffers[] = {"dp.batch_arena", "dp.batch_graphs", "d
 void FinishSmall(td_ctx* ctx, const int32_t* ns, const uint64_t* adj_concat,
                  const std::vector<size_t>& off, const int32_t* ub_seed, const float* scores,
                  std::vector<BnBOut>& out, double* ms) {
-  std::map<std::string, size_t> held;
-  for (const char* k : kBatchBuffers) held[k] = ctx->Held(k);
   std::vector<int> left;
   for (size_t i = 0; i < out.size(); ++i)
     if (ns[i] <= kFinishMaxN && !out[i].certified) left.push_back(static_cast<int>(i));
+  if (left.empty()) return;
+  std::map<std::string, size_t> held;
+  for (const char* k : kBatchBuffers) held[k] = ctx->Held(k);
   for (size_t at = 0; at < left.size();) {
     std::vector<int32_t> n, seed;
     std::vector<uint64_t> adj;

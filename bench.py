@@ -660,10 +660,7 @@ def main():
                 "low_bits": ctx.get_param("dp.low_bits"),
                 "tiles_per_lane": ctx.get_param("dp.tiles_per_lane"),
                 "block": ctx.get_param("dp.block"),
-                "xcd_remap": ctx.get_param("dp.xcd_remap"),
-                "class_bits": ctx.get_param("dp.class_bits"),
                 "grid_mult": ctx.get_param("dp.grid_mult"),
-                "packed": ctx.get_param("dp.packed"),
                 "streams": ctx.get_param("dp.streams"),
                 "autotuned": tuned_ms is not None,
             },

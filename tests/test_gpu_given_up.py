@@ -32,11 +32,13 @@ def test_batch_reports_both_launches(oracle):
     ctx = api.Context()
     want = [oracle.dp_fast(g) for g in graphs()]
     print("batch", flush=True)
-    tds, pars, st = api.dp_solve_batch(ctx, graphs(), 0)
-    assert list(zip(tds, pars)) == want and st.level_kernels == 1
+    for _ in range(2):  # the first call also loads and captures
+        tds, pars, st = api.dp_solve_batch(ctx, graphs(), 0)
+        assert list(zip(tds, pars)) == want and st.level_kernels == 1
     ctx.set_param("dp.flow_spin", 0)
-    tds, pars, late = api.dp_solve_batch(ctx, graphs(), 0)
-    assert list(zip(tds, pars)) == want
+    for _ in range(2):
+        tds, pars, late = api.dp_solve_batch(ctx, graphs(), 0)
+        assert list(zip(tds, pars)) == want
     assert late.level_kernels == 2 and late.launches >= st.launches + 2
     # the persistent kernel's time is in it: a workgroup by itself takes more
     # than 256 workgroups took
